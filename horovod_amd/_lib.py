@@ -73,6 +73,8 @@ _PROTOTYPES = {
     "hvdhip_fusion_unpack_record": (c_int, [c_void_p, c_void_p, c_double, c_void_p, c_void_p]),
     "hvdhip_reduce_sum": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "hvdhip_reduce_sum_k": (c_int, [c_void_p, _PV, c_int, c_int64, c_int, c_void_p]),
+    "hvdhip_ranks_sum": (c_int, [_PV, _PV, POINTER(c_int64), c_int, c_int, c_int, c_int, c_int, c_double, c_double,
+                                 c_uint, c_void_p, c_void_p]),
     "hvdhip_adasum_plan_create": (c_int, [POINTER(c_int), c_int, c_int, _PV]),
     "hvdhip_adasum_plan_destroy": (c_int, [c_void_p]),
     "hvdhip_adasum_dot_norms": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),

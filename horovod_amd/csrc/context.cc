@@ -230,6 +230,7 @@ const char* hvdhip_error_string(int code) {
   case HVDHIP_ERR_UNSUPPORTED_DTYPE: return "data type not supported by this operation";
   case HVDHIP_ERR_OUT_OF_MEMORY: return "out of device memory";
   case HVDHIP_ERR_TOO_LARGE: return "size exceeds what one launch can cover";
+  case HVDHIP_ERR_OVERLAP: return "an output overlaps another tensor of the call";
   default: return "unknown hvdhip error";
   }
 }

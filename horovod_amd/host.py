@@ -22,6 +22,11 @@ def _size_array(values):
     return (c_size_t * len(raw)).from_buffer(raw) if len(raw) else (c_size_t * 0)()
 
 
+def _count_array(values):
+    raw = array.array("q", values)
+    return (c_int64 * len(raw)).from_buffer(raw) if len(raw) else (c_int64 * 0)()
+
+
 class Stream:
     """A stream of the library (GPUContext::StreamCreate)."""
 
@@ -172,6 +177,23 @@ def reduce_sum_k(resident_ptr, incoming_ptrs, n, dtype, stream):
                                     stream.handle), "hvdhip_reduce_sum_k")
 
 
+RANKS_SUM_MAX_WORLD = 256
+_ERR_OVERLAP = -5
+
+
+def ranks_sum(output_ptrs, input_ptrs, counts, world, in_dtype, wire_dtype, out_dtype, prescale, postscale, stream,
+              pad=False, event=None):
+    """input_ptrs is rank-major (world * len(counts) addresses).  Returns False, with nothing queued, if an output
+    overlaps another tensor of the call."""
+    rc = lib().hvdhip_ranks_sum(_ptr_array(output_ptrs), _ptr_array(input_ptrs), _count_array(counts), len(counts),
+                                world, in_dtype, wire_dtype, out_dtype, prescale, postscale, 1 if pad else 0,
+                                stream.handle, event)
+    if rc == _ERR_OVERLAP:
+        return False
+    check(rc, "hvdhip_ranks_sum")
+    return True
+
+
 FP16_SCALE_FP32_FACTOR = 0  # ScaleBufferCPUImpl<unsigned short, float>, ops/collective_operations.h:99-127
 FP16_SCALE_HALF_FACTOR = 1  # scale_buffer_k<__half>, ops/cuda/cuda_kernels.cu:96-136,167
 
@@ -185,5 +207,5 @@ def get_fp16_scale_mode():
 
 
 __all__ = ["Stream", "Timer", "FusionPlan", "AdasumPlan", "batched_d2d_memcpy", "batched_scaled_d2d_memcpy",
-           "scale_buffer", "reduce_sum", "reduce_sum_k", "DTYPE", "FP16_SCALE_FP32_FACTOR", "FP16_SCALE_HALF_FACTOR",
+           "scale_buffer", "reduce_sum", "reduce_sum_k", "ranks_sum", "RANKS_SUM_MAX_WORLD", "DTYPE", "FP16_SCALE_FP32_FACTOR", "FP16_SCALE_HALF_FACTOR",
            "set_fp16_scale_mode", "get_fp16_scale_mode"]

@@ -7,17 +7,18 @@ AdasumGpuAllreduceOp, ops/adasum_gpu_operations.cc:64-310).  Here there is nothi
 negotiate: a cycle takes every request enqueued since the last one, fuses them with the same
 rule (through the C++ adapter) and queues, for every fused response,
 
-    wait for the framework's ready events -> pack (prescale, optional fp16 narrowing)
-    -> combine with the other ranks' buffers -> unpack (postscale, widening) -> completion event
+    wait for the framework's ready events -> the sum over ranks in one pass (prescale, optional fp16
+    narrowing, the additions in rank order, postscale, widening) -> completion event
 
 on one of the engine's streams through the C ABI of libhvdhip.so.  Nothing here computes.
 
 One GPU cannot hold a real communicator, so the *world* is simulated: ``size`` ranks of which
 this process is rank 0.  What ranks 1..size-1 contribute comes from ``peer_source(rank, name,
 tensor)``; by default every rank holds the same values, which is what the reference's own
-tests arrange by seeding all ranks alike (test/parallel/test_torch.py:251-445).  The peers'
-tensors go through the same pack kernel into buffers of their own, as they would on their own
-GPU, and the collective is the local reduce-sum (or the Adasum tree) over those resident buffers.
+tests arrange by seeding all ranks alike (test/parallel/test_torch.py:251-445).  All of
+them sit in this GPU's memory, so a sum needs no fusion buffer: the kernel reads every rank's tensors
+where they are, with the roundings that packing, summing and unpacking would make.  Adasum packs
+every node's tensors into a buffer and combines the buffers pairwise.
 """
 import ctypes
 from ctypes import c_int, c_int64, c_void_p
@@ -224,13 +225,8 @@ class Engine:
 
     def _execute(self, group):
         first = group[0][0]
-        tdt, wire = first.tensor_dtype, first.wire_dtype
-        es = dtype_size(wire)
         slot, s, requests = self._begin(group)
         counts = [e.count for _, e in group]
-        fused = len(group) > 1 or wire != tdt
-        flags = PACK_CAST_THEN_SCALE if wire != tdt else 0
-
         # the other ranks' tensors (framework stream), then this response's stream waits for them
         peers = [[self._peer_tensor(rank, r, e) for r, e in group] for rank in range(1, self.size)]
         if self.peer_source is not None and peers:
@@ -238,50 +234,71 @@ class Engine:
             made.record()
             check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(made.cuda_event)), "hvdhip_stream_wait_event")
             first.keepalive.append(made)
-
-        if fused:
-            plan = self._plan([e.tensor.data_ptr() for _, e in group], [e.output.data_ptr() for _, e in group],
-                              counts, tdt, wire)
-            nbytes = plan.buffer_len
-        else:
-            nbytes = group[0][1].count * es
-
-        # The other ranks' buffers first: with peer_source=None they are made from this rank's own
-        # tensors, which an in-place request (output is tensor) overwrites below.
-        peer_bufs = []
-        for rank, tensors in enumerate(peers, start=1):
-            pb = self._buffer(slot, rank, nbytes)
-            if fused:
-                ptrs = [t.data_ptr() for t in tensors]
-                self._plan(ptrs, ptrs, counts, tdt, wire).pack(pb, first.prescale, s, flags)
+        inputs = [[e.tensor.data_ptr() for _, e in group]] + [[t.data_ptr() for t in ts] for ts in peers]
+        outputs = [e.output.data_ptr() for _, e in group]
+        event = self._acquire(s)
+        try:
+            if not any(counts):
+                check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
+            elif first.op == ADASUM and peers:
+                self._adasum(slot, s, first, inputs, outputs, counts, event)
             else:
-                self._scale_or_copy(tensors[0].data_ptr(), pb, counts[0], first.prescale, tdt, s)
-            peer_bufs.append(pb)
+                self._sum(slot, s, first, inputs, outputs, counts, event)
+        except Exception:
+            check(lib().hvdhip_event_release(s.handle, event), "hvdhip_event_release")
+            raise
+        self._finish(s, requests, event)
 
-        if fused:
-            result = self._buffer(slot, 0, nbytes)
-            plan.pack(result, first.prescale, s, flags)
-            offsets = plan.offsets() + [nbytes]
-            layer_counts = [(offsets[i + 1] - offsets[i]) // es for i in range(len(group))]  # pad bytes are zero
-        else:
-            e = group[0][1]
-            result = e.output.data_ptr()
-            self._scale_or_copy(e.tensor.data_ptr(), result, e.count, first.prescale, tdt, s)
-            layer_counts = [e.count]
-        nelem = nbytes // es
+    @staticmethod
+    def _acquire(s):
+        """An event of the stream's pool for a response's completion."""
+        ev = c_void_p()
+        check(lib().hvdhip_event_acquire(s.handle, ctypes.byref(ev)), "hvdhip_event_acquire")
+        return ev
 
-        if nelem and peer_bufs:
-            if first.op == ADASUM:
-                self._adasum(slot, result, peer_bufs, nelem, layer_counts, wire, s)
-            else:
-                self._sum(result, peer_bufs, nelem, wire, s)
+    def _sum(self, slot, s, req, inputs, outputs, counts, event):
+        """outputs = postscale * (sum over ranks of prescale * inputs), in one pass if the outputs lie over no
+        other tensor of the response."""
+        tdt, wire = req.tensor_dtype, req.wire_dtype
+        if self.size <= H.RANKS_SUM_MAX_WORLD:
+            flat = [p for rank in inputs for p in rank]
+            if H.ranks_sum(outputs, flat, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s, event=event):
+                return
+        offsets, nbytes = self._offsets(counts, wire)
+        buf = self._to_buffer(slot, s, req, inputs, counts, offsets, nbytes)
+        self._from_buffer(buf, s, req, outputs, counts, offsets, event)
 
-        if fused:
-            plan.unpack(result, first.postscale, s)
-        elif first.postscale != 1.0 and nelem:
-            H.scale_buffer(result, result, nelem, first.postscale, tdt, s)
+    @staticmethod
+    def _offsets(counts, dtype):
+        """Byte offset of every entry in a fusion buffer and the buffer's length: each entry padded to 16
+        bytes (ops/gpu_operations.cc:141)."""
+        es, at, offsets = dtype_size(dtype), 0, []
+        for n in counts:
+            offsets.append(at)
+            at += (n * es + 15) // 16 * 16
+        return offsets, at
 
-        self._finish(s, requests)
+    def _to_buffer(self, slot, s, req, inputs, counts, offsets, nbytes):
+        """The sum of the ranks' scaled tensors in the stream slot's fusion buffer."""
+        tdt, wire = req.tensor_dtype, req.wire_dtype
+        buf = self._buffer(slot, 0, nbytes)
+        head, rest = inputs[:H.RANKS_SUM_MAX_WORLD], inputs[H.RANKS_SUM_MAX_WORLD:]
+        H.ranks_sum([buf + o for o in offsets], [p for rank in head for p in rank], counts, len(head), tdt, wire, wire,
+                    req.prescale, 1.0, s, pad=True)
+        for rank in rest:  # more ranks than one pass takes: one by one
+            one = self._buffer(slot, 1, nbytes)
+            H.ranks_sum([one + o for o in offsets], rank, counts, 1, tdt, wire, wire, req.prescale, 1.0, s, pad=True)
+            H.reduce_sum(buf, one, nbytes // dtype_size(wire), wire, s)
+        return buf
+
+    def _from_buffer(self, buf, s, req, outputs, counts, offsets, event):
+        tdt, wire = req.tensor_dtype, req.wire_dtype
+        if H.ranks_sum(outputs, [buf + o for o in offsets], counts, 1, wire, wire, tdt, 1.0, req.postscale, s,
+                       event=event):
+            return
+        for out, o, n in zip(outputs, offsets, counts):  # outputs that share memory: in order
+            H.ranks_sum([out], [buf + o], [n], 1, wire, wire, tdt, 1.0, req.postscale, s)
+        check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
 
     def _begin(self, group):
         """Picks the stream slot of a fused response and makes it wait for the framework."""
@@ -297,11 +314,9 @@ class Engine:
                   "hvdhip_stream_wait_event")
         return slot, s, requests
 
-    def _finish(self, s, requests):
-        ev = c_void_p()  # completion marker from the event pool
-        check(lib().hvdhip_event_acquire(s.handle, ctypes.byref(ev)), "hvdhip_event_acquire")
-        check(lib().hvdhip_event_record(ev, s.handle), "hvdhip_event_record")
-        marker = Marker(s, ev, len(requests))
+    @staticmethod
+    def _finish(s, requests, event):
+        marker = Marker(s, event, len(requests))
         for r in requests:
             r.markers.append(marker)
 
@@ -334,42 +349,37 @@ class Engine:
         if nbytes:
             H.batched_d2d_memcpy(into_buf, from_src, nbytes, s)
             H.batched_d2d_memcpy(out_dst, from_buf, nbytes, s)
-        self._finish(s, requests)
+        event = self._acquire(s)
+        check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
+        self._finish(s, requests, event)
 
-    @staticmethod
-    def _scale_or_copy(src, dst, count, scale, dtype, s):
-        """ops/nccl_operations.cc:176-186: an unfused tensor is scaled out of place into its
-        output, or copied there when there is nothing to scale."""
-        if count == 0:
-            return
-        if scale != 1.0:
-            H.scale_buffer(src, dst, count, scale, dtype, s)
-        elif src != dst:
-            H.batched_d2d_memcpy([dst], [src], [count * dtype_size(dtype)], s)
-
-    @staticmethod
-    def _sum(result, peer_bufs, nelem, dtype, s):
-        for i in range(0, len(peer_bufs), 16):
-            H.reduce_sum_k(result, peer_bufs[i:i + 16], nelem, dtype, s)
-
-    def _adasum(self, slot, result, peer_bufs, nelem, layer_counts, dtype, s):
+    def _adasum(self, slot, s, req, inputs, outputs, counts, event):
         """Ranks of one node are summed (the reduce-scatter leg of
         ops/adasum_gpu_operations.cc:174-197), then the node results are combined pairwise at
         distances 1, 2, 4 ... like the levels of Adasum::FusedAllreduce (ops/adasum/adasum.h:194-340)."""
-        bufs = [result] + peer_bufs
-        L = self.local_size
-        leaders = []
-        for node in range(self.size // L):
-            lead = bufs[node * L]
-            if L > 1:
-                self._sum(lead, bufs[node * L + 1:node * L + L], nelem, dtype, s)
-            leaders.append(lead)
-        plan = self._adasum_plan(slot, layer_counts, dtype)
+        wire, L = req.wire_dtype, self.local_size
+        flags = PACK_CAST_THEN_SCALE if wire != req.tensor_dtype else 0
+        plans = [self._plan(ptrs, ptrs if rank else outputs, counts, req.tensor_dtype, wire)
+                 for rank, ptrs in enumerate(inputs)]
+        nbytes = plans[0].buffer_len
+        bufs = [self._buffer(slot, rank, nbytes) for rank in range(self.size)]
+        for rank in [*range(1, self.size), 0]:
+            plans[rank].pack(bufs[rank], req.prescale, s, flags)
+        offsets = plans[0].offsets() + [nbytes]
+        es = dtype_size(wire)
+        layers = [(hi - lo) // es for lo, hi in zip(offsets, offsets[1:])]  # pad bytes are zero
+        leaders = bufs[::L]
+        for node, lead in enumerate(leaders):
+            for i in range(node * L + 1, node * L + L, 16):
+                more = bufs[i:min(i + 16, node * L + L)]
+                H.reduce_sum_k(lead, more, nbytes // es, wire, s)
+        combine = self._adasum_plan(slot, layers, wire)
         d = 1
         while d < len(leaders):
             for i in range(0, len(leaders), 2 * d):
-                plan.combine(leaders[i], leaders[i + d], s)
+                combine.combine(leaders[i], leaders[i + d], s)
             d *= 2
+        plans[0].unpack(bufs[0], req.postscale, s, event=event)
 
     # ---- completion -----------------------------------------------------
 

@@ -55,6 +55,8 @@ enum hvdhip_dtype {
 /* A plan or batched copy needs more than 2^23 workgroups (32 GiB at 4 KiB each) in one launch.
  * Contiguous entry points (scale, reduce) have no such limit: they slice. */
 #define HVDHIP_ERR_TOO_LARGE (-4)
+/* hvdhip_ranks_sum(): an output overlaps another output or another entry's input. */
+#define HVDHIP_ERR_OVERLAP (-5)
 
 /* Flags of hvdhip_fusion_pack(). */
 #define HVDHIP_PACK_DEFAULT 0u
@@ -316,6 +318,35 @@ int hvdhip_reduce_sum(void* resident, const void* incoming, int64_t num_elements
  * was tried in the kernel and changes nothing. */
 int hvdhip_reduce_sum_k(void* resident, const void* const* incoming, int k, int64_t num_elements,
                         int dtype, void* stream);
+
+/* The sum over `world` ranks of n fused tensors that all sit in memory this device
+ * reads, in one pass: what packing every rank's tensors (hvdhip_fusion_pack),
+ * summing the buffers in rank order (hvdhip_reduce_sum_k) and unpacking the sum
+ * (hvdhip_fusion_unpack) give, to the bit, without the buffers in between.
+ * inputs[r * n + i] is rank r's tensor of entry i, outputs[i] the result;
+ * num_elements[i] may be 0.  All three arrays are HOST arrays, read before the
+ * call returns; nothing is kept of them, and nothing is allocated.
+ *
+ * Every rank's element is brought to wire_dtype and multiplied by prescale, the
+ * ranks are added with a rounding to wire_dtype after each, the sum is
+ * multiplied by postscale and brought to out_dtype; a factor of 1 leaves the
+ * value alone.  The three dtypes are equal, or the wire is FLOAT16 and the others
+ * FLOAT16 or FLOAT32 (converted first, scaled as FLOAT16: the order of
+ * HVDHIP_PACK_CAST_THEN_SCALE and of the converting unpack).  With world == 1 this
+ * is a scaled batched copy.
+ *
+ * An output may be one of its own entry's inputs; any other overlap between an
+ * output and an output or input returns HVDHIP_ERR_OVERLAP and nothing is launched.
+ * HVDHIP_RANKS_SUM_PAD_OUTPUTS: outputs lie in a fusion buffer; the up to 15 bytes
+ * behind each are zeroed to the next multiple of 16 of its size, and the stores go
+ * through the Infinity Cache for the kernel that reads them next.
+ * event: NULL, or an event that reads as recorded behind the call (as in
+ * hvdhip_fusion_unpack_record). */
+#define HVDHIP_RANKS_SUM_PAD_OUTPUTS 1u
+#define HVDHIP_RANKS_SUM_MAX_WORLD 256
+int hvdhip_ranks_sum(void* const* outputs, const void* const* inputs, const int64_t* num_elements, int n,
+                     int world, int in_dtype, int wire_dtype, int out_dtype, double prescale,
+                     double postscale, unsigned flags, void* stream, void* event);
 
 /* ------------------------------------------------------------------------ */
 /* Adasum: Adasum<Comm>::FusedPairwiseReduceWithComm on one device          */

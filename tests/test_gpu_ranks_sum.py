@@ -1,0 +1,120 @@
+"""hvdhip_ranks_sum against the oracle's scale -> sum -> scale at the edges of its chunks (4 KiB), rows per
+launch (64, or fewer for many ranks) and ranks per batch (8)."""
+import numpy as np
+import pytest
+import torch
+
+from horovod_amd import DTYPE
+from horovod_amd import host as H
+
+pytestmark = pytest.mark.gpu
+
+NP = {"uint8": np.uint8, "int8": np.int8, "int16": np.int16, "int32": np.int32, "int64": np.int64,
+      "float16": np.float16, "float32": np.float32, "float64": np.float64}
+
+
+def _values(rng, n, dtype):
+    if dtype.startswith("float"):
+        return rng.uniform(-2, 2, n).astype(NP[dtype])
+    return rng.integers(0, 120, n).astype(NP[dtype])
+
+
+def _expected(orc, ranks, dtype, wire, pre, post):
+    code = DTYPE[wire]
+    acc = None
+    for v in ranks:
+        w = v.astype(np.float16) if wire != dtype else v
+        w = orc.scale_buffer(w, pre, code) if pre != 1.0 else w
+        acc = w if acc is None else orc.sum(w, acc.copy(), code)
+    acc = orc.scale_buffer(acc, post, code) if post != 1.0 else acc
+    return acc.astype(NP[dtype])
+
+
+@pytest.mark.parametrize("dtype,wire", [(d, d) for d in NP] + [("float32", "float16")])
+@pytest.mark.parametrize("world", [1, 2, 7, 8, 9, 20])
+def test_ranks_sum_equals_scale_sum_scale(gpu, orc, dtype, wire, world):
+    rng = np.random.default_rng(world)
+    tile = 4096 // np.dtype(NP[dtype]).itemsize
+    counts = [1, 0, 3, tile - 1, tile, tile + 1, 5 * tile + 7, 255] + [int(x) for x in rng.integers(1, 40, 70)]
+    pre, post = (1.0, 1.0) if dtype == "int16" else ((0.125, 0.3) if world % 2 else (1.0, 0.7))
+    host = [[_values(rng, c, dtype) for c in counts] for _ in range(world)]
+    # one element into the allocation each: only element alignment is promised
+    dev = [[torch.from_numpy(np.concatenate([v[:1], v])).cuda()[1 if v.size else 0:] for v in rank] for rank in host]
+    out = [torch.zeros(c + 1, dtype=dev[0][0].dtype, device="cuda") for c in counts]
+    torch.cuda.synchronize()
+    code, wcode = DTYPE[dtype], DTYPE[wire]
+    assert H.ranks_sum([o.data_ptr() for o in out], [t.data_ptr() for r in dev for t in r], counts, world, code, wcode,
+                       code, pre, post, gpu.stream)
+    # in place as well: rank 0's tensors are the outputs
+    mine = [t.data_ptr() for t in dev[0]]
+    assert H.ranks_sum(mine, [t.data_ptr() for r in dev for t in r], counts, world, code, wcode, code, pre, post,
+                       gpu.stream)
+    gpu.stream.synchronize()
+    for i, c in enumerate(counts):
+        if c == 0:
+            continue
+        want = _expected(orc, [host[r][i] for r in range(world)], dtype, wire, pre, post)
+        got = out[i].cpu().numpy()
+        assert np.array_equal(got[:c].view(np.uint8), want.view(np.uint8)), (i, c)
+        assert got[c] == 0, "wrote behind its tensor"
+        assert np.array_equal(dev[0][i].cpu().numpy().view(np.uint8), want.view(np.uint8)), (i, c)
+
+
+def test_ranks_sum_into_and_out_of_a_buffer(gpu, orc):
+    """FLOAT32 tensors into a FLOAT16 fusion buffer, pad bytes zeroed, and out again."""
+    rng = np.random.default_rng(3)
+    counts = [5, 1024, 2049, 1]
+    offs = np.cumsum([0] + [(2 * c + 15) // 16 * 16 for c in counts])
+    a, b = ([rng.uniform(-2, 2, c).astype(np.float32) for c in counts] for _ in range(2))
+    da, db = ([torch.from_numpy(v).cuda() for v in x] for x in (a, b))
+    buf = torch.full((int(offs[-1]),), 255, dtype=torch.uint8, device="cuda")
+    out = [torch.zeros_like(t) for t in da]
+    torch.cuda.synchronize()
+    f32, f16 = DTYPE["float32"], DTYPE["float16"]
+    at = [buf.data_ptr() + int(o) for o in offs[:-1]]
+    assert H.ranks_sum(at, [t.data_ptr() for t in da + db], counts, 2, f32, f16, f16, 0.25, 1.0, gpu.stream, pad=True)
+    assert H.ranks_sum([t.data_ptr() for t in out], at, counts, 1, f16, f16, f32, 1.0, 3.0, gpu.stream)
+    gpu.stream.synchronize()
+    image = buf.cpu().numpy()
+    for i, c in enumerate(counts):
+        half = [v.astype(np.float16) for v in (a[i], b[i])]
+        want = _expected(orc, half, "float16", "float16", 0.25, 1.0)
+        piece = image[offs[i]:offs[i + 1]]
+        assert np.array_equal(piece[:2 * c], want.view(np.uint8)) and not piece[2 * c:].any()
+        got = out[i].cpu().numpy()
+        assert np.array_equal(got, orc.scale_buffer(want, 3.0, f16).astype(np.float32))
+
+
+def test_ranks_sum_refuses_overlap(gpu):
+    t = torch.zeros(4096, dtype=torch.float32, device="cuda")
+    p, f32 = t.data_ptr(), DTYPE["float32"]
+    call = lambda outs, ins, counts, world: H.ranks_sum(outs, ins, counts, world, f32, f32, f32, 1.0, 1.0, gpu.stream)  # noqa: E731
+    assert call([p, p + 400], [p, p + 400], [100, 100], 1)
+    assert not call([p, p + 396], [p + 8192, p + 12000], [100, 100], 1)        # output over output
+    assert not call([p], [p + 4], [100], 1)                                    # output over a shifted input
+    assert not call([p, p + 400], [p, p + 400, p + 400, p], [100, 100], 2)     # output over another entry's input
+
+
+@pytest.mark.parametrize("case", ["peers_are_outputs", "same_output_twice", "more_ranks_than_one_pass"])
+def test_engine_sums_through_a_buffer_where_one_pass_cannot(monkeypatch, case):
+    import horovod_amd.torch as hvd
+    hvd.shutdown()
+    size = 5 if case == "more_ranks_than_one_pass" else 2
+    x, y = (torch.arange(n, dtype=torch.float32, device="cuda") + n for n in (1000, 1000))
+    xs, ys = x.cpu(), y.cpu()
+    if case == "more_ranks_than_one_pass":
+        monkeypatch.setattr(H, "RANKS_SUM_MAX_WORLD", 2)
+    # rank 1 passes the other entry's tensor, which is overwritten in place
+    hvd.init(size=size, peer_source=(lambda r, name, t: y if t is x else x) if case == "peers_are_outputs" else None)
+    try:
+        if case == "same_output_twice":
+            y, ys = x, xs
+        handles = [hvd.allreduce_async_(t, op=hvd.Sum) for t in (x, y)]
+        for h in handles:
+            hvd.synchronize(h)
+        if case == "peers_are_outputs":
+            assert torch.equal(x.cpu(), xs + ys) and torch.equal(y.cpu(), xs + ys)
+        else:
+            assert torch.equal(x.cpu(), size * xs) and torch.equal(y.cpu(), size * ys)
+    finally:
+        hvd.shutdown()
