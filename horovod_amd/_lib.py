@@ -75,6 +75,9 @@ _PROTOTYPES = {
     "hvdhip_reduce_sum_k": (c_int, [c_void_p, _PV, c_int, c_int64, c_int, c_void_p]),
     "hvdhip_ranks_sum": (c_int, [_PV, _PV, POINTER(c_int64), c_int, c_int, c_int, c_int, c_int, c_double, c_double,
                                  c_uint, c_void_p, c_void_p]),
+    "hvdhip_adasum_ranks_workspace": (c_int64, [POINTER(c_int64), c_int, c_int, c_int]),
+    "hvdhip_adasum_ranks": (c_int, [_PV, _PV, POINTER(c_int64), c_int, c_int, c_int, c_int, c_int, c_double, c_double,
+                                    c_void_p, c_int64, c_void_p, c_void_p]),
     "hvdhip_adasum_plan_create": (c_int, [POINTER(c_int), c_int, c_int, _PV]),
     "hvdhip_adasum_plan_destroy": (c_int, [c_void_p]),
     "hvdhip_adasum_dot_norms": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -1,0 +1,104 @@
+// ranks.h -- shared by the kernels that read every rank's tensors where they sit in this device's memory
+// (not installed): the addresses in a launch's arguments, an element's way to the wire type and back,
+// and the checks of a call.
+#ifndef HVDHIP_RANKS_H
+#define HVDHIP_RANKS_H
+
+#include "internal.h"
+#include "vecmem.h"
+
+namespace hvdhip {
+
+constexpr uint32_t kMaxRows = 64;   // one lane of a wavefront looks at each
+constexpr uint32_t kQwords = 440;   // addresses and counts: with `first` and the scalars below 4 KiB
+
+// first[i]: the first chunk of row i; beyond the last row a number no chunk reaches.
+// q: a few words per row, the same number for every row of a launch (addresses and the element count).
+struct Rows {
+  uint32_t first[kMaxRows];
+  uint64_t q[kQwords];
+};
+
+// The row that `chunk` of a launch belongs to; every wavefront finds it by itself: a lane per row compares
+// the row's first chunk, and the count of lanes at or below is the row.
+__device__ __forceinline__ uint32_t row_of(const Rows& rows, uint32_t nrows, uint32_t chunk) {
+  if (nrows <= 1) return 0;
+  return (uint32_t)__popcll(__ballot(rows.first[threadIdx.x & 63] <= chunk)) - 1;
+}
+
+enum : uint32_t { kScaleIn = 1, kScaleOut = 2, kPadOut = 4 };
+
+// The factor of a scaled type, prepared once per workgroup from the doubles of the launch.
+template <typename T>
+struct Factor {
+  typedef double type;
+};
+template <>
+struct Factor<float> {
+  typedef float type;
+};
+template <>
+struct Factor<half_t> {
+  typedef float type;
+};
+
+// ScaleBufferCPUImpl's element (ops/collective_operations.h:91-127), as in xfer.hip.
+template <typename T>
+__device__ __forceinline__ T scaled(T x, typename Factor<T>::type s) {
+  return (T)(s * x);
+}
+template <>
+__device__ __forceinline__ half_t scaled<half_t>(half_t x, float s) {
+  return (half_t)opaque(s * (float)x);
+}
+
+// N elements on their way in (tensor type S to wire type W) and out (W to D): converted before or
+// after the wire, scaled on it (compress, then scale: horovod/torch/compression.py:49-55 before the
+// fp16 ScaleBuffer; the converting unpack scales the half and widens).  16-bit integers are summed and
+// copied but never scaled.
+template <typename W, int N>
+__device__ __forceinline__ void scale_all(Arr<W, N>& x, typename Factor<W>::type s) {
+  if constexpr (!std::is_same<W, uint16_t>::value) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) x.v[j] = scaled<W>(x.v[j], s);
+  }
+}
+template <typename S, typename W, int N>
+__device__ __forceinline__ Arr<W, N> to_wire(const Arr<S, N>& x, typename Factor<W>::type s, bool scale) {
+  Arr<W, N> y;
+#pragma unroll
+  for (int j = 0; j < N; ++j) y.v[j] = (W)x.v[j];
+  if (scale) scale_all(y, s);
+  return y;
+}
+template <typename W, typename D, int N>
+__device__ __forceinline__ Arr<D, N> from_wire(Arr<W, N> x, typename Factor<W>::type s, bool scale) {
+  if (scale) scale_all(x, s);
+  Arr<D, N> y;
+#pragma unroll
+  for (int j = 0; j < N; ++j) y.v[j] = (D)x.v[j];
+  return y;
+}
+
+template <typename S, typename D>
+constexpr int kVec = 16 / (int)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
+
+struct RanksCall {
+  void* const* outputs;
+  const void* const* inputs;  // rank-major: inputs[rank * n + entry]
+  const int64_t* counts;
+  int n;
+  uint32_t world;
+  double pre, post;
+  uint32_t flags;
+  hipStream_t stream;
+  hipEvent_t completion;
+};
+
+// Checks the arguments of a call and fills in its flags and factors (HVDHIP_ERR_OVERLAP: an output overlaps
+// another output, or an input that is not exactly its own entry's).
+int check_ranks_call(RanksCall* c, int in_dtype, int wire_dtype, int out_dtype);
+
+}  // namespace hvdhip
+
+#endif  // HVDHIP_RANKS_H

@@ -19,48 +19,12 @@
 #include <cstring>
 #include <vector>
 
-#include "internal.h"
-#include "vecmem.h"
+#include "ranks.h"
 
 namespace hvdhip {
 namespace {
 
-constexpr uint32_t kMaxRows = 64;   // one lane of a wavefront looks at each
-constexpr uint32_t kQwords = 440;   // addresses and counts: with `first` and the scalars below 4 KiB
 constexpr int kTogether = 8;        // ranks whose loads are in flight at once
-
-// first[i]: the first chunk of row i; beyond the last row a number no chunk reaches.
-// q: per row {output, elements, input of rank 0, 1 ...}.
-struct Rows {
-  uint32_t first[kMaxRows];
-  uint64_t q[kQwords];
-};
-
-enum : uint32_t { kScaleIn = 1, kScaleOut = 2, kPadOut = 4 };
-
-// The factor of a scaled type, prepared once per workgroup from the doubles of the launch.
-template <typename T>
-struct Factor {
-  typedef double type;
-};
-template <>
-struct Factor<float> {
-  typedef float type;
-};
-template <>
-struct Factor<half_t> {
-  typedef float type;
-};
-
-// ScaleBufferCPUImpl's element (ops/collective_operations.h:91-127), as in xfer.hip.
-template <typename T>
-__device__ __forceinline__ T scaled(T x, typename Factor<T>::type s) {
-  return (T)(s * x);
-}
-template <>
-__device__ __forceinline__ half_t scaled<half_t>(half_t x, float s) {
-  return (half_t)opaque(s * (float)x);
-}
 
 template <typename T, int VEC>
 __device__ __forceinline__ void add_to(Arr<T, VEC>& acc, const Arr<T, VEC>& x) {
@@ -97,41 +61,8 @@ __device__ __forceinline__ void add_to<int8_t, 16>(Arr<int8_t, 16>& acc, const A
   add_bytes(reinterpret_cast<uint8_t*>(acc.v), reinterpret_cast<const uint8_t*>(x.v));
 }
 
-// N elements on their way in (tensor type S to wire type W) and out (W to D): converted before or
-// after the wire, scaled on it (compress, then scale: horovod/torch/compression.py:49-55 before the
-// fp16 ScaleBuffer; the converting unpack scales the half and widens).  16-bit integers are summed and
-// copied but never scaled.
-template <typename W, int N>
-__device__ __forceinline__ void scale_all(Arr<W, N>& x, typename Factor<W>::type s) {
-  if constexpr (!std::is_same<W, uint16_t>::value) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) x.v[j] = scaled<W>(x.v[j], s);
-  }
-}
-template <typename S, typename W, int N>
-__device__ __forceinline__ Arr<W, N> to_wire(const Arr<S, N>& x, typename Factor<W>::type s, bool scale) {
-  Arr<W, N> y;
-#pragma unroll
-  for (int j = 0; j < N; ++j) y.v[j] = (W)x.v[j];
-  if (scale) scale_all(y, s);
-  return y;
-}
-template <typename W, typename D, int N>
-__device__ __forceinline__ Arr<D, N> from_wire(Arr<W, N> x, typename Factor<W>::type s, bool scale) {
-  if (scale) scale_all(x, s);
-  Arr<D, N> y;
-#pragma unroll
-  for (int j = 0; j < N; ++j) y.v[j] = (D)x.v[j];
-  return y;
-}
-
-template <typename S, typename D>
-constexpr int kVec = 16 / (int)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
-
 // One workgroup per chunk of kWG * kVec elements: 4 KiB of the wider side, one 16-byte access per lane
-// and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  Which
-// tensor a chunk belongs to every wavefront finds by itself: a lane per row compares the row's first
-// chunk, and the count of lanes at or below is the row.  The arguments stay in the scalar cache, so a
+// and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The arguments stay in the scalar cache, so a
 // workgroup waits for one vector load (the search) and one batch of scalar loads (its row) before its
 // data loads go out.  Two or four accesses per lane in a loop (8 and 16 KiB) are 3-10 % slower at 8 ranks
 // (BERT-large 446 -> 489 us), loads without the non-temporal hint 8 %; runs of 64 KiB to 1 MiB per XCD
@@ -143,9 +74,8 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
   constexpr uint32_t kTile = kWG * VEC;
   constexpr bool kBytes = sizeof(S) == 1;  // byte elements are read through windows (vecmem.h)
   const uint32_t chunk = xcd_tile(blockIdx.x, XcdOrder{shift, ordered});
-  uint32_t row = 0;
-  if (nrows > 1) row = (uint32_t)__popcll(__ballot(rows.first[threadIdx.x & 63] <= chunk)) - 1;
-  const uint64_t* q = rows.q + row * (world + 2);
+  const uint32_t row = row_of(rows, nrows, chunk);
+  const uint64_t* q = rows.q + row * (world + 2);  // {output, elements, input of rank 0, 1 ...}
   const uint64_t start = (uint64_t)(chunk - rows.first[row]) * kTile;
   const uint64_t left = q[1] - start;
   const uint32_t m = left < kTile ? (uint32_t)left : kTile;
@@ -193,20 +123,8 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
 
 // ---- host side ---------------------------------------------------------------------------------
 
-struct Call {
-  void* const* outputs;
-  const void* const* inputs;  // rank-major: inputs[rank * n + entry]
-  const int64_t* counts;
-  int n;
-  uint32_t world;
-  double pre, post;
-  uint32_t flags;
-  hipStream_t stream;
-  hipEvent_t completion;
-};
-
 template <typename S, typename W, typename D, int K, int ST>
-hipError_t launch_rows(const Call& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
+hipError_t launch_rows(const RanksCall& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
   constexpr uint32_t kTileBytes = kWG * kVec<S, D> * (uint32_t)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
   const XcdOrder order = xcd_order(chunks, kTileBytes);
   return launch_with(last ? c.completion : nullptr, ranks_sum_k<S, W, D, K, ST>, chunks, c.stream, order.shift,
@@ -214,7 +132,7 @@ hipError_t launch_rows(const Call& c, const Rows& rows, uint32_t nrows, uint32_t
 }
 
 template <typename S, typename W, typename D, int ST>
-hipError_t launch_by_world(const Call& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
+hipError_t launch_by_world(const RanksCall& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
   switch (c.world) {
   case 1: return launch_rows<S, W, D, 1, ST>(c, rows, nrows, chunks, last);
   case 2: return launch_rows<S, W, D, 2, ST>(c, rows, nrows, chunks, last);
@@ -230,7 +148,7 @@ hipError_t launch_by_world(const Call& c, const Rows& rows, uint32_t nrows, uint
 // Fills launches with as many rows as their arguments hold.  A tensor that would take a launch beyond
 // kMaxWorkgroups chunks is cut there and goes on in the next one.
 template <typename S, typename W, typename D>
-int run(const Call& c) {
+int run(const RanksCall& c) {
   constexpr uint64_t kTile = (uint64_t)kWG * kVec<S, D>;
   const uint32_t max_rows = std::min(kMaxRows, kQwords / (c.world + 2));
   int entry = 0;
@@ -274,7 +192,7 @@ int run(const Call& c) {
 
 // Whether an input overlaps an output anywhere but exactly at its own entry's.  Within an entry every lane
 // reads all its inputs before it stores, and no other lane touches those addresses.
-bool overlaps(const Call& c, uint64_t in_size, uint64_t out_size) {
+bool overlaps(const RanksCall& c, uint64_t in_size, uint64_t out_size) {
   struct Range {
     uint64_t lo, hi;
     int entry;
@@ -319,14 +237,9 @@ bool scalable_dtype(int dtype) {
 
 using namespace hvdhip;
 
-extern "C" int hvdhip_ranks_sum(void* const* outputs, const void* const* inputs, const int64_t* num_elements, int n,
-                                int world, int in_dtype, int wire_dtype, int out_dtype, double prescale,
-                                double postscale, unsigned flags, void* stream, void* event) {
-  if (n < 0 || (n > 0 && (!outputs || !inputs || !num_elements)))
+int hvdhip::check_ranks_call(RanksCall* c, int in_dtype, int wire_dtype, int out_dtype) {
+  if (c->n < 0 || (c->n > 0 && (!c->outputs || !c->inputs || !c->counts)))
     return fail(HVDHIP_ERR_INVALID_ARGUMENT, "bad entry arrays");
-  if (world < 1 || world > HVDHIP_RANKS_SUM_MAX_WORLD)
-    return fail(HVDHIP_ERR_INVALID_ARGUMENT, "world = %d is outside 1..%d", world, HVDHIP_RANKS_SUM_MAX_WORLD);
-  if (flags & ~HVDHIP_RANKS_SUM_PAD_OUTPUTS) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "unknown flags 0x%x", flags);
   const int64_t is = dtype_size(in_dtype), os = dtype_size(out_dtype);
   if (is < 0 || os < 0) return fail(HVDHIP_ERR_UNSUPPORTED_DTYPE, "unknown dtype");
   const bool same = in_dtype == wire_dtype && wire_dtype == out_dtype;
@@ -335,33 +248,43 @@ extern "C" int hvdhip_ranks_sum(void* const* outputs, const void* const* inputs,
   if (!same && !halves)
     return fail(HVDHIP_ERR_UNSUPPORTED_DTYPE, "dtypes %d, %d, %d: only FLOAT32 converts, to and from FLOAT16 on the wire",
                 in_dtype, wire_dtype, out_dtype);
-  if (world > 1 && wire_dtype == HVDHIP_BOOL)
+  if (c->world > 1 && wire_dtype == HVDHIP_BOOL)
     return fail(HVDHIP_ERR_UNSUPPORTED_DTYPE, "dtype %d cannot be summed", wire_dtype);
-  if ((prescale != 1.0 || postscale != 1.0) && !scalable_dtype(wire_dtype))
+  if ((c->pre != 1.0 || c->post != 1.0) && !scalable_dtype(wire_dtype))
     return fail(HVDHIP_ERR_UNSUPPORTED_DTYPE, "dtype %d cannot be scaled by a factor other than 1", wire_dtype);
-  for (int i = 0; i < n; ++i) {
-    if (num_elements[i] < 0) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "entry %d has a negative size", i);
-    if (num_elements[i] == 0) continue;
-    if (!outputs[i] || (uintptr_t)outputs[i] % (uintptr_t)os)
+  for (int i = 0; i < c->n; ++i) {
+    if (c->counts[i] < 0) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "entry %d has a negative size", i);
+    if (c->counts[i] == 0) continue;
+    if (!c->outputs[i] || (uintptr_t)c->outputs[i] % (uintptr_t)os)
       return fail(HVDHIP_ERR_INVALID_ARGUMENT, "the output of entry %d is NULL or not aligned to its element size", i);
-    for (int r = 0; r < world; ++r) {
-      const uintptr_t p = (uintptr_t)inputs[(size_t)r * (size_t)n + (size_t)i];
+    for (int r = 0; r < (int)c->world; ++r) {
+      const uintptr_t p = (uintptr_t)c->inputs[(size_t)r * (size_t)c->n + (size_t)i];
       if (!p || p % (uintptr_t)is)
         return fail(HVDHIP_ERR_INVALID_ARGUMENT, "rank %d of entry %d is NULL or not aligned to its element size", r, i);
     }
   }
-  Call c = {outputs, inputs, num_elements, n, (uint32_t)world, prescale, postscale, 0, static_cast<hipStream_t>(stream),
-            static_cast<hipEvent_t>(event)};
-  if (overlaps(c, (uint64_t)is, (uint64_t)os))
+  if (overlaps(*c, (uint64_t)is, (uint64_t)os))
     return fail(HVDHIP_ERR_OVERLAP, "an output overlaps another output or another entry's input");
-  if (prescale != 1.0) c.flags |= kScaleIn;
-  if (postscale != 1.0) c.flags |= kScaleOut;
-  if (flags & HVDHIP_RANKS_SUM_PAD_OUTPUTS) c.flags |= kPadOut;
+  if (c->pre != 1.0) c->flags |= kScaleIn;
+  if (c->post != 1.0) c->flags |= kScaleOut;
   if (wire_dtype == HVDHIP_FLOAT16) {
-    c.pre = fp16_scale_factor(prescale);
-    c.post = fp16_scale_factor(postscale);
+    c->pre = fp16_scale_factor(c->pre);
+    c->post = fp16_scale_factor(c->post);
   }
-  int rc;
+  return 0;
+}
+
+extern "C" int hvdhip_ranks_sum(void* const* outputs, const void* const* inputs, const int64_t* num_elements, int n,
+                                int world, int in_dtype, int wire_dtype, int out_dtype, double prescale,
+                                double postscale, unsigned flags, void* stream, void* event) {
+  if (world < 1 || world > HVDHIP_RANKS_SUM_MAX_WORLD)
+    return fail(HVDHIP_ERR_INVALID_ARGUMENT, "world = %d is outside 1..%d", world, HVDHIP_RANKS_SUM_MAX_WORLD);
+  if (flags & ~HVDHIP_RANKS_SUM_PAD_OUTPUTS) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "unknown flags 0x%x", flags);
+  RanksCall c = {outputs, inputs, num_elements, n, (uint32_t)world, prescale, postscale, 0,
+                 static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(event)};
+  int rc = check_ranks_call(&c, in_dtype, wire_dtype, out_dtype);
+  if (rc) return rc;
+  if (flags & HVDHIP_RANKS_SUM_PAD_OUTPUTS) c.flags |= kPadOut;
   switch (wire_dtype) {
   case HVDHIP_UINT8: case HVDHIP_BOOL: rc = run<uint8_t, uint8_t, uint8_t>(c); break;
   case HVDHIP_INT8: rc = run<int8_t, int8_t, int8_t>(c); break;

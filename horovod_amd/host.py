@@ -194,6 +194,25 @@ def ranks_sum(output_ptrs, input_ptrs, counts, world, in_dtype, wire_dtype, out_
     return True
 
 
+def adasum_ranks_workspace(counts, world, wire_dtype):
+    nbytes = lib().hvdhip_adasum_ranks_workspace(_count_array(counts), len(counts), world, wire_dtype)
+    if nbytes < 0:
+        check(int(nbytes), "hvdhip_adasum_ranks_workspace")
+    return nbytes
+
+
+def adasum_ranks(output_ptrs, input_ptrs, counts, world, in_dtype, wire_dtype, out_dtype, prescale, postscale,
+                 workspace_ptr, workspace_bytes, stream, event=None):
+    """Arguments and result of ranks_sum(), with Adasum's pairwise tree in place of the sum."""
+    rc = lib().hvdhip_adasum_ranks(_ptr_array(output_ptrs), _ptr_array(input_ptrs), _count_array(counts), len(counts),
+                                   world, in_dtype, wire_dtype, out_dtype, prescale, postscale, workspace_ptr,
+                                   workspace_bytes, stream.handle, event)
+    if rc == _ERR_OVERLAP:
+        return False
+    check(rc, "hvdhip_adasum_ranks")
+    return True
+
+
 FP16_SCALE_FP32_FACTOR = 0  # ScaleBufferCPUImpl<unsigned short, float>, ops/collective_operations.h:99-127
 FP16_SCALE_HALF_FACTOR = 1  # scale_buffer_k<__half>, ops/cuda/cuda_kernels.cu:96-136,167
 
@@ -207,5 +226,6 @@ def get_fp16_scale_mode():
 
 
 __all__ = ["Stream", "Timer", "FusionPlan", "AdasumPlan", "batched_d2d_memcpy", "batched_scaled_d2d_memcpy",
-           "scale_buffer", "reduce_sum", "reduce_sum_k", "ranks_sum", "RANKS_SUM_MAX_WORLD", "DTYPE", "FP16_SCALE_FP32_FACTOR", "FP16_SCALE_HALF_FACTOR",
+           "scale_buffer", "reduce_sum", "reduce_sum_k", "ranks_sum", "RANKS_SUM_MAX_WORLD", "adasum_ranks",
+           "adasum_ranks_workspace", "DTYPE", "FP16_SCALE_FP32_FACTOR", "FP16_SCALE_HALF_FACTOR",
            "set_fp16_scale_mode", "get_fp16_scale_mode"]

@@ -30,7 +30,6 @@ from .._lib import adapter_lib, check, dtype_size, lib
 
 SUM = 1      # ReduceOp values, common/operations.h:35-40
 ADASUM = 2
-PACK_CAST_THEN_SCALE = 1
 
 TORCH_TO_HVD = {
     torch.uint8: 0, torch.int8: 1, torch.int16: 3, torch.int32: 4, torch.int64: 5,
@@ -79,7 +78,7 @@ class Marker:
 
 class Engine:
     def __init__(self, size=1, local_size=1, peer_source=None, fusion_threshold=64 << 20, num_streams=1,
-                 batch_d2d_memcopies=True, max_plans=128):
+                 batch_d2d_memcopies=True):
         if size < 1 or local_size < 1 or size % local_size:
             raise ValueError("size must be a positive multiple of local_size")
         self.size, self.local_size, self.peer_source = size, local_size, peer_source
@@ -89,10 +88,7 @@ class Engine:
         self.slot = 0
         self.queue = []
         self.inflight = {}       # tensor name -> request, until synchronised
-        self.buffers = {}        # (slot, rank) -> torch uint8 tensor
-        self.plans = {}          # insertion-ordered: least recently used first
-        self.adasum_plans = {}
-        self.max_plans = max_plans
+        self.buffers = {}        # (slot, what for) -> torch uint8 tensor
         self.cycles = 0
         self.responses = 0       # fused responses executed so far
         self.ready = {}          # framework stream -> event recorded at the start of the current cycle
@@ -181,34 +177,14 @@ class Engine:
 
     # ---- resources ------------------------------------------------------
 
-    def _buffer(self, slot, rank, nbytes):
-        t = self.buffers.get((slot, rank))
+    def _buffer(self, slot, what, nbytes):
+        t = self.buffers.get((slot, what))
         if t is None or t.numel() < nbytes:
             if t is not None:
                 self.streams[slot].synchronize()  # queued kernels may still use the smaller buffer
             t = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device="cuda")
-            self.buffers[(slot, rank)] = t
+            self.buffers[(slot, what)] = t
         return t.data_ptr()
-
-    def _plan(self, tensors, outputs, counts, tensor_dtype, wire_dtype):
-        key = (tuple(tensors), tuple(outputs), tuple(counts), tensor_dtype, wire_dtype)
-        plan = self.plans.pop(key, None)
-        if plan is None:
-            if len(self.plans) >= self.max_plans:
-                self.plans.pop(next(iter(self.plans))).destroy()
-            plan = H.FusionPlan(tensors, outputs, counts, tensor_dtype, wire_dtype)
-        self.plans[key] = plan
-        return plan
-
-    def _adasum_plan(self, slot, layer_counts, dtype):
-        # an Adasum plan owns the partial sums of the combine in flight: one per stream slot
-        key = (slot, tuple(layer_counts), dtype)
-        plan = self.adasum_plans.get(key)
-        if plan is None:
-            if len(self.adasum_plans) >= self.max_plans:
-                self.adasum_plans.pop(next(iter(self.adasum_plans))).destroy()
-            plan = self.adasum_plans[key] = H.AdasumPlan(layer_counts, dtype)
-        return plan
 
     def _peer_tensor(self, rank, request, entry):
         if self.peer_source is None:
@@ -278,10 +254,10 @@ class Engine:
             at += (n * es + 15) // 16 * 16
         return offsets, at
 
-    def _to_buffer(self, slot, s, req, inputs, counts, offsets, nbytes):
-        """The sum of the ranks' scaled tensors in the stream slot's fusion buffer."""
+    def _to_buffer(self, slot, s, req, inputs, counts, offsets, nbytes, which=0):
+        """The sum of the ranks' scaled tensors in one of the stream slot's buffers."""
         tdt, wire = req.tensor_dtype, req.wire_dtype
-        buf = self._buffer(slot, 0, nbytes)
+        buf = self._buffer(slot, which, nbytes)
         head, rest = inputs[:H.RANKS_SUM_MAX_WORLD], inputs[H.RANKS_SUM_MAX_WORLD:]
         H.ranks_sum([buf + o for o in offsets], [p for rank in head for p in rank], counts, len(head), tdt, wire, wire,
                     req.prescale, 1.0, s, pad=True)
@@ -357,29 +333,24 @@ class Engine:
         """Ranks of one node are summed (the reduce-scatter leg of
         ops/adasum_gpu_operations.cc:174-197), then the node results are combined pairwise at
         distances 1, 2, 4 ... like the levels of Adasum::FusedAllreduce (ops/adasum/adasum.h:194-340)."""
-        wire, L = req.wire_dtype, self.local_size
-        flags = PACK_CAST_THEN_SCALE if wire != req.tensor_dtype else 0
-        plans = [self._plan(ptrs, ptrs if rank else outputs, counts, req.tensor_dtype, wire)
-                 for rank, ptrs in enumerate(inputs)]
-        nbytes = plans[0].buffer_len
-        bufs = [self._buffer(slot, rank, nbytes) for rank in range(self.size)]
-        for rank in [*range(1, self.size), 0]:
-            plans[rank].pack(bufs[rank], req.prescale, s, flags)
-        offsets = plans[0].offsets() + [nbytes]
-        es = dtype_size(wire)
-        layers = [(hi - lo) // es for lo, hi in zip(offsets, offsets[1:])]  # pad bytes are zero
-        leaders = bufs[::L]
-        for node, lead in enumerate(leaders):
-            for i in range(node * L + 1, node * L + L, 16):
-                more = bufs[i:min(i + 16, node * L + L)]
-                H.reduce_sum_k(lead, more, nbytes // es, wire, s)
-        combine = self._adasum_plan(slot, layers, wire)
-        d = 1
-        while d < len(leaders):
-            for i in range(0, len(leaders), 2 * d):
-                combine.combine(leaders[i], leaders[i + d], s)
-            d *= 2
-        plans[0].unpack(bufs[0], req.postscale, s, event=event)
+        tdt, wire, L, nodes = req.tensor_dtype, req.wire_dtype, self.local_size, self.size // self.local_size
+        if nodes == 1:
+            return self._sum(slot, s, req, inputs, outputs, counts, event)
+        offsets, nbytes = self._offsets(counts, wire)
+        source, prescale = tdt, req.prescale
+        if L > 1:
+            sums = [self._to_buffer(slot, s, req, inputs[node * L:(node + 1) * L], counts, offsets, nbytes, 2 + node)
+                    for node in range(nodes)]
+            inputs, source, prescale = [[b + o for o in offsets] for b in sums], wire, 1.0
+        flat = [p for node in inputs for p in node]
+        space = H.adasum_ranks_workspace(counts, nodes, wire)
+        work = self._buffer(slot, "adasum", space)
+        if H.adasum_ranks(outputs, flat, counts, nodes, source, wire, tdt, prescale, req.postscale, work, space, s,
+                          event=event):
+            return
+        buf = self._buffer(slot, 0, nbytes)  # outputs that share memory with other tensors
+        H.adasum_ranks([buf + o for o in offsets], flat, counts, nodes, source, wire, wire, prescale, 1.0, work, space, s)
+        self._from_buffer(buf, s, req, outputs, counts, offsets, event)
 
     # ---- completion -----------------------------------------------------
 
@@ -419,9 +390,6 @@ class Engine:
                 self.wait(r)
             except HorovodInternalError:
                 pass
-        for plan in list(self.plans.values()) + list(self.adasum_plans.values()):
-            plan.destroy()
-        self.plans, self.adasum_plans = {}, {}
         for s in self.streams:
             s.destroy()
         self.streams, self.buffers = [], {}

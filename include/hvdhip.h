@@ -402,6 +402,22 @@ int hvdhip_adasum_dot_and_norm_sqrds(const void* a, const void* b, int dtype, in
 int hvdhip_adasum_dispatch_scaled_add(int dtype, int count, double acoeff, void* a,
                                       double bcoeff, const void* b, void* stream);
 
+/* Adasum over `world` ranks (a power of two) of n fused tensors that all sit in memory this
+ * device reads, every tensor a layer of its own: what packing every rank's tensors, combining the
+ * buffers pairwise at distances 1, 2, 4 ... (Adasum::FusedAllreduce, ops/adasum/adasum.h:194-340) and
+ * unpacking the first give, with the same roundings; the order of the double sums is fixed by the
+ * sizes.  inputs, outputs, num_elements, the dtypes and factors, overlaps and event are those of
+ * hvdhip_ranks_sum(); wire_dtype is FLOAT16, FLOAT32 or FLOAT64.
+ * workspace: device memory on a 256-byte boundary of at least
+ * hvdhip_adasum_ranks_workspace() bytes (a negative return is an error code), the caller's again once the
+ * queued work is done. */
+#define HVDHIP_ADASUM_RANKS_MAX_WORLD 65536
+int64_t hvdhip_adasum_ranks_workspace(const int64_t* num_elements, int n, int world, int wire_dtype);
+int hvdhip_adasum_ranks(void* const* outputs, const void* const* inputs, const int64_t* num_elements, int n,
+                        int world, int in_dtype, int wire_dtype, int out_dtype, double prescale,
+                        double postscale, void* workspace, int64_t workspace_bytes, void* stream,
+                        void* event);
+
 /* hvdhip_adasum_combine for a single layer of count elements, for callers that cannot
  * allocate.  It has no counterpart in the reference: it exists for code under HIP graph
  * capture, tight serving loops and harnesses that forbid hipMalloc, which cannot create the

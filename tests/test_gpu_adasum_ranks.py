@@ -1,0 +1,83 @@
+"""hvdhip_adasum_ranks against the oracle's pairwise combine, level by level, at the edges of its chunks (16 KiB of
+the wire type), of the partial sums that a consumer adds itself (512 per tensor), of the tensors one launch carries
+(44 of eight ranks) and of the ranks one launch reads (8)."""
+import numpy as np
+import pytest
+import torch
+
+from horovod_amd import DTYPE
+from horovod_amd import host as H
+
+pytestmark = pytest.mark.gpu
+
+NP = {"float16": np.float16, "float32": np.float32, "float64": np.float64}
+
+
+def _tree(orc, ranks, wire, pre, post):
+    code = DTYPE[wire]
+    level = [v.astype(NP[wire]) for v in ranks]
+    level = [orc.scale_buffer(v, pre, code) if pre != 1.0 else v for v in level]
+    while len(level) > 1:
+        level = [orc.adasum_pairwise(a, b, [a.size], code)[0] for a, b in zip(level[::2], level[1::2])]
+    return orc.scale_buffer(level[0], post, code) if post != 1.0 else level[0]
+
+
+@pytest.mark.parametrize("dtype,wire", [(d, d) for d in NP] + [("float32", "float16")])
+@pytest.mark.parametrize("world,shape", [(2, "edges"), (4, "edges"), (8, "edges"), (32, "edges"), (4, "long"),
+                                         (8, "rows")])
+def test_adasum_ranks_equals_the_pairwise_tree(gpu, orc, dtype, wire, world, shape):
+    rng = np.random.default_rng(world)
+    chunk = 16384 // np.dtype(NP[wire]).itemsize
+    counts = {"edges": [1, 0, 3, chunk - 1, chunk, chunk + 1, 2 * chunk + 7, 255],
+              "long": [5, 512 * chunk, 512 * chunk + 1, 0],
+              "rows": [int(x) for x in rng.integers(0, 300, 100)]}[shape]
+    pre, post = (0.125, 0.3) if world % 8 else (1.0, 1.0)
+    host = [[rng.normal(0.0, 0.01 * (1 + r), c).astype(NP[dtype]) for c in counts] for r in range(world)]
+    # one element into the allocation each: only element alignment is promised
+    dev = [[torch.from_numpy(np.concatenate([v[:1], v])).cuda()[1 if v.size else 0:] for v in rank] for rank in host]
+    out = [torch.zeros(c + 1, dtype=dev[0][0].dtype, device="cuda") for c in counts]
+    code, wcode = DTYPE[dtype], DTYPE[wire]
+    need = H.adasum_ranks_workspace(counts, world, wcode)
+    work = torch.full((need + 256,), 255, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    flat = [t.data_ptr() for r in dev for t in r]
+    for to in ([o.data_ptr() for o in out], [t.data_ptr() for t in dev[0]]):  # and in place: rank 0's tensors
+        assert H.adasum_ranks(to, flat, counts, world, code, wcode, code, pre, post, work.data_ptr(), need, gpu.stream)
+    gpu.stream.synchronize()
+    assert bool((work[need:] == 255).all()), "wrote behind the workspace"
+    levels = world.bit_length() - 1
+    for i, c in enumerate(counts):
+        if c == 0:
+            continue
+        ranks = [host[r][i] for r in range(world)]
+        want = _tree(orc, ranks, wire, pre, post).astype(np.float64)
+        got = out[i].cpu().numpy()
+        assert got[c] == 0, "wrote behind its tensor"
+        assert np.array_equal(got[:c].view(np.uint8), dev[0][i].cpu().numpy().view(np.uint8)), (i, c)
+        diff = np.abs(got[:c].astype(np.float64) - want)
+        # The oracle adds the c products of a sum one after the other: off by up to c units of 2^-53 of |a||b|, which
+        # moves a coefficient (at most 1.5) by half of that; a rounding to the wire type that tips moves by an ulp.
+        # Both scale with the ranks' magnitudes, which a level multiplies by at most 1.5.
+        size = sum(np.abs(v.astype(np.float64)) for v in ranks) * 1.5 ** levels * pre * post
+        ulp = {"float16": 2.0 ** -10, "float32": 2.0 ** -23, "float64": 2.0 ** -52}[wire]
+        assert (diff <= levels * (ulp + (c + 64) * 2.0 ** -53) * size + 2.0 ** -24).all(), (i, c, diff.max())
+        if wire != "float64":  # a tipped rounding needs a value within about 1e-13 of a midpoint
+            assert np.count_nonzero(diff) <= 2 + 1e-5 * c, (i, c, np.count_nonzero(diff))
+
+
+def test_adasum_ranks_refuses(gpu):
+    t = torch.zeros(8192, dtype=torch.float32, device="cuda")
+    work = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
+    p, f32 = t.data_ptr(), DTYPE["float32"]
+
+    def call(outs, ins, counts, world, space, dtype=f32):
+        return H.adasum_ranks(outs, ins, counts, world, dtype, dtype, dtype, 1.0, 1.0, work.data_ptr(), space, gpu.stream)
+
+    need = H.adasum_ranks_workspace([100, 100], 2, f32)
+    assert call([p, p + 400], [p, p + 400, p + 8192, p + 8592], [100, 100], 2, need)
+    assert not call([p, p + 396], [p + 8192, p + 8592] * 2, [100, 100], 2, need)  # output over output
+    assert not call([p], [p + 4, p + 8192], [100], 2, need)                        # output over a shifted input
+    for args in (([p], [p] * 3, [100], 3, 1 << 16), ([p], [p] * 2, [100], 2, 16), ([p], [p] * 2, [100], 2, 1 << 16, DTYPE["int32"])):
+        with pytest.raises(Exception):
+            call(*args)
+    gpu.stream.synchronize()
