@@ -38,6 +38,12 @@ TORCH_TO_HVD = {
 _ADASUM_DTYPES = (6, 7, 8)
 
 
+def _current_stream():
+    """What torch.cuda.current_stream() makes its Stream object from: (stream_id, device_index, device_type).  One per
+    tensor is enough of them to matter (2.5 us for the object, 0.3 us for this)."""
+    return torch._C._cuda_getCurrentStream(torch._C._cuda_getDevice())
+
+
 class HorovodInternalError(RuntimeError):
     """An error of the op layer surfacing in the caller (horovod/common/exceptions.py:18-23)."""
 
@@ -51,17 +57,20 @@ class Entry:
 
 
 class Request:
+    __slots__ = ("kind", "entries", "op", "prescale", "postscale", "divisor", "tensor_dtype", "wire_dtype", "device",
+                 "producer", "markers", "submitted", "error", "grouped")
+
     def __init__(self, entries, op, prescale, postscale, divisor, tensor_dtype, wire_dtype, device,
-                 kind="allreduce"):
+                 kind="allreduce", grouped=False):
         self.kind = kind
         self.entries = entries
         self.op, self.prescale, self.postscale, self.divisor = op, float(prescale), float(postscale), divisor
         self.tensor_dtype, self.wire_dtype, self.device = tensor_dtype, wire_dtype, device
-        self.producer = None     # the framework stream that was current at enqueue
+        self.producer = None     # the framework stream that was current at enqueue (torch's identifiers)
         self.markers = []        # one Marker per fused response that carries one of the entries
-        self.keepalive = []      # peer tensors in flight
         self.submitted = False
         self.error = None
+        self.grouped = grouped
 
     def key(self):
         return (self.kind, self.op, self.device, self.tensor_dtype, self.wire_dtype, self.prescale, self.postscale)
@@ -70,10 +79,12 @@ class Request:
 class Marker:
     """Completion event of one fused response, shared by the requests it carried
     (ops/gpu_operations.cc:50-56 records one per response)."""
-    __slots__ = ("stream", "event", "refs")
+    __slots__ = ("stream", "event", "refs", "done", "keepalive")
 
-    def __init__(self, stream, event, refs):
+    def __init__(self, stream, event, refs, keepalive):
         self.stream, self.event, self.refs = stream, event, refs
+        self.done = False
+        self.keepalive = keepalive  # the other ranks' tensors, until the response has completed
 
 
 class Engine:
@@ -91,27 +102,28 @@ class Engine:
         self.buffers = {}        # (slot, what for) -> torch uint8 tensor
         self.cycles = 0
         self.responses = 0       # fused responses executed so far
-        self.ready = {}          # framework stream -> event recorded at the start of the current cycle
+        self.ready = {}          # framework stream -> event recorded during the current cycle
 
     # ---- queueing -------------------------------------------------------
 
     def enqueue(self, request):
+        inflight = self.inflight
         for e in request.entries:
-            if e.name in self.inflight:
+            if e.name in inflight:
                 # common/tensor_queue.cc:27-31
                 raise HorovodInternalError(
                     "Requested to allreduce a tensor with the same name as another tensor that is "
                     "currently being processed.  If you want to request another tensor, use a different "
                     "tensor name.")
         for e in request.entries:
-            self.inflight[e.name] = request
+            inflight[e.name] = request
         # The reference records a ready event per request on the framework's stream
         # (RecordReadyEvent, horovod/torch/ready_event.cc).  A cycle here runs on the caller's own
         # thread, after every enqueue it serves, so one event per producing stream and cycle, recorded
-        # when the cycle starts, orders the same work and costs one record instead of one per tensor.
+        # during the cycle, orders the same work and costs one record instead of one per tensor.
         if request.kind == "allgather":
             self._prepare_allgather(request)
-        request.producer = torch.cuda.current_stream()
+        request.producer = _current_stream()
         self.queue.append(request)
 
     def _prepare_allgather(self, request):
@@ -145,21 +157,22 @@ class Engine:
             return
         self.cycles += 1
         self.ready = {}
+        flat, sizes, keys, classes = [], [], [], {}
         for r in pending:
-            if r.producer not in self.ready:
-                ev = torch.cuda.Event()
-                ev.record(r.producer)
-                self.ready[r.producer] = ev
-        flat = [(r, e) for r in pending for e in r.entries]
+            key = classes.setdefault(r.key(), len(classes))
+            gathers = r.kind == "allgather"
+            es = dtype_size(r.tensor_dtype if gathers else r.wire_dtype)
+            for e in r.entries:
+                nbytes = (e.output.numel() if gathers else e.count) * es
+                if self.batch_d2d_memcopies and not gathers:  # no padding on that path
+                    nbytes = (nbytes + 15) // 16 * 16
+                flat.append((r, e))
+                sizes.append(nbytes)
+                keys.append(key)
         n = len(flat)
-        pad = (lambda b: 16 * ((b + 15) // 16)) if self.batch_d2d_memcopies else (lambda b: b)
-        sizes = (c_int64 * n)(*[
-            e.output.numel() * dtype_size(r.tensor_dtype) if r.kind == "allgather"  # no padding on that path
-            else pad(e.count * dtype_size(r.wire_dtype)) for r, e in flat])
-        classes = {}
-        keys = (c_int * n)(*[classes.setdefault(r.key(), len(classes)) for r, _ in flat])
         group_of = (c_int * n)()
-        ngroups = adapter_lib().hvd_adapter_fuse_keyed(sizes, keys, n, self.fusion_threshold, 0, group_of)
+        ngroups = adapter_lib().hvd_adapter_fuse_keyed((c_int64 * n)(*sizes), (c_int * n)(*keys), n,
+                                                       self.fusion_threshold, 0, group_of)
         groups = [[] for _ in range(ngroups)]
         for i in range(n):
             groups[group_of[i]].append(flat[i])
@@ -186,44 +199,51 @@ class Engine:
             self.buffers[(slot, what)] = t
         return t.data_ptr()
 
-    def _peer_tensor(self, rank, request, entry):
-        if self.peer_source is None:
-            return entry.tensor
-        t = self.peer_source(rank, entry.name, entry.tensor)
-        if (not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != entry.tensor.dtype
-                or t.numel() != entry.count or not t.is_contiguous()):
-            raise ValueError("peer_source must return a contiguous device tensor of the shape and dtype of %r"
-                             % entry.name)
-        request.keepalive.append(t)
-        return t
+    def _peers(self, group, addresses):
+        """The tensors that the other ranks pass for a group's entries; their addresses are appended rank by rank."""
+        source, dtype, peers = self.peer_source, group[0][1].tensor.dtype, []
+        for rank in range(1, self.size):
+            for _, e in group:
+                t = source(rank, e.name, e.tensor)
+                if (not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != dtype or t.numel() != e.count
+                        or not t.is_contiguous()):
+                    raise ValueError("peer_source must return a contiguous device tensor of the shape and dtype of %r"
+                                     % e.name)
+                peers.append(t)
+                addresses.append(t.data_ptr())
+        return peers
 
     # ---- one fused response --------------------------------------------
 
     def _execute(self, group):
         first = group[0][0]
-        slot, s, requests = self._begin(group)
         counts = [e.count for _, e in group]
-        # the other ranks' tensors (framework stream), then this response's stream waits for them
-        peers = [[self._peer_tensor(rank, r, e) for r, e in group] for rank in range(1, self.size)]
-        if self.peer_source is not None and peers:
-            made = torch.cuda.Event()
-            made.record()
-            check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(made.cuda_event)), "hvdhip_stream_wait_event")
-            first.keepalive.append(made)
-        inputs = [[e.tensor.data_ptr() for _, e in group]] + [[t.data_ptr() for t in ts] for ts in peers]
+        inputs = [e.tensor.data_ptr() for _, e in group]  # rank-major: inputs[rank * len(group) + entry]
+        peers = made = None
+        if self.peer_source is None:
+            inputs *= self.size
+        elif self.size > 1:
+            # the other ranks' tensors (framework stream); this response's stream waits for them, which
+            # covers what that stream did before
+            peers = self._peers(group, inputs)
+            made = _current_stream()
+            peers.append(self._record(made))
+        slot, s, requests = self._begin(group, made)
+        if made is not None:
+            self._wait_for(s, peers[-1])
         outputs = [e.output.data_ptr() for _, e in group]
         event = self._acquire(s)
         try:
             if not any(counts):
                 check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
-            elif first.op == ADASUM and peers:
+            elif first.op == ADASUM and self.size > 1:
                 self._adasum(slot, s, first, inputs, outputs, counts, event)
             else:
                 self._sum(slot, s, first, inputs, outputs, counts, event)
         except Exception:
             check(lib().hvdhip_event_release(s.handle, event), "hvdhip_event_release")
             raise
-        self._finish(s, requests, event)
+        self._finish(s, requests, event, peers)
 
     @staticmethod
     def _acquire(s):
@@ -237,8 +257,7 @@ class Engine:
         other tensor of the response."""
         tdt, wire = req.tensor_dtype, req.wire_dtype
         if self.size <= H.RANKS_SUM_MAX_WORLD:
-            flat = [p for rank in inputs for p in rank]
-            if H.ranks_sum(outputs, flat, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s, event=event):
+            if H.ranks_sum(outputs, inputs, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s, event=event):
                 return
         offsets, nbytes = self._offsets(counts, wire)
         buf = self._to_buffer(slot, s, req, inputs, counts, offsets, nbytes)
@@ -256,14 +275,15 @@ class Engine:
 
     def _to_buffer(self, slot, s, req, inputs, counts, offsets, nbytes, which=0):
         """The sum of the ranks' scaled tensors in one of the stream slot's buffers."""
-        tdt, wire = req.tensor_dtype, req.wire_dtype
+        tdt, wire, n = req.tensor_dtype, req.wire_dtype, len(counts)
         buf = self._buffer(slot, which, nbytes)
-        head, rest = inputs[:H.RANKS_SUM_MAX_WORLD], inputs[H.RANKS_SUM_MAX_WORLD:]
-        H.ranks_sum([buf + o for o in offsets], [p for rank in head for p in rank], counts, len(head), tdt, wire, wire,
-                    req.prescale, 1.0, s, pad=True)
-        for rank in rest:  # more ranks than one pass takes: one by one
+        head = min(len(inputs) // n, H.RANKS_SUM_MAX_WORLD)
+        H.ranks_sum([buf + o for o in offsets], inputs[:head * n], counts, head, tdt, wire, wire, req.prescale, 1.0, s,
+                    pad=True)
+        for at in range(head * n, len(inputs), n):  # more ranks than one pass takes: one by one
             one = self._buffer(slot, 1, nbytes)
-            H.ranks_sum([one + o for o in offsets], rank, counts, 1, tdt, wire, wire, req.prescale, 1.0, s, pad=True)
+            H.ranks_sum([one + o for o in offsets], inputs[at:at + n], counts, 1, tdt, wire, wire, req.prescale, 1.0, s,
+                        pad=True)
             H.reduce_sum(buf, one, nbytes // dtype_size(wire), wire, s)
         return buf
 
@@ -276,23 +296,35 @@ class Engine:
             H.ranks_sum([out], [buf + o], [n], 1, wire, wire, tdt, 1.0, req.postscale, s)
         check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
 
-    def _begin(self, group):
-        """Picks the stream slot of a fused response and makes it wait for the framework."""
+    @staticmethod
+    def _record(producer):
+        ev = torch.cuda.Event()
+        stream_id, device_index, device_type = producer
+        ev.record(torch.cuda.Stream(stream_id=stream_id, device_index=device_index, device_type=device_type))
+        return ev
+
+    @staticmethod
+    def _wait_for(s, ev):
+        check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(ev.cuda_event)), "hvdhip_stream_wait_event")
+
+    def _begin(self, group, covered=None):
+        """Picks the stream slot of a fused response and makes it wait for the framework's streams, all but
+        the one that the caller makes it wait for."""
         self.responses += 1
         slot, self.slot = self.slot, (self.slot + 1) % len(self.streams)
         s = self.streams[slot]
-        requests = []
-        for r, _ in group:
-            if r not in requests:
-                requests.append(r)
+        requests = list(dict.fromkeys(r for r, _ in group))
         for producer in {r.producer for r in requests}:
-            check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(self.ready[producer].cuda_event)),
-                  "hvdhip_stream_wait_event")
+            if producer == covered:
+                continue
+            if producer not in self.ready:
+                self.ready[producer] = self._record(producer)
+            self._wait_for(s, self.ready[producer])
         return slot, s, requests
 
     @staticmethod
-    def _finish(s, requests, event):
-        marker = Marker(s, event, len(requests))
+    def _finish(s, requests, event, keepalive=None):
+        marker = Marker(s, event, len(requests), keepalive)
         for r in requests:
             r.markers.append(marker)
 
@@ -339,17 +371,17 @@ class Engine:
         offsets, nbytes = self._offsets(counts, wire)
         source, prescale = tdt, req.prescale
         if L > 1:
-            sums = [self._to_buffer(slot, s, req, inputs[node * L:(node + 1) * L], counts, offsets, nbytes, 2 + node)
-                    for node in range(nodes)]
-            inputs, source, prescale = [[b + o for o in offsets] for b in sums], wire, 1.0
-        flat = [p for node in inputs for p in node]
+            ranks = L * len(counts)
+            sums = [self._to_buffer(slot, s, req, inputs[node * ranks:(node + 1) * ranks], counts, offsets, nbytes,
+                                    2 + node) for node in range(nodes)]
+            inputs, source, prescale = [b + o for b in sums for o in offsets], wire, 1.0
         space = H.adasum_ranks_workspace(counts, nodes, wire)
         work = self._buffer(slot, "adasum", space)
-        if H.adasum_ranks(outputs, flat, counts, nodes, source, wire, tdt, prescale, req.postscale, work, space, s,
+        if H.adasum_ranks(outputs, inputs, counts, nodes, source, wire, tdt, prescale, req.postscale, work, space, s,
                           event=event):
             return
         buf = self._buffer(slot, 0, nbytes)  # outputs that share memory with other tensors
-        H.adasum_ranks([buf + o for o in offsets], flat, counts, nodes, source, wire, wire, prescale, 1.0, work, space, s)
+        H.adasum_ranks([buf + o for o in offsets], inputs, counts, nodes, source, wire, wire, prescale, 1.0, work, space, s)
         self._from_buffer(buf, s, req, outputs, counts, offsets, event)
 
     # ---- completion -----------------------------------------------------
@@ -371,14 +403,15 @@ class Engine:
             self.run_cycle()
         try:
             for m in request.markers:
-                check(lib().hvdhip_event_synchronize(m.event), "hvdhip_event_synchronize")
+                if not m.done:
+                    check(lib().hvdhip_event_synchronize(m.event), "hvdhip_event_synchronize")
+                    m.done, m.keepalive = True, None
         finally:
             for m in request.markers:
                 m.refs -= 1
                 if m.refs == 0:  # the last request of the response hands the event back to its pool
                     check(lib().hvdhip_event_release(m.stream.handle, m.event), "hvdhip_event_release")
             request.markers = []
-            request.keepalive = []
             for e in request.entries:
                 self.inflight.pop(e.name, None)
         if request.error is not None:

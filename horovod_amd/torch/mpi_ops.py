@@ -178,18 +178,17 @@ def _submit(tensors, outputs, names, op, prescale_factor, postscale_factor, wire
     for t in tensors:
         _check(t)
     first = tensors[0]
+    dtype, device = first.dtype, first.device
     for t, o in zip(tensors, outputs):
-        if t.dtype != first.dtype or t.device != first.device:
+        if t is not first and (t.dtype != dtype or t.device != device):
             raise ValueError('Tensors of one grouped allreduce must share dtype and device.')
-        if o.shape != t.shape or o.dtype != t.dtype or o.device != t.device or not o.is_contiguous():
+        if o is not t and (o.shape != t.shape or o.dtype != dtype or o.device != device or not o.is_contiguous()):
             raise ValueError('Output must be a contiguous tensor of the shape, dtype and device of the input.')
-    red, pre, post = _factors(op, prescale_factor, postscale_factor,
-                              torch.float16 if wire_dtype is not None else first.dtype)
-    tdt = TORCH_TO_HVD[first.dtype]
+    red, pre, post = _factors(op, prescale_factor, postscale_factor, torch.float16 if wire_dtype is not None else dtype)
+    tdt = TORCH_TO_HVD[dtype]
     wire = tdt if wire_dtype is None else TORCH_TO_HVD[wire_dtype]
     req = Request([Entry(n, t, o) for n, t, o in zip(names, tensors, outputs)], red, pre, post, 1, tdt, wire,
-                  first.device.index)
-    req.grouped = grouped
+                  device.index, grouped=grouped)
     try:
         eng.enqueue(req)
     except RuntimeError as e:
@@ -313,7 +312,6 @@ def allgather_async(tensor, name=None):
     output = tensor.new()
     req = Request([Entry(_name(name, 'allgather'), tensor, output)], SUM, 1.0, 1.0, 1, TORCH_TO_HVD[tensor.dtype],
                   TORCH_TO_HVD[tensor.dtype], tensor.device.index, kind="allgather")
-    req.grouped = False
     try:
         eng.enqueue(req)
     except RuntimeError as e:
