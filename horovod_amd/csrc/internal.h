@@ -138,16 +138,21 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t block, XcdOrder o) {
 // without an error).  Returns the launch call's own status, for HVDHIP_CHECK_LAUNCH.
 // completion: an event to be bound to the kernel's completion signal (the launch's stop event).
 template <typename... KArgs, typename... Args>
-inline hipError_t launch_with(hipEvent_t completion, void (*kernel)(KArgs...), dim3 workgroups,
-                              hipStream_t stream, Args... args) {
+inline hipError_t launch_shaped(hipEvent_t completion, void (*kernel)(KArgs...), dim3 workgroups, uint32_t lanes,
+                                hipStream_t stream, Args... args) {
   static_assert(sizeof...(KArgs) == sizeof...(Args), "one argument per kernel parameter");
   std::tuple<KArgs...> values{KArgs(args)...};
   void* addresses[sizeof...(KArgs) ? sizeof...(KArgs) : 1];
   std::apply([&](auto&... v) { size_t i = 0; ((addresses[i++] = static_cast<void*>(&v)), ...); }, values);
   const void* handle = reinterpret_cast<const void*>(kernel);
   if (completion)
-    return hipExtLaunchKernel(handle, workgroups, dim3(kWG), addresses, 0, stream, nullptr, completion, 0);
-  return hipLaunchKernel(handle, workgroups, dim3(kWG), addresses, 0, stream);
+    return hipExtLaunchKernel(handle, workgroups, dim3(lanes), addresses, 0, stream, nullptr, completion, 0);
+  return hipLaunchKernel(handle, workgroups, dim3(lanes), addresses, 0, stream);
+}
+template <typename... KArgs, typename... Args>
+inline hipError_t launch_with(hipEvent_t completion, void (*kernel)(KArgs...), dim3 workgroups,
+                              hipStream_t stream, Args... args) {
+  return launch_shaped(completion, kernel, workgroups, kWG, stream, args...);
 }
 template <typename... KArgs, typename... Args>
 inline hipError_t launch(void (*kernel)(KArgs...), dim3 workgroups, hipStream_t stream, Args... args) {

@@ -6,8 +6,8 @@
 // summed into the first, which is unpacked -- moves every byte three times (2 per packing rank,
 // world + 1 for the sum, 2 for the unpack: 27 passes over the tensors for 8 ranks where 9 do).
 // It is bound by memory in both forms: ResNet-50's gradients (102 MB) of 8 ranks took 222 us of
-// kernels and take 160 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 2.4 ms (8 read
-// streams from HBM: 5.8-6.1 TB/s).  Results are the same to the bit: the same roundings in the
+// kernels and take 151 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 2.2 ms (8 read
+// streams from HBM: 6.1-6.5 TB/s).  Results are the same to the bit: the same roundings in the
 // same order (to the wire type after the prescale and after every rank).
 //
 // There is no table in device memory.  A launch carries the addresses of up to kMaxRows tensors
@@ -25,6 +25,13 @@ namespace hvdhip {
 namespace {
 
 constexpr int kTogether = 8;        // ranks whose loads are in flight at once
+
+// ranks_split_k: K ranks over this many wavefronts, two ranks each (the last may have one), and vectors of a rank that a
+// lane loads.
+template <int K>
+constexpr int kSplitWaves = K <= 4 ? 2 : 4;
+template <int K>
+constexpr int kSplitVecs = K == 2 * kSplitWaves<K> ? 1 : 2;
 
 template <typename T, int VEC>
 __device__ __forceinline__ void add_to(Arr<T, VEC>& acc, const Arr<T, VEC>& x) {
@@ -61,8 +68,8 @@ __device__ __forceinline__ void add_to<int8_t, 16>(Arr<int8_t, 16>& acc, const A
   add_bytes(reinterpret_cast<uint8_t*>(acc.v), reinterpret_cast<const uint8_t*>(x.v));
 }
 
-// One workgroup per chunk of kWG * kVec elements: 4 KiB of the wider side, one 16-byte access per lane
-// and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The arguments stay in the scalar cache, so a
+// For 1, 2 and more than 8 ranks.  One workgroup per chunk of kWG * kVec elements: 4 KiB of the wider side, one 16-byte
+// access per lane and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The arguments stay in the scalar cache, so a
 // workgroup waits for one vector load (the search) and one batch of scalar loads (its row) before its
 // data loads go out.  Two or four accesses per lane in a loop (8 and 16 KiB) are 3-10 % slower at 8 ranks
 // (BERT-large 446 -> 489 us), loads without the non-temporal hint 8 %; runs of 64 KiB to 1 MiB per XCD
@@ -121,35 +128,112 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
   }
 }
 
+// The same for 3 to 8 ranks, split over the wavefronts of a workgroup: wavefront w loads the tile of ranks w and
+// w + WV, all meet in LDS as wire values, and the first U wavefronts add them in rank order and store.  What bounds the
+// sum of many streams is how much of them is in flight: 2,048 workgroups of the kernel above have 64 MiB of 8 ranks under
+// way, more than latency times bandwidth by far and spread over as many DRAM pages, and stream at 6.0 TB/s; a plain
+// sum of 8 x 128 MiB gains when it is held to fewer resident wavefronts (201 -> 185 us) and most with this tile of
+// 1 KiB per rank and two loads per lane (181 us).  fp32, 8 ranks: BERT-large's layers of one response 158.5 -> 151
+// us (6.5 TB/s), with fp16 on the wire 159.5 -> 150.5, fp16 80.5 -> 76.5, ResNet-50's gradients 158 -> 151.5; 4 ranks
+// 85.8 -> 83.7, 5 ranks 106 -> 99, 6 ranks 123 -> 118, below 16 MiB per rank no difference.  With an odd number of ranks a wavefront has
+// one load to wait for, so a lane takes two vectors of each (5 ranks, one vector: 112 us); more per workgroup in a
+// loop that loads ahead is slower (4 tiles: 161 us, 8: 176).  Runs of 256 KiB per XCD gain 1-4 % at 3 to 6 ranks; with 8
+// ResNet-50's take 155 us in them.
+template <typename S, typename W, typename D, int K, int ST>
+__global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t shift, uint32_t ordered, uint32_t nrows,
+                                                                     double pre, double post, uint32_t flags,
+                                                                     Rows rows) {
+  constexpr int VEC = kVec<S, D>, WV = kSplitWaves<K>, U = kSplitVecs<K>;
+  constexpr uint32_t kTile = 64 * U * VEC;
+  constexpr bool kBytes = sizeof(S) == 1;
+  static_assert(U <= WV, "a wavefront per 64 vectors of the sum");
+  __shared__ Arr<W, VEC> lds[K][64 * U];
+  const uint32_t chunk = xcd_tile(blockIdx.x, XcdOrder{shift, ordered});
+  const uint32_t row = row_of(rows, nrows, chunk);
+  const uint64_t* q = rows.q + row * (K + 2);  // {output, elements, input of rank 0, 1 ...}
+  const uint64_t start = (uint64_t)(chunk - rows.first[row]) * kTile;
+  const uint64_t left = q[1] - start;
+  const uint32_t m = left < kTile ? (uint32_t)left : kTile;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const typename Factor<W>::type fin = (typename Factor<W>::type)pre, fout = (typename Factor<W>::type)post;
+  const bool scale_in = flags & kScaleIn, scale_out = flags & kScaleOut;
+  auto source = [&](uint32_t rank) { return as_global<const S>(q[2 + rank]) + start; };
+  const bool second = K == 2 * WV || wave + WV < K;
+  const gptr<const S> src[2] = {source(wave), source(second ? wave + WV : wave)};
+  const uint32_t nv = m / VEC;
+  auto load = [&](gptr<const S> p, uint32_t v) {
+    if constexpr (kBytes) {
+      return ldw<S, VEC>(load_window(p, m), v * 16u);
+    } else {
+      return ldv<S, VEC>(p + (size_t)v * VEC);
+    }
+  };
+  Arr<S, VEC> x[U][2];
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) {
+    const uint32_t v = u * 64 + lane;
+    if (v < nv) {
+      x[u][0] = load(src[0], v);
+      if (second) x[u][1] = load(src[1], v);
+    }
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) {
+    const uint32_t v = u * 64 + lane;
+    if (v < nv) {
+      lds[wave][v] = to_wire<S, W, VEC>(x[u][0], fin, scale_in);
+      if (second) lds[wave + WV][v] = to_wire<S, W, VEC>(x[u][1], fin, scale_in);
+    }
+  }
+  __syncthreads();
+  gptr<D> out = as_global<D>(q[0]) + start;
+  const Window win = store_window<ST>(out, m * (uint32_t)sizeof(D));
+  const uint32_t v = threadIdx.x;
+  if (v < nv) {
+    Arr<W, VEC> acc = lds[0][v];
+#pragma unroll
+    for (int k = 1; k < K; ++k) add_to<W, VEC>(acc, lds[k][v]);
+    stw<ST, D, VEC>(win, v * (uint32_t)(VEC * sizeof(D)), from_wire<W, D, VEC>(acc, fout, scale_out));
+  }
+  const uint32_t t = nv * VEC + threadIdx.x;  // fewer than VEC elements remain
+  if (t < m) {
+    auto wire = [&](uint32_t r) { return to_wire<S, W, 1>(Arr<S, 1>{source(r)[t]}, fin, scale_in); };
+    Arr<W, 1> acc = wire(0);
+    for (uint32_t r = 1; r < K; ++r) add_to<W, 1>(acc, wire(r));
+    out[t] = from_wire<W, D, 1>(acc, fout, scale_out).v[0];
+  }
+  if constexpr (ST == kStoreWT) {  // into a fusion buffer: zeros up to the next 16-byte boundary
+    const uint32_t pad = (uint32_t)(0u - (uint32_t)q[1] * (uint32_t)sizeof(D)) & 15u;
+    if (left <= kTile && threadIdx.x < pad) as_global<uint8_t>(q[0])[q[1] * sizeof(D) + threadIdx.x] = 0;
+  }
+}
+
 // ---- host side ---------------------------------------------------------------------------------
+
+// A launch of ranks_split_k for K from 3 to 8, of ranks_sum_k for K = 1, 2 and (K = 0) more than 8 ranks.
+template <int K>
+constexpr bool kSplit = K >= 3;
 
 template <typename S, typename W, typename D, int K, int ST>
 hipError_t launch_rows(const RanksCall& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
-  constexpr uint32_t kTileBytes = kWG * kVec<S, D> * (uint32_t)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
-  const XcdOrder order = xcd_order(chunks, kTileBytes);
-  return launch_with(last ? c.completion : nullptr, ranks_sum_k<S, W, D, K, ST>, chunks, c.stream, order.shift,
-                     order.ordered, nrows, c.world, c.pre, c.post, c.flags, rows);
-}
-
-template <typename S, typename W, typename D, int ST>
-hipError_t launch_by_world(const RanksCall& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
-  switch (c.world) {
-  case 1: return launch_rows<S, W, D, 1, ST>(c, rows, nrows, chunks, last);
-  case 2: return launch_rows<S, W, D, 2, ST>(c, rows, nrows, chunks, last);
-  case 3: return launch_rows<S, W, D, 3, ST>(c, rows, nrows, chunks, last);
-  case 4: return launch_rows<S, W, D, 4, ST>(c, rows, nrows, chunks, last);
-  case 5: return launch_rows<S, W, D, 5, ST>(c, rows, nrows, chunks, last);
-  case 6: return launch_rows<S, W, D, 6, ST>(c, rows, nrows, chunks, last);
-  case 7: return launch_rows<S, W, D, 7, ST>(c, rows, nrows, chunks, last);
-  default: return launch_rows<S, W, D, kTogether, ST>(c, rows, nrows, chunks, last);
+  constexpr uint32_t kVecBytes = kVec<S, D> * (uint32_t)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
+  hipEvent_t completion = last ? c.completion : nullptr;
+  if constexpr (kSplit<K>) {
+    const XcdOrder order = K < 8 ? xcd_order(chunks, 64 * kSplitVecs<K> * kVecBytes) : XcdOrder{0, 0};
+    return launch_shaped(completion, ranks_split_k<S, W, D, K, ST>, chunks, 64 * kSplitWaves<K>, c.stream, order.shift,
+                         order.ordered, nrows, c.pre, c.post, c.flags, rows);
+  } else {
+    const XcdOrder order = xcd_order(chunks, kWG * kVecBytes);
+    return launch_with(completion, ranks_sum_k<S, W, D, K ? K : kTogether, ST>, chunks, c.stream, order.shift,
+                       order.ordered, nrows, c.world, c.pre, c.post, c.flags, rows);
   }
 }
 
 // Fills launches with as many rows as their arguments hold.  A tensor that would take a launch beyond
 // kMaxWorkgroups chunks is cut there and goes on in the next one.
-template <typename S, typename W, typename D>
-int run(const RanksCall& c) {
-  constexpr uint64_t kTile = (uint64_t)kWG * kVec<S, D>;
+template <typename S, typename W, typename D, int K>
+int run_ranks(const RanksCall& c) {
+  constexpr uint64_t kTile = (uint64_t)(kSplit<K> ? 64 * kSplitVecs<K> : kWG) * kVec<S, D>;
   const uint32_t max_rows = std::min(kMaxRows, kQwords / (c.world + 2));
   int entry = 0;
   uint64_t done = 0;  // elements of the current entry that earlier launches took
@@ -183,11 +267,26 @@ int run(const RanksCall& c) {
     for (uint32_t i = nrows; i < kMaxRows; ++i) rows.first[i] = ~0u;
     const bool last = entry == c.n;
     const hipError_t status = c.flags & kPadOut
-                                  ? launch_by_world<S, W, D, kStoreWT>(c, rows, nrows, (uint32_t)chunks, last)
-                                  : launch_by_world<S, W, D, kStoreNT>(c, rows, nrows, (uint32_t)chunks, last);
+                                  ? launch_rows<S, W, D, K, kStoreWT>(c, rows, nrows, (uint32_t)chunks, last)
+                                  : launch_rows<S, W, D, K, kStoreNT>(c, rows, nrows, (uint32_t)chunks, last);
     HVDHIP_CHECK_LAUNCH("ranks_sum_k", status);
   }
   return 0;
+}
+
+template <typename S, typename W, typename D>
+int run(const RanksCall& c) {
+  switch (c.world) {
+  case 1: return run_ranks<S, W, D, 1>(c);
+  case 2: return run_ranks<S, W, D, 2>(c);
+  case 3: return run_ranks<S, W, D, 3>(c);
+  case 4: return run_ranks<S, W, D, 4>(c);
+  case 5: return run_ranks<S, W, D, 5>(c);
+  case 6: return run_ranks<S, W, D, 6>(c);
+  case 7: return run_ranks<S, W, D, 7>(c);
+  case 8: return run_ranks<S, W, D, 8>(c);
+  default: return run_ranks<S, W, D, 0>(c);
+  }
 }
 
 // Whether an input overlaps an output anywhere but exactly at its own entry's.  Within an entry every lane

@@ -60,6 +60,31 @@ def test_ranks_sum_equals_scale_sum_scale(gpu, orc, dtype, wire, world):
         assert np.array_equal(dev[0][i].cpu().numpy().view(np.uint8), want.view(np.uint8)), (i, c)
 
 
+@pytest.mark.parametrize("dtype,wire", [(d, d) for d in ("uint8", "float16", "float32", "float64")] + [("float32", "float16")])
+@pytest.mark.parametrize("world", [3, 4, 5, 6, 7, 8])
+def test_ranks_sum_at_the_edges_of_split_tiles(gpu, orc, dtype, wire, world):
+    """Tiles of 64 and 128 vectors, the ranks over two or four wavefronts of which the last may have one rank."""
+    rng = np.random.default_rng(10 + world)
+    vec = 16 // np.dtype(NP[dtype]).itemsize
+    counts = [vec - 1, vec, 63 * vec + 1] + [t * vec + d for t in (64, 128, 192, 256) for d in (-1, 0, 1)] + [9999]
+    counts = [max(1, c) for c in counts]
+    host = [[_values(rng, c, dtype) for c in counts] for _ in range(world)]
+    dev = [[torch.from_numpy(np.concatenate([v[:1], v])).cuda()[1:] for v in rank] for rank in host]
+    code, wcode = DTYPE[dtype], DTYPE[wire]
+    offs = np.cumsum([0] + [(c * np.dtype(NP[dtype]).itemsize + 15) // 16 * 16 for c in counts])
+    buf = torch.full((int(offs[-1]) + 16,), 255, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert H.ranks_sum([buf.data_ptr() + int(o) for o in offs[:-1]], [t.data_ptr() for r in dev for t in r], counts, world,
+                       code, wcode, code, 0.5, 0.3, gpu.stream, pad=True)
+    gpu.stream.synchronize()
+    image = buf.cpu().numpy()
+    assert (image[offs[-1]:] == 255).all(), "wrote behind the buffer"
+    for i, c in enumerate(counts):
+        want = _expected(orc, [host[r][i] for r in range(world)], dtype, wire, 0.5, 0.3).view(np.uint8)
+        piece = image[offs[i]:offs[i + 1]]
+        assert np.array_equal(piece[:want.size], want) and not piece[want.size:].any(), (i, c)
+
+
 def test_ranks_sum_into_and_out_of_a_buffer(gpu, orc):
     """FLOAT32 tensors into a FLOAT16 fusion buffer, pad bytes zeroed, and out again."""
     rng = np.random.default_rng(3)
