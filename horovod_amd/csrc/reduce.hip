@@ -10,7 +10,7 @@
 // while reading the resident chunk once and writing it once.
 //
 // Pure streaming: 16-byte accesses per lane, all loads of a tile in flight
-// before the first add; no LDS, no matrix cores.
+// before the first add; no matrix cores.
 #include "internal.h"
 #include "vecmem.h"
 
@@ -123,9 +123,89 @@ __global__ __launch_bounds__(kWG) void reduce_k(T* resident, uint64_t n, uint32_
   }
 }
 
+// Wavefronts over which the K + 1 streams are split, two or three each, and vectors of a stream that a lane loads.
+template <int K>
+constexpr int kSplitWaves = K <= 3 ? 2 : 4;
+template <int K>
+constexpr int kSplitVecs = (K + 1) % kSplitWaves<K> == 0 ? 1 : 2;
+
+// The same sum with the streams split over the wavefronts of a workgroup: wavefront w loads its tile of streams
+// w, w + WV ... (stream 0 is the resident chunk), all meet in LDS, and the first U wavefronts add them in peer order
+// and store.  It has a quarter of reduce_k's bytes under way (2,048 workgroups of 1 KiB per stream instead of 4), which
+// the memory serves faster once they are more than latency times bandwidth: 33 million fp32 and 7 peers 175 -> 170 us
+// (7.0 TB/s), 3 peers 95.5 -> 90.8, 5 peers 138 -> 129, 8 peers 194.5 -> 188, 15 peers 370 -> 357; fp16 and 7 peers
+// 88.6 -> 86.7.  A wavefront with one stream less than another waits for less, so there a lane takes two vectors.
+template <typename T, int K, int ST>
+__global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* resident, uint64_t n, uint32_t shift,
+                                                                      uint32_t ordered, const T* p0, const T* p1,
+                                                                      const T* p2, const T* p3, const T* p4,
+                                                                      const T* p5, const T* p6, const T* p7) {
+  constexpr int VEC = 16 / (int)sizeof(T), WV = kSplitWaves<K>, U = kSplitVecs<K>, R = K + 1, L = (R + WV - 1) / WV;
+  constexpr uint32_t kTile = 64 * U * VEC;
+  typedef Arr<T, VEC> V;
+  __shared__ V lds[R][64 * U];
+  const T* const ps[kMaxK + 1] = {resident, p0, p1, p2, p3, p4, p5, p6, p7};
+  const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
+  const uint64_t left = n - start;
+  const uint32_t m = left < kTile ? (uint32_t)left : kTile;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nv = m / VEC;
+#pragma unroll
+  for (int w = 0; w < WV; ++w) {  // a branch per wavefront keeps the streams' addresses in scalar registers
+    if (wave != (uint32_t)w) continue;
+    V x[U][L];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) {
+        const uint32_t v = u * 64 + lane;
+        if (w + i * WV < R && v < nv) {
+          gptr<const T> p = as_global(ps[w + i * WV] + start);
+          if constexpr (sizeof(T) == 1) {
+            x[u][i] = ldw<T, VEC>(load_window(p, m), v * 16u);
+          } else {
+            x[u][i] = ldv<T, VEC>(p + (size_t)v * VEC);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) {
+        const uint32_t v = u * 64 + lane;
+        if (w + i * WV < R && v < nv) lds[w + i * WV][v] = x[u][i];
+      }
+    }
+  }
+  __syncthreads();
+  gptr<T> r = as_global(resident + start);
+  const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
+  const uint32_t v = threadIdx.x;
+  if (v < nv) {
+    V acc = lds[0][v];
+#pragma unroll
+    for (int k = 1; k < R; ++k) accumulate<T, VEC>(acc, lds[k][v]);
+    stw<ST, T, VEC>(out, v * 16u, acc);
+  }
+  const uint32_t t = nv * VEC + threadIdx.x;
+  if (t < m) {
+    T acc = r[t];
+#pragma unroll
+    for (int k = 1; k < R; ++k) acc = Add<T>::f(acc, as_global(ps[k] + start)[t]);
+    r[t] = acc;
+  }
+}
+
+// Streams of this many bytes between them are summed by reduce_split_k, from three peers on.  Below, the device holds
+// reduce_k's whole grid at once and its longer way through LDS shows: 3 peers of 8 MB 8.0 us and 8.4 split, of 32 MB
+// 24.8 and 24.5; 7 peers of 4.2 MB 8.35 and 8.4, of 8.1 MB (fp16) 13.55 and 13.4, of 16 MB 24.2 and 23.5.
+constexpr uint64_t kSplitFrom = 48ull << 20;
+
 template <typename T, int K>
 int launch_k(void* resident, const void* const* incoming, int64_t n, hipStream_t stream) {
-  const uint32_t tile = chunk_bytes(Family::kReduce) / (uint32_t)sizeof(T);
+  const bool split = K >= 3 && (uint64_t)n * sizeof(T) * (K + 1) >= kSplitFrom;
+  const uint32_t tile = split ? 64 * kSplitVecs<K> * 16 / (uint32_t)sizeof(T)
+                              : chunk_bytes(Family::kReduce) / (uint32_t)sizeof(T);
   uint64_t done = 0, left = (uint64_t)n;
   while (left > 0) {  // one launch unless the chunk needs more than kMaxWorkgroups workgroups
     const uint64_t slice = left < kMaxWorkgroups * tile ? left : kMaxWorkgroups * tile;
@@ -134,6 +214,12 @@ int launch_k(void* resident, const void* const* incoming, int64_t n, hipStream_t
     for (int k = 0; k < kMaxK; ++k) p[k] = k < K ? static_cast<const T*>(incoming[k]) + done : nullptr;
     const XcdOrder order = xcd_order(blocks, tile * (uint32_t)sizeof(T));
     const hipError_t status = with_store_policy(K <= 2 ? Stores::kReduceFew : Stores::kReduceMany, [&](auto st) {
+      if constexpr (K >= 3) {
+        if (split)
+          return launch_shaped(nullptr, reduce_split_k<T, K, decltype(st)::value>, blocks, 64 * kSplitWaves<K>, stream,
+                               static_cast<T*>(resident) + done, slice, order.shift, order.ordered, p[0], p[1], p[2],
+                               p[3], p[4], p[5], p[6], p[7]);
+      }
       return launch(reduce_k<T, K, decltype(st)::value>, blocks, stream, static_cast<T*>(resident) + done, slice,
                     tile, order.shift, order.ordered, 0u, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]);
     });

@@ -149,3 +149,24 @@ def test_tile_order_across_xcd_groups(gpu, orc, dtype, n_tiles):
     assert np.all(out[n * es:] == 0x5A)
     gpu.H.reduce_sum(d_v.data_ptr(), d_p.data_ptr(), n, dtype, gpu.stream)
     assert np.array_equal(gpu.download(d_v)[:n * es], orc.sum(_raw(p), _raw(v), dtype).view(np.uint8))
+
+
+@pytest.mark.parametrize("dtype", [U8, F16, F32, F64])
+@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8, 11])
+def test_reduce_sum_k_of_streams_split_over_wavefronts(gpu, orc, dtype, k):
+    """From 48 MiB of all streams on: tiles of 64 or 128 vectors, at a size that they divide, one element either side
+    of it, and with a ragged end; the elements behind the chunk stay."""
+    rng = np.random.default_rng(k)
+    es = SIZE_OF[dtype]
+    base = ((48 << 20) // (min(k, 8) + 1) // es // (2048 // es) + 1) * (2048 // es)
+    host = [(rng.integers(0, 100, base + 80) * (1 if dtype == U8 else 0.37)).astype(NP_OF[dtype]) for _ in range(k + 1)]
+    peers = [gpu.upload(h) for h in host[1:]]
+    for n in (base - 1, base, base + 1, base + 77):
+        resident = gpu.upload(host[0])
+        gpu.H.reduce_sum_k(resident.data_ptr(), [p.data_ptr() for p in peers], n, dtype, gpu.stream)
+        want = _raw(host[0]).copy()
+        total = want[:n].copy()
+        for h in host[1:]:
+            total = orc.sum(_raw(h)[:n], total, dtype)
+        want[:n] = total
+        assert np.array_equal(gpu.download(resident), want.view(np.uint8)), n
