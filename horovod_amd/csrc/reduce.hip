@@ -11,6 +11,8 @@
 //
 // Pure streaming: 16-byte accesses per lane, all loads of a tile in flight
 // before the first add; no matrix cores.
+#include <algorithm>
+
 #include "internal.h"
 #include "vecmem.h"
 
@@ -196,6 +198,82 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
   }
 }
 
+// Nine to fifteen peers in one launch: half as many wavefronts as streams, two streams each (the last may have one).
+// In two launches of up to eight peers the resident chunk is written and read once more: 33 million fp32 and 9 peers
+// 242 us in two, 210 in one (6.9 TB/s), 10 peers 259 and 226, 15 peers 357 and 349, fp16 and 12 peers 154 and 137;
+// 300,000 fp32 and 9 peers 10 and 6.4.  (With eight wavefronts for any number 10 peers take 267 us.)
+constexpr int kMostWaves = 8;
+constexpr int kManyStreams = 2 * kMostWaves;
+template <typename T>
+struct Streams {
+  const T* p[kManyStreams];  // the resident chunk, then the peers
+};
+template <typename T, int ST>
+__global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, uint64_t n, uint32_t shift,
+                                                                 uint32_t ordered, uint32_t streams, Streams<T> s) {
+  constexpr int VEC = 16 / (int)sizeof(T);
+  constexpr uint32_t kTile = 64 * VEC;
+  typedef Arr<T, VEC> V;
+  __shared__ V lds[kManyStreams][64];
+  const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
+  const uint64_t left = n - start;
+  const uint32_t m = left < kTile ? (uint32_t)left : kTile;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nv = m / VEC, waves = (streams + 1) / 2;
+#pragma unroll
+  for (uint32_t w = 0; w < kMostWaves; ++w) {  // as above
+    if (wave != w || lane >= nv) continue;
+    V x[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      if (w + i * waves < streams) {
+        gptr<const T> p = as_global(s.p[w + i * waves] + start);
+        if constexpr (sizeof(T) == 1) {
+          x[i] = ldw<T, VEC>(load_window(p, m), lane * 16u);
+        } else {
+          x[i] = ldv<T, VEC>(p + (size_t)lane * VEC);
+        }
+      }
+    }
+    lds[w][lane] = x[0];
+    if (w + waves < streams) lds[w + waves][lane] = x[1];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  gptr<T> r = as_global(resident + start);
+  const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
+  if (lane < nv) {
+    V acc = lds[0][lane];
+    for (uint32_t k = 1; k < streams; ++k) accumulate<T, VEC>(acc, lds[k][lane]);
+    stw<ST, T, VEC>(out, lane * 16u, acc);
+  }
+  const uint32_t t = nv * VEC + lane;
+  if (t < m) {
+    T acc = r[t];
+    for (uint32_t k = 1; k < streams; ++k) acc = Add<T>::f(acc, as_global(s.p[k] + start)[t]);
+    r[t] = acc;
+  }
+}
+
+template <typename T>
+int launch_many(void* resident, const void* const* incoming, int k, int64_t n, hipStream_t stream) {
+  const uint32_t tile = 64 * 16 / (uint32_t)sizeof(T);
+  for (uint64_t done = 0; done < (uint64_t)n;) {
+    const uint64_t slice = std::min((uint64_t)n - done, kMaxWorkgroups / 2 * tile);  // twice the lanes of the others
+    const uint32_t blocks = (uint32_t)((slice + tile - 1) / tile);
+    Streams<T> s = {};
+    s.p[0] = static_cast<T*>(resident) + done;
+    for (int i = 0; i < k; ++i) s.p[i + 1] = static_cast<const T*>(incoming[i]) + done;
+    const XcdOrder order = xcd_order(blocks, tile * (uint32_t)sizeof(T));
+    const hipError_t status = with_store_policy(Stores::kReduceMany, [&](auto st) {
+      return launch_shaped(nullptr, reduce_many_k<T, decltype(st)::value>, blocks, 64 * (uint32_t)(k / 2 + 1), stream,
+                           static_cast<T*>(resident) + done, slice, order.shift, order.ordered, (uint32_t)(k + 1), s);
+    });
+    HVDHIP_CHECK_LAUNCH("reduce_many_k", status);
+    done += slice;
+  }
+  return 0;
+}
+
 // Streams of this many bytes between them are summed by reduce_split_k, from three peers on.  Below, the device holds
 // reduce_k's whole grid at once and its longer way through LDS shows: 3 peers of 8 MB 8.0 us and 8.4 split, of 32 MB
 // 24.8 and 24.5; 7 peers of 4.2 MB 8.35 and 8.4, of 8.1 MB (fp16) 13.55 and 13.4, of 16 MB 24.2 and 23.5.
@@ -232,6 +310,7 @@ int launch_k(void* resident, const void* const* incoming, int64_t n, hipStream_t
 
 template <typename T>
 int launch_t(void* resident, const void* const* incoming, int k, int64_t n, hipStream_t stream) {
+  if (k > kMaxK && k < kManyStreams) return launch_many<T>(resident, incoming, k, n, stream);
   while (k > 0) {
     int rc;
     int step = k < kMaxK ? k : kMaxK;

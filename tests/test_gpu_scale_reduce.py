@@ -152,7 +152,7 @@ def test_tile_order_across_xcd_groups(gpu, orc, dtype, n_tiles):
 
 
 @pytest.mark.parametrize("dtype", [U8, F16, F32, F64])
-@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8, 11])
+@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8])
 def test_reduce_sum_k_of_streams_split_over_wavefronts(gpu, orc, dtype, k):
     """From 48 MiB of all streams on: tiles of 64 or 128 vectors, at a size that they divide, one element either side
     of it, and with a ragged end; the elements behind the chunk stay."""
@@ -170,3 +170,22 @@ def test_reduce_sum_k_of_streams_split_over_wavefronts(gpu, orc, dtype, k):
             total = orc.sum(_raw(h)[:n], total, dtype)
         want[:n] = total
         assert np.array_equal(gpu.download(resident), want.view(np.uint8)), n
+
+
+@pytest.mark.parametrize("dtype", [U8, F16, F32, F64])
+@pytest.mark.parametrize("k", [9, 10, 15])
+def test_reduce_sum_k_of_nine_to_fifteen_peers_in_one_launch(gpu, orc, dtype, k):
+    """At the edges of the 1 KiB tile; addresses aligned to an element only, the elements behind the chunk stay."""
+    rng = np.random.default_rng(k)
+    tile = 1024 // SIZE_OF[dtype]
+    for n in (1, 16 // SIZE_OF[dtype], tile - 1, tile, tile + 1, 40 * tile + 3):
+        host = [_vals(rng, n + 2, dtype, 1e-3) for _ in range(k + 1)]
+        dev = [gpu.upload(h) for h in host]
+        at = [d.data_ptr() + SIZE_OF[dtype] for d in dev]
+        gpu.H.reduce_sum_k(at[0], at[1:], n, dtype, gpu.stream)
+        want = _raw(host[0]).copy()
+        total = want[1:-1].copy()
+        for h in host[1:]:
+            total = orc.sum(np.ascontiguousarray(_raw(h)[1:-1]), total, dtype)
+        want[1:-1] = total
+        assert np.array_equal(gpu.download(dev[0]), want.view(np.uint8)), n
