@@ -64,7 +64,7 @@ __device__ __forceinline__ void accumulate<uint8_t, 16>(Arr<uint8_t, 16>& acc, c
   __builtin_memcpy(acc.v, a, 16);
 }
 
-constexpr int kMaxK = 8;  // peers per launch; more are folded in by further launches
+constexpr int kMaxK = 8;  // peers per launch of reduce_k and reduce_split_k (reduce_many_k takes 9 to 15)
 
 // Workgroup b accumulates K peers into tile t = xcd_tile(b), elements [t*tile, (t+1)*tile).
 //
