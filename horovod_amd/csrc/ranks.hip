@@ -69,11 +69,11 @@ __device__ __forceinline__ void add_to<int8_t, 16>(Arr<int8_t, 16>& acc, const A
 }
 
 // For 1, 2 and more than 8 ranks.  One workgroup per chunk of kWG * kVec elements: 4 KiB of the wider side, one 16-byte
-// access per lane and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The arguments stay in the scalar cache, so a
-// workgroup waits for one vector load (the search) and one batch of scalar loads (its row) before its
-// data loads go out.  Two or four accesses per lane in a loop (8 and 16 KiB) are 3-10 % slower at 8 ranks
-// (BERT-large 446 -> 489 us), loads without the non-temporal hint 8 %; runs of 64 KiB to 1 MiB per XCD
-// measure within 2 % of each other.
+// access per lane and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The
+// arguments stay in the scalar cache, so a workgroup waits for one vector load (the search) and one batch of scalar
+// loads (its row) before its data loads go out.  Two or four accesses per lane in a loop (8 and 16 KiB) are 3-10 %
+// slower at 8 ranks (BERT-large 446 -> 489 us), loads without the non-temporal hint 8 %; runs of 64 KiB to 1 MiB per
+// XCD measure within 2 % of each other.
 template <typename S, typename W, typename D, int K, int ST>
 __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t ordered, uint32_t nrows, uint32_t world,
                                                    double pre, double post, uint32_t flags, Rows rows) {
@@ -135,10 +135,10 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
 // sum of 8 x 128 MiB gains when it is held to fewer resident wavefronts (201 -> 185 us) and most with this tile of
 // 1 KiB per rank and two loads per lane (181 us).  fp32, 8 ranks: BERT-large's layers of one response 158.5 -> 151
 // us (6.5 TB/s), with fp16 on the wire 159.5 -> 150.5, fp16 80.5 -> 76.5, ResNet-50's gradients 158 -> 151.5; 4 ranks
-// 85.8 -> 83.7, 5 ranks 106 -> 99, 6 ranks 123 -> 118, below 16 MiB per rank no difference.  With an odd number of ranks a wavefront has
-// one load to wait for, so a lane takes two vectors of each (5 ranks, one vector: 112 us); more per workgroup in a
-// loop that loads ahead is slower (4 tiles: 161 us, 8: 176).  Runs of 256 KiB per XCD gain 1-4 % at 3 to 6 ranks; with 8
-// ResNet-50's take 155 us in them.
+// 85.8 -> 83.7, 5 ranks 106 -> 99, 6 ranks 123 -> 118, below 16 MiB per rank no difference.  With an odd number of
+// ranks a wavefront has one load to wait for, so a lane takes two vectors of each (5 ranks, one vector: 112 us); more
+// per workgroup in a loop that loads ahead is slower (4 tiles: 161 us, 8: 176).  Runs of 256 KiB per XCD gain 1-4 % at
+// 3 to 6 ranks; with 8 ResNet-50's take 155 us in them.
 template <typename S, typename W, typename D, int K, int ST>
 __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t shift, uint32_t ordered, uint32_t nrows,
                                                                      double pre, double post, uint32_t flags,

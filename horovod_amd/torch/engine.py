@@ -257,7 +257,8 @@ class Engine:
         other tensor of the response."""
         tdt, wire = req.tensor_dtype, req.wire_dtype
         if self.size <= H.RANKS_SUM_MAX_WORLD:
-            if H.ranks_sum(outputs, inputs, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s, event=event):
+            if H.ranks_sum(outputs, inputs, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s,
+                           event=event):
                 return
         offsets, nbytes = self._offsets(counts, wire)
         buf = self._to_buffer(slot, s, req, inputs, counts, offsets, nbytes)
