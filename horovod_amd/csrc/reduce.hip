@@ -125,6 +125,20 @@ __global__ __launch_bounds__(kWG) void reduce_k(T* resident, uint64_t n, uint32_
   }
 }
 
+// Sixteen bytes of a stream on their way through LDS: one register quadruple for every type.  As an Arr of bytes the
+// compiler takes a load apart into sixteen registers wherever two branches meet, and waits for it to do so, one load
+// after the other: 512 MiB of uint8 streams, 5 peers 112 us and 86 in this form, 8 peers 142 and 86.
+typedef RawSel<16>::type Quad;
+template <typename T>
+__device__ __forceinline__ Quad load_quad(gptr<const T> p, uint32_t bytes, uint32_t v) {
+  if constexpr (sizeof(T) == 1) {
+    return __builtin_bit_cast(Quad, ldw<T, 16>(load_window(p, bytes), v * 16u));
+  } else {
+    constexpr int VEC = 16 / (int)sizeof(T);
+    return __builtin_bit_cast(Quad, ldv<T, VEC>(p + (size_t)v * VEC));
+  }
+}
+
 // Wavefronts over which the K + 1 streams are split, two or three each, and vectors of a stream that a lane loads.
 template <int K>
 constexpr int kSplitWaves = K <= 3 ? 2 : 4;
@@ -145,7 +159,7 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
   constexpr int VEC = 16 / (int)sizeof(T), WV = kSplitWaves<K>, U = kSplitVecs<K>, R = K + 1, L = (R + WV - 1) / WV;
   constexpr uint32_t kTile = 64 * U * VEC;
   typedef Arr<T, VEC> V;
-  __shared__ V lds[R][64 * U];
+  __shared__ Quad lds[R][64 * U];
   const T* const ps[kMaxK + 1] = {resident, p0, p1, p2, p3, p4, p5, p6, p7};
   const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
   const uint64_t left = n - start;
@@ -154,20 +168,13 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
 #pragma unroll
   for (int w = 0; w < WV; ++w) {  // a branch per wavefront keeps the streams' addresses in scalar registers
     if (wave != (uint32_t)w) continue;
-    V x[U][L];
+    Quad x[U][L];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int i = 0; i < L; ++i) {
         const uint32_t v = u * 64 + lane;
-        if (w + i * WV < R && v < nv) {
-          gptr<const T> p = as_global(ps[w + i * WV] + start);
-          if constexpr (sizeof(T) == 1) {
-            x[u][i] = ldw<T, VEC>(load_window(p, m), v * 16u);
-          } else {
-            x[u][i] = ldv<T, VEC>(p + (size_t)v * VEC);
-          }
-        }
+        if (w + i * WV < R && v < nv) x[u][i] = load_quad<T>(as_global(ps[w + i * WV] + start), m, v);
       }
     }
 #pragma unroll
@@ -184,9 +191,9 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
   const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
   const uint32_t v = threadIdx.x;
   if (v < nv) {
-    V acc = lds[0][v];
+    V acc = __builtin_bit_cast(V, lds[0][v]);
 #pragma unroll
-    for (int k = 1; k < R; ++k) accumulate<T, VEC>(acc, lds[k][v]);
+    for (int k = 1; k < R; ++k) accumulate<T, VEC>(acc, __builtin_bit_cast(V, lds[k][v]));
     stw<ST, T, VEC>(out, v * 16u, acc);
   }
   const uint32_t t = nv * VEC + threadIdx.x;
@@ -200,8 +207,8 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
 
 // Nine to fifteen peers in one launch: half as many wavefronts as streams, two streams each (the last may have one).
 // In two launches of up to eight peers the resident chunk is written and read once more: 33 million fp32 and 9 peers
-// 242 us in two, 210 in one (6.9 TB/s), 10 peers 259 and 226, 15 peers 357 and 349, fp16 and 12 peers 154 and 137;
-// 300,000 fp32 and 9 peers 10 and 6.4.  (With eight wavefronts for any number 10 peers take 267 us.)
+// 242 us in two, 210 in one (6.9 TB/s), 10 peers 259 and 226, 15 peers 357 and 337, fp16 and 12 peers 154 and 137,
+// uint8 and 12 peers of 40 million 96 and 86; 300,000 fp32 and 9 peers 10 and 6.4.  (With eight wavefronts for any number 10 peers take 267 us.)
 constexpr int kMostWaves = 8;
 constexpr int kManyStreams = 2 * kMostWaves;
 template <typename T>
@@ -214,7 +221,7 @@ __global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, ui
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr uint32_t kTile = 64 * VEC;
   typedef Arr<T, VEC> V;
-  __shared__ V lds[kManyStreams][64];
+  __shared__ Quad lds[kManyStreams][64];
   const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
   const uint64_t left = n - start;
   const uint32_t m = left < kTile ? (uint32_t)left : kTile;
@@ -222,28 +229,21 @@ __global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, ui
 #pragma unroll
   for (uint32_t w = 0; w < kMostWaves; ++w) {  // as above
     if (wave != w || lane >= nv) continue;
-    V x[2];
-#pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-      if (w + i * waves < streams) {
-        gptr<const T> p = as_global(s.p[w + i * waves] + start);
-        if constexpr (sizeof(T) == 1) {
-          x[i] = ldw<T, VEC>(load_window(p, m), lane * 16u);
-        } else {
-          x[i] = ldv<T, VEC>(p + (size_t)lane * VEC);
-        }
-      }
-    }
-    lds[w][lane] = x[0];
-    if (w + waves < streams) lds[w + waves][lane] = x[1];
+    // The last wavefront's second stream may be its first once more: a branch there has the compiler wait for
+    // the first before it asks for the second.
+    const uint32_t other = w + waves < streams ? w + waves : w;
+    const Quad x = load_quad<T>(as_global(s.p[w] + start), m, lane);
+    const Quad y = load_quad<T>(as_global(s.p[other] + start), m, lane);
+    lds[w][lane] = x;
+    lds[other][lane] = y;
   }
   __syncthreads();
   if (wave != 0) return;
   gptr<T> r = as_global(resident + start);
   const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
   if (lane < nv) {
-    V acc = lds[0][lane];
-    for (uint32_t k = 1; k < streams; ++k) accumulate<T, VEC>(acc, lds[k][lane]);
+    V acc = __builtin_bit_cast(V, lds[0][lane]);
+    for (uint32_t k = 1; k < streams; ++k) accumulate<T, VEC>(acc, __builtin_bit_cast(V, lds[k][lane]));
     stw<ST, T, VEC>(out, lane * 16u, acc);
   }
   const uint32_t t = nv * VEC + lane;

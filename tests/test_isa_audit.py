@@ -153,3 +153,26 @@ def test_contiguous_kernels_reach_their_first_load_without_a_scalar_branch(kerne
         assert sum(op == "s_waitcnt" for op in head) <= 2, (name, head)
         checked += 1
     assert checked >= 100, checked
+
+
+def test_split_sums_ask_for_all_their_streams_before_they_wait(kernels):
+    """A wavefront of reduce_split_k or reduce_many_k has its loads in flight together: no wait for everything
+    outstanding stands between two of them, other than behind the stores to LDS that end a wavefront's part."""
+    checked = 0
+    for name, lines in kernels.items():
+        if "reduce_split_k" not in name and "reduce_many_k" not in name:
+            continue
+        loads, waited = 0, False  # since the last store to LDS
+        for ins in lines:
+            op = ins.split()[0]
+            if op in ("global_load_dwordx4", "buffer_load_dwordx4"):
+                assert not waited, name
+                loads += 1
+            elif op.startswith("ds_write"):
+                loads, waited = 0, False
+            elif op == "s_waitcnt" and "vmcnt(0)" in ins:
+                waited = loads > 0
+            elif op == "s_barrier":
+                break
+        checked += 1
+    assert checked >= 98, checked
