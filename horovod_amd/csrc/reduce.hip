@@ -275,13 +275,17 @@ int launch_many(void* resident, const void* const* incoming, int k, int64_t n, h
 }
 
 // Streams of this many bytes between them are summed by reduce_split_k, from three peers on.  Below, the device holds
-// reduce_k's whole grid at once and its longer way through LDS shows: 3 peers of 8 MB 8.0 us and 8.4 split, of 32 MB
-// 24.8 and 24.5; 7 peers of 4.2 MB 8.35 and 8.4, of 8.1 MB (fp16) 13.55 and 13.4, of 16 MB 24.2 and 23.5.
-constexpr uint64_t kSplitFrom = 48ull << 20;
+// reduce_k's whole grid at once and its longer way through LDS shows, above all where the streams still lie in the
+// Infinity Cache.  fp32, us of a launch over the same buffers again: 3 peers and 64 MiB 9.4 and 10.2 split, 128 MiB 20.2
+// and 21.1, 192 MiB 33.8 and 32.8; 5 peers and 48 MiB 7.2 and 7.5, 96 MiB 15.0 and 14.7; 6 peers and 64 MiB 9.6 and
+// 10.1; 8 peers and 64 MiB 9.7 and 10.5, 96 MiB the same; 7 peers and 64 MiB 9.5 and 9.3, 96 MiB 14.8 and 14.3.  Over
+// buffers that take turns: 3 peers and 64 MiB 12.2 and 12.6, 192 MiB 38.8 and 38.0; 7 peers and 96 MiB 17.8 and 17.3.
+template <int K>
+constexpr uint64_t kSplitFrom = (K == 3 ? 192ull : 96ull) << 20;
 
 template <typename T, int K>
 int launch_k(void* resident, const void* const* incoming, int64_t n, hipStream_t stream) {
-  const bool split = K >= 3 && (uint64_t)n * sizeof(T) * (K + 1) >= kSplitFrom;
+  const bool split = K >= 3 && (uint64_t)n * sizeof(T) * (K + 1) >= kSplitFrom<K>;
   const uint32_t tile = split ? 64 * kSplitVecs<K> * 16 / (uint32_t)sizeof(T)
                               : chunk_bytes(Family::kReduce) / (uint32_t)sizeof(T);
   uint64_t done = 0, left = (uint64_t)n;
