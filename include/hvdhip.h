@@ -333,7 +333,8 @@ int hvdhip_reduce_sum_k(void* resident, const void* const* incoming, int k, int6
  * value alone.  The three dtypes are equal, or the wire is FLOAT16 and the others
  * FLOAT16 or FLOAT32 (converted first, scaled as FLOAT16: the order of
  * HVDHIP_PACK_CAST_THEN_SCALE and of the converting unpack).  With world == 1 this
- * is a scaled batched copy.
+ * is a scaled batched copy, and an output that is its input, of the same type and
+ * with factors of 1, is left alone.
  *
  * An output may be one of its own entry's inputs; any other overlap between an
  * output and an output or input returns HVDHIP_ERR_OVERLAP and nothing is launched.
