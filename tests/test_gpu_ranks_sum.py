@@ -85,6 +85,31 @@ def test_ranks_sum_at_the_edges_of_split_tiles(gpu, orc, dtype, wire, world):
         assert np.array_equal(piece[:want.size], want) and not piece[want.size:].any(), (i, c)
 
 
+@pytest.mark.parametrize("dtype,wire", [("uint8", "uint8"), ("int64", "int64"), ("float16", "float16"), ("float32", "float32"),
+                                        ("float64", "float64"), ("float32", "float16")])
+@pytest.mark.parametrize("world", [9, 10, 11, 12, 15, 16, 17, 23, 31, 64, 255, 256])
+def test_ranks_sum_in_batches_of_eight_four_two_and_one(gpu, orc, dtype, wire, world):
+    """Every remainder of the ranks beyond eight, for whole vectors and for the elements behind the last; factors that
+    are no powers of two, so that a product that was not rounded before its addition would show."""
+    rng = np.random.default_rng(world)
+    vec = 16 // np.dtype(NP[dtype]).itemsize
+    counts = [1, vec, vec + 1, 2 * vec - 1, 256 * vec + vec - 1, 300]
+    pre, post = (0.3, 0.7) if dtype.startswith("float") else (1.0, 1.0)
+    host = [[_values(rng, c, dtype) for c in counts] for _ in range(world)]
+    dev = [[torch.from_numpy(np.concatenate([v[:1], v])).cuda()[1:] for v in rank] for rank in host]
+    out = [torch.zeros(c + 1, dtype=dev[0][0].dtype, device="cuda") for c in counts]
+    torch.cuda.synchronize()
+    code, wcode = DTYPE[dtype], DTYPE[wire]
+    assert H.ranks_sum([o.data_ptr() for o in out], [t.data_ptr() for r in dev for t in r], counts, world, code, wcode,
+                       code, pre, post, gpu.stream)
+    gpu.stream.synchronize()
+    for i, c in enumerate(counts):
+        want = _expected(orc, [host[r][i] for r in range(world)], dtype, wire, pre, post)
+        got = out[i].cpu().numpy()
+        assert np.array_equal(got[:c].view(np.uint8), want.view(np.uint8)), (i, c)
+        assert got[c] == 0, "wrote behind its tensor"
+
+
 def test_ranks_sum_into_and_out_of_a_buffer(gpu, orc):
     """FLOAT32 tensors into a FLOAT16 fusion buffer, pad bytes zeroed, and out again."""
     rng = np.random.default_rng(3)

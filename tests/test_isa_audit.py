@@ -182,3 +182,23 @@ def test_split_sums_ask_for_all_their_streams_before_they_wait(kernels):
                 break
         checked += 1
     assert checked >= 98, checked
+
+
+def test_sums_of_many_ranks_load_eight_at_a_time(kernels):
+    """Beyond eight ranks ranks_sum_k goes on in batches: eight loads stand in a row once before the loop over the
+    ranks and once in it, for vectors and (second pair) for the elements behind the last vector."""
+    checked = 0
+    for name, lines in kernels.items():
+        m = re.search(r"ranks_sum_kI\w+?Li8ELi[01]EEE", name)
+        if not m:
+            continue
+        runs, run = [], 0
+        for ins in lines:
+            if re.match(r"(global|buffer)_load_", ins):
+                run += 1
+            elif "vmcnt(0)" in ins or ins.startswith(("s_cbranch", "s_branch")):
+                runs.append(run)
+                run = 0
+        assert runs.count(8) >= 3, (name, runs)
+        checked += 1
+    assert checked == 22, checked
