@@ -18,7 +18,7 @@
 // (17 vectors), but a level's norm as a difference of the ranks' products has no digits left where ranks nearly cancel.
 //
 // All roundings are those of the separate steps: to the wire type after the prescale, after every level's scaled add
-// and in the output.  The sums are taken in double in an order that depends on the sizes alone.
+// and in the output.  The sums are taken in double in an order that depends on the tensor's size alone.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -107,8 +107,40 @@ struct Sums {
   }
 };
 
+// A lane's part of a row's `chunks` triples: every LANES-th from `lane` on, of which there is at least one.
+template <uint32_t LANES>
+__device__ __forceinline__ Triple lane_sum(const double* s, uint32_t chunks, uint32_t lane) {
+  Triple t = {0., 0., 0.};
+  for (uint32_t i = lane; i < chunks; i += LANES * kSumsPerLane) {
+    Triple r[kSumsPerLane];
+#pragma unroll
+    for (uint32_t u = 0; u < kSumsPerLane; ++u) {  // unconditional, so that all are in flight together
+      const uint64_t at = 3 * (uint64_t)(i + LANES * u < chunks ? i + LANES * u : lane);
+      r[u] = Triple{s[at], s[at + 1], s[at + 2]};
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kSumsPerLane; ++u) {
+      const bool in = i + LANES * u < chunks;
+      t.d += in ? r[u].d : 0.;
+      t.a += in ? r[u].a : 0.;
+      t.b += in ? r[u].b : 0.;
+    }
+  }
+  return t;
+}
+
+// The sum of at most kReaddMax triples by one wavefront, in lane 63.  Whether a row's consumers add it or coeffs_k does
+// on account of a longer row beside it, the order is this one: a tensor's result does not depend on its company.
+__device__ __forceinline__ Triple short_row_sum(const double* s, uint32_t chunks, uint32_t lane) {
+  Triple t = lane_sum<64>(s, chunks, lane);
+  t.d = wave_sum(t.d);
+  t.a = wave_sum(t.a);
+  t.b = wave_sum(t.b);
+  return t;
+}
+
 // The coefficients of NP consecutive pairs of a row.  Without a table of them, wavefront w adds pair w's partial
-// sums, in an order that depends on their number alone: all workgroups of the row agree to the bit.
+// sums.
 template <int NP>
 __device__ __forceinline__ void row_coeffs(const Level& l, const Place& p, uint32_t first_chunk, uint32_t chunks,
                                            uint32_t pair, double (&c)[2 * NP]) {
@@ -125,25 +157,7 @@ __device__ __forceinline__ void row_coeffs(const Level& l, const Place& p, uint3
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (wave < NP) {
     const double* s = l.in_sums + 3 * ((uint64_t)(pair + wave) * l.chunks + first_chunk);
-    Triple t = {0., 0., 0.};
-    for (uint32_t i = lane; i < chunks; i += 64 * kSumsPerLane) {
-      Triple r[kSumsPerLane];
-#pragma unroll
-      for (uint32_t u = 0; u < kSumsPerLane; ++u) {  // unconditional, so that all are in flight together
-        const uint32_t at = 3 * (i + 64 * u < chunks ? i + 64 * u : lane);
-        r[u] = Triple{s[at], s[at + 1], s[at + 2]};
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < kSumsPerLane; ++u) {
-        const bool in = i + 64 * u < chunks;
-        t.d += in ? r[u].d : 0.;
-        t.a += in ? r[u].a : 0.;
-        t.b += in ? r[u].b : 0.;
-      }
-    }
-    t.d = wave_sum(t.d);
-    t.a = wave_sum(t.a);
-    t.b = wave_sum(t.b);
+    const Triple t = short_row_sum(s, chunks, lane);
     if (lane == 63) layer_coeffs(t, l.guard, &shared[2 * wave], &shared[2 * wave + 1]);
   }
   __syncthreads();
@@ -289,26 +303,14 @@ __global__ __launch_bounds__(kWG) void coeffs_k(const double* __restrict__ sums,
   const uint32_t row = blockIdx.x, pair = blockIdx.y;
   const uint32_t first = rows.first[row], count = rows.first[row + 1] - first;
   const double* s = sums + 3 * ((uint64_t)pair * chunks + first);
-  Triple t = {0., 0., 0.};
-  for (uint32_t i = threadIdx.x; i < count; i += kWG * kSumsPerLane) {
-    Triple r[kSumsPerLane];
-#pragma unroll
-    for (uint32_t u = 0; u < kSumsPerLane; ++u) {
-      const uint64_t at = 3 * (uint64_t)(i + kWG * u < count ? i + kWG * u : threadIdx.x);
-      r[u] = Triple{s[at], s[at + 1], s[at + 2]};
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < kSumsPerLane; ++u) {
-      const bool in = i + kWG * u < count;
-      t.d += in ? r[u].d : 0.;
-      t.a += in ? r[u].a : 0.;
-      t.b += in ? r[u].b : 0.;
-    }
-  }
-  const Triple r = wg_reduce(t);
-  if (threadIdx.x == 0) {
-    double* c = coeffs + 2 * ((uint64_t)pair * kMaxRows + row);
-    layer_coeffs(r, guard, &c[0], &c[1]);
+  double* c = coeffs + 2 * ((uint64_t)pair * kMaxRows + row);
+  if (count <= kReaddMax) {
+    if (threadIdx.x >= 64) return;
+    const Triple r = short_row_sum(s, count, threadIdx.x);
+    if (threadIdx.x == 63) layer_coeffs(r, guard, &c[0], &c[1]);
+  } else {
+    const Triple r = wg_reduce(lane_sum<kWG>(s, count, threadIdx.x));
+    if (threadIdx.x == 0) layer_coeffs(r, guard, &c[0], &c[1]);
   }
 }
 

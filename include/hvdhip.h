@@ -407,7 +407,7 @@ int hvdhip_adasum_dispatch_scaled_add(int dtype, int count, double acoeff, void*
  * device reads, every tensor a layer of its own: what packing every rank's tensors, combining the
  * buffers pairwise at distances 1, 2, 4 ... (Adasum::FusedAllreduce, ops/adasum/adasum.h:194-340) and
  * unpacking the first give, with the same roundings; the order of the double sums is fixed by the
- * sizes.  inputs, outputs, num_elements, the dtypes and factors, overlaps and event are those of
+ * tensor's own size.  inputs, outputs, num_elements, the dtypes and factors, overlaps and event are those of
  * hvdhip_ranks_sum(); wire_dtype is FLOAT16, FLOAT32 or FLOAT64.
  * workspace: device memory on a 256-byte boundary of at least
  * hvdhip_adasum_ranks_workspace() bytes (a negative return is an error code), the caller's again once the

@@ -65,6 +65,37 @@ def test_adasum_ranks_equals_the_pairwise_tree(gpu, orc, dtype, wire, world, sha
             assert np.count_nonzero(diff) <= 2 + 1e-5 * c, (i, c, np.count_nonzero(diff))
 
 
+@pytest.mark.parametrize("world", [2, 8, 16])
+def test_adasum_ranks_does_not_depend_on_the_other_tensors(gpu, world):
+    """A tensor of up to 512 chunks gives the same bits by itself and beside one of more, where the coefficients of
+    all come from a launch of their own.  In float64, with ranks that have much in common, a coefficient's last bit
+    shows in most elements, and sums in another order move it in some pair of some tensor."""
+    gen = torch.Generator(device="cuda").manual_seed(world)
+    chunk, code = 16384 // 8, DTYPE["float64"]
+    counts = [130 * chunk + 5 * i for i in range(6)] + [300 * chunk + 17, 512 * chunk, 513 * chunk]
+
+    def normal(c):
+        return torch.empty(c, dtype=torch.float64, device="cuda").normal_(0.0, 0.01, generator=gen)
+
+    common = [normal(c) for c in counts]
+    dev = [[t + normal(t.numel()) for t in common] for _ in range(world)]
+
+    def combine(which):
+        sizes = [counts[i] for i in which]
+        out = [torch.zeros(c, dtype=torch.float64, device="cuda") for c in sizes]
+        need = H.adasum_ranks_workspace(sizes, world, code)
+        work = torch.empty(need, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        assert H.adasum_ranks([o.data_ptr() for o in out], [r[i].data_ptr() for r in dev for i in which], sizes, world,
+                              code, code, code, 1.0, 1.0, work.data_ptr(), need, gpu.stream)
+        gpu.stream.synchronize()
+        return out
+
+    together = combine(range(len(counts)))
+    for i in range(len(counts)):
+        assert torch.equal(combine([i])[0].view(torch.int64), together[i].view(torch.int64)), counts[i]
+
+
 def test_adasum_ranks_refuses(gpu):
     t = torch.zeros(8192, dtype=torch.float32, device="cuda")
     work = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
