@@ -42,9 +42,11 @@ struct Factor<half_t> {
   typedef float type;
 };
 
-// ScaleBufferCPUImpl's element (ops/collective_operations.h:91-127), as in xfer.hip.
+// ScaleBufferCPUImpl's element (ops/collective_operations.h:91-127), as in xfer.hip.  Device code contracts by default,
+// and what follows here is a sum: the product has to be rounded by itself first.
 template <typename T>
 __device__ __forceinline__ T scaled(T x, typename Factor<T>::type s) {
+#pragma clang fp contract(off)
   return (T)(s * x);
 }
 template <>
