@@ -36,7 +36,14 @@ constexpr int kSplitVecs = K == 2 * kSplitWaves<K> ? 1 : 2;
 template <typename T, int VEC>
 __device__ __forceinline__ void add_to(Arr<T, VEC>& acc, const Arr<T, VEC>& x) {
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) acc.v[j] = (T)(acc.v[j] + x.v[j]);
+  for (int j = 0; j < VEC; ++j) {
+    if constexpr (std::is_integral<T>::value) {  // wraps, which signed addition is not defined to do
+      typedef typename std::make_unsigned<T>::type U;
+      acc.v[j] = (T)((U)acc.v[j] + (U)x.v[j]);
+    } else {
+      acc.v[j] = (T)(acc.v[j] + x.v[j]);
+    }
+  }
 }
 // Halves as packed adds (one rounding, which equals fp32 add and narrowing: see reduce.hip).
 template <>

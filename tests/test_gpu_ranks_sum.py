@@ -110,6 +110,25 @@ def test_ranks_sum_in_batches_of_eight_four_two_and_one(gpu, orc, dtype, wire, w
         assert got[c] == 0, "wrote behind its tensor"
 
 
+@pytest.mark.parametrize("dtype", ["uint8", "int8", "int16", "int32", "int64"])
+@pytest.mark.parametrize("world", [2, 5, 8, 11])
+def test_integer_sums_wrap(gpu, dtype, world):
+    rng = np.random.default_rng(world)
+    info, n = np.iinfo(NP[dtype]), 5003
+    host = [rng.integers(info.min, info.max, n, dtype=NP[dtype], endpoint=True) for _ in range(world)]
+    host[0][:9], host[1][:9] = info.max, info.max
+    dev = [torch.from_numpy(v).cuda() for v in host]
+    out = torch.zeros_like(dev[0])
+    torch.cuda.synchronize()
+    code = DTYPE[dtype]
+    assert H.ranks_sum([out.data_ptr()], [t.data_ptr() for t in dev], [n], world, code, code, code, 1.0, 1.0, gpu.stream)
+    gpu.stream.synchronize()
+    want = host[0].copy()
+    for v in host[1:]:
+        want += v  # numpy's arrays wrap
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
 def test_ranks_sum_into_and_out_of_a_buffer(gpu, orc):
     """FLOAT32 tensors into a FLOAT16 fusion buffer, pad bytes zeroed, and out again."""
     rng = np.random.default_rng(3)

@@ -5,6 +5,7 @@ import os
 import re
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -21,6 +22,14 @@ __global__ void scaled_sum_k(T* out, const T* a, const T* b, double pre) {
   add_to<T, 1>(acc, to_wire<T, T, 1>(Arr<T, 1>{b[threadIdx.x]}, f, true));
   out[threadIdx.x] = acc.v[0];
 }
+template <typename T>
+__global__ void sum_k(T* out, const T* a, const T* b) {
+  Arr<T, 1> acc = {a[threadIdx.x]};
+  add_to<T, 1>(acc, Arr<T, 1>{b[threadIdx.x]});
+  out[threadIdx.x] = acc.v[0];
+}
+template __global__ void sum_k<int32_t>(int32_t*, const int32_t*, const int32_t*);
+template __global__ void sum_k<int64_t>(int64_t*, const int64_t*, const int64_t*);
 template __global__ void scaled_sum_k<float>(float*, const float*, const float*, double);
 template __global__ void scaled_sum_k<double>(double*, const double*, const double*, double);
 """
@@ -28,23 +37,31 @@ template __global__ void scaled_sum_k<double>(double*, const double*, const doub
 
 @pytest.fixture(scope="module")
 def probe(tmp_path_factory):
-    """probe(kernel name): its assembly."""
+    """probe(kernel name, "asm" or "ir"): its assembly or the compiler's intermediate code."""
     if shutil.which("hipcc") is None:
         pytest.skip("hipcc is not installed")
     tmp = tmp_path_factory.mktemp("arithmetic")
-    src, out = str(tmp / "probe.hip"), str(tmp / "probe.s")
+    src = str(tmp / "probe.hip")
     with open(src, "w") as f:
         f.write(PROBE)
     cmd = ["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
            "-packed-fp32-ops", "-Wno-unused-function", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-S",
-           "--cuda-device-only", "-o", out, src]
-    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=600)
-    assert r.returncode == 0, r.stdout.decode(errors="replace")[-2000:]
-    text = open(out).read()
+           "--cuda-device-only", src]
 
-    def body(name):
-        start = re.search(r"^_Z\d+" + name + r"\w*:", text, re.M).end()
-        return text[start:text.index("s_endpgm", start)]
+    def compiled(kind):
+        out = str(tmp / kind)
+        r = subprocess.run(cmd + ["-o", out] + (["-emit-llvm"] if kind == "ir" else []), stdout=subprocess.PIPE,
+                           stderr=subprocess.STDOUT, timeout=600)
+        assert r.returncode == 0, r.stdout.decode(errors="replace")[-2000:]
+        return open(out).read()
+
+    with ThreadPoolExecutor(2) as pool:
+        texts = dict(zip(("asm", "ir"), pool.map(compiled, ("asm", "ir"))))
+
+    def body(name, kind):
+        text = texts[kind]
+        start = re.search(r"^(define .*@)?_Z\d+" + name + r"\w*[:(]", text, re.M).end()
+        return text[start:text.index("s_endpgm" if kind == "asm" else "\n}", start)]
 
     return body
 
@@ -53,6 +70,13 @@ def probe(tmp_path_factory):
 def test_a_scaled_element_is_rounded_before_it_is_added(probe, bits):
     """Packing stores the product in the wire type; summing reads it from there.  A fused multiply-add would round
     once where that rounds twice."""
-    body = probe("scaled_sum_kI" + ("f" if bits == 32 else "d"))
+    body = probe("scaled_sum_kI" + ("f" if bits == 32 else "d"), "asm")
     assert "v_mul_f%d" % bits in body and "v_add_f%d" % bits in body, body
     assert not re.search(r"v_(fma|fmac|mad|mac)\w*_f%d" % bits, body), body
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_integer_sums_wrap(probe, bits):
+    """Overflow is defined, as in reduce.hip: the compiler has no leave to assume that there is none (nsw)."""
+    body = probe("sum_kI" + ("i" if bits == 32 else "l"), "ir")
+    assert re.search(r"= add i%d " % bits, body) and not re.search(r"= add \w*nsw i%d " % bits, body), body
