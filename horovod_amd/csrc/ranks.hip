@@ -17,6 +17,7 @@
 // step spent 16 ms on rebuilding them whenever more sets rotated than it held.
 #include <algorithm>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "ranks.h"
@@ -391,8 +392,12 @@ int hvdhip::check_ranks_call(RanksCall* c, int in_dtype, int wire_dtype, int out
         return fail(HVDHIP_ERR_INVALID_ARGUMENT, "rank %d of entry %d is NULL or not aligned to its element size", r, i);
     }
   }
-  if (overlaps(*c, (uint64_t)is, (uint64_t)os))
-    return fail(HVDHIP_ERR_OVERLAP, "an output overlaps another output or another entry's input");
+  try {
+    if (overlaps(*c, (uint64_t)is, (uint64_t)os))
+      return fail(HVDHIP_ERR_OVERLAP, "an output overlaps another output or another entry's input");
+  } catch (const std::bad_alloc&) {  // must not leave through a C interface
+    return fail(HVDHIP_ERR_OUT_OF_MEMORY, "no host memory to compare %d outputs", c->n);
+  }
   if (c->pre != 1.0) c->flags |= kScaleIn;
   if (c->post != 1.0) c->flags |= kScaleOut;
   if (wire_dtype == HVDHIP_FLOAT16) {
