@@ -241,7 +241,7 @@ class Engine:
             else:
                 self._sum(slot, s, first, inputs, outputs, counts, event)
         except Exception:
-            check(lib().hvdhip_event_release(s.handle, event), "hvdhip_event_release")
+            self._give_up(s, event)
             raise
         self._finish(s, requests, event, peers)
 
@@ -251,6 +251,15 @@ class Engine:
         ev = c_void_p()
         check(lib().hvdhip_event_acquire(s.handle, ctypes.byref(ev)), "hvdhip_event_acquire")
         return ev
+
+    @staticmethod
+    def _give_up(s, event):
+        """For a response that failed after part of it was queued: that part may still read the ranks' tensors and
+        write the outputs, which nothing holds on to once the caller has the error."""
+        try:
+            s.synchronize()
+        finally:
+            check(lib().hvdhip_event_release(s.handle, event), "hvdhip_event_release")
 
     def _sum(self, slot, s, req, inputs, outputs, counts, event):
         """outputs = postscale * (sum over ranks of prescale * inputs), in one pass if the outputs lie over no
@@ -355,7 +364,7 @@ class Engine:
             # synchronization that follows, as scripts that read the rows on the host do
             check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
         except Exception:
-            check(lib().hvdhip_event_release(s.handle, event), "hvdhip_event_release")
+            self._give_up(s, event)
             raise
         self._finish(s, requests, event)
 

@@ -187,3 +187,35 @@ def test_engine_sums_through_a_buffer_where_one_pass_cannot(monkeypatch, case):
             assert torch.equal(x.cpu(), size * xs) and torch.equal(y.cpu(), size * ys)
     finally:
         hvd.shutdown()
+
+
+def test_a_response_that_fails_halfway_waits_for_what_it_queued(monkeypatch):
+    """Adasum over two nodes of four ranks, and no buffer for the second node's sum: the first one's is under way
+    and reads tensors that the caller is free to drop once it has the error."""
+    import horovod_amd.torch as hvd
+    from horovod_amd.torch import mpi_ops
+    hvd.shutdown()
+    hvd.init(size=8, local_size=4)
+    engine = mpi_ops._engine
+    buffer = engine._buffer
+
+    def no_second_node(slot, what, nbytes):
+        if what == 3:
+            raise MemoryError("no second buffer")
+        return buffer(slot, what, nbytes)
+
+    try:
+        t = torch.zeros(1 << 29, dtype=torch.float32, device="cuda")
+        stream = torch.cuda.ExternalStream(engine.streams[0].handle.value)
+        engine._buffer(0, 2, t.numel() * 4)
+        torch.cuda.synchronize()
+        monkeypatch.setattr(engine, "_buffer", no_second_node)
+        handle = hvd.allreduce_async(t, op=hvd.Adasum)
+        engine.run_cycle()
+        assert stream.query()  # 2 GiB: more than a millisecond of work
+        with pytest.raises(hvd.HorovodInternalError, match="no second buffer"):
+            hvd.synchronize(handle)
+        monkeypatch.undo()
+        assert torch.equal(hvd.allreduce(t[:1000], op=hvd.Adasum), t[:1000])
+    finally:
+        hvd.shutdown()
