@@ -234,7 +234,11 @@ class Engine:
         outputs = [e.output.data_ptr() for _, e in group]
         event = self._acquire(s)
         try:
-            if not any(counts):
+            plain = first.wire_dtype == first.tensor_dtype
+            stays = self.size == 1 and inputs == outputs and plain and first.prescale == first.postscale == 1.0
+            if len(group) == 1 and plain and not stays:
+                inputs = self._aligned(slot, s, inputs, counts[0], first.tensor_dtype)
+            if stays or not any(counts):
                 check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
             elif first.op == ADASUM and self.size > 1:
                 self._adasum(slot, s, first, inputs, outputs, counts, event)
@@ -244,6 +248,19 @@ class Engine:
             self._give_up(s, event)
             raise
         self._finish(s, requests, event, peers)
+
+    def _aligned(self, slot, s, inputs, count, dtype):
+        """Foreign memory may lie on addresses that no element type fits.  Alone in its response such a tensor is
+        copied as bytes first; fused ones are refused, as they are by a fusion plan."""
+        es = dtype_size(dtype)
+        if count == 0 or not any(p % es for p in inputs):
+            return inputs
+        sources, stride = list(dict.fromkeys(inputs)), (count * es + 255) // 256 * 256
+        buf = self._buffer(slot, "aligned", len(sources) * stride)
+        at = {p: buf + i * stride for i, p in enumerate(sources)}
+        as_bytes = TORCH_TO_HVD[torch.uint8]
+        H.ranks_sum(list(at.values()), sources, [count * es] * len(sources), 1, as_bytes, as_bytes, as_bytes, 1.0, 1.0, s)
+        return [at[p] for p in inputs]
 
     @staticmethod
     def _acquire(s):
@@ -356,6 +373,8 @@ class Engine:
                     places.append(at)
                     counts.append(n)
                     at += n * es
+        if any(p % es for p in sources):  # foreign memory that no element type fits: bytes
+            counts, dtype = [n * es for n in counts], TORCH_TO_HVD[torch.uint8]
         event = self._acquire(s)
         try:
             if not H.ranks_sum(places, sources, counts, 1, dtype, dtype, dtype, 1.0, 1.0, s):

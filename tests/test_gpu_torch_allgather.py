@@ -150,3 +150,30 @@ def test_allgather_errors(hvd):
     with pytest.raises(hvd.HorovodInternalError, match="same name"):
         hvd.allgather_async(t, name="dup")  # test_torch.py:936-955
     assert hvd.synchronize(h).shape == (8,)
+
+
+@pytest.mark.parametrize("size", [1, 3])
+def test_memory_on_odd_addresses(hvd, size):
+    """Tensors over foreign memory whose address is no multiple of their element size: gathered, and summed where they
+    are alone in their response."""
+    rng = np.random.default_rng(size)
+    want = rng.standard_normal(1003).astype(np.float32)
+    raw = torch.from_numpy(np.concatenate([np.zeros(2, np.uint8), want.view(np.uint8)])).cuda()
+
+    class Foreign:
+        __cuda_array_interface__ = {"shape": want.shape, "typestr": "<f4", "data": (raw.data_ptr() + 2, False),
+                                    "version": 2, "strides": None}
+
+    t = torch.as_tensor(Foreign(), device="cuda")
+    assert t.data_ptr() % 4 == 2 and t.is_contiguous()
+    hvd.init(size=size)
+    assert np.array_equal(hvd.allgather(t).cpu().numpy(), np.tile(want, size))
+    total = want
+    for _ in range(size - 1):
+        total = total + want
+    assert np.array_equal(hvd.allreduce(t, op=hvd.Sum).cpu().numpy(), total)
+    if size == 1:
+        assert np.array_equal(hvd.allreduce_(t, op=hvd.Sum).cpu().numpy(), want)
+    else:
+        with pytest.raises(hvd.HorovodInternalError, match="aligned"):
+            hvd.grouped_allreduce([t, t], op=hvd.Sum)
