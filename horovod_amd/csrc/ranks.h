@@ -43,10 +43,13 @@ struct Factor<half_t> {
 };
 
 // ScaleBufferCPUImpl's element (ops/collective_operations.h:91-127), as in xfer.hip.  Device code contracts by default,
-// and what follows here is a sum: the product has to be rounded by itself first.
+// and what follows here is a sum: the product has to be rounded by itself first.  A byte's product goes through 32 bits:
+// straight to a byte it is undefined outside of the byte's range, and the compiler leaves what lies above eight bits in
+// the register.
 template <typename T>
 __device__ __forceinline__ T scaled(T x, typename Factor<T>::type s) {
 #pragma clang fp contract(off)
+  if constexpr (sizeof(T) == 1) return (T)(int32_t)(s * x);
   return (T)(s * x);
 }
 template <>

@@ -129,6 +129,23 @@ def test_integer_sums_wrap(gpu, dtype, world):
     assert np.array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("dtype", ["uint8", "int8"])
+@pytest.mark.parametrize("world", [1, 2, 4, 9])
+@pytest.mark.parametrize("pre,post", [(3.0, 1.0), (7.3, 0.5), (-1.0, 1.0), (1.0, 3.7), (5.0, 5.0)])
+def test_scaled_bytes_beyond_their_range_wrap_like_the_oracle(gpu, orc, dtype, world, pre, post):
+    """Every byte value, scaled to several times its range, and no trace of it in the bytes beside."""
+    rng = np.random.default_rng(world)
+    n = 5 * 256 + 3
+    host = [rng.permutation(np.arange(n) % 256).astype(np.uint8).view(NP[dtype]) for _ in range(world)]
+    dev = [torch.from_numpy(v).cuda() for v in host]
+    out = torch.zeros_like(dev[0])
+    torch.cuda.synchronize()
+    code = DTYPE[dtype]
+    assert H.ranks_sum([out.data_ptr()], [t.data_ptr() for t in dev], [n], world, code, code, code, pre, post, gpu.stream)
+    gpu.stream.synchronize()
+    assert np.array_equal(out.cpu().numpy(), _expected(orc, host, dtype, dtype, pre, post))
+
+
 def test_ranks_sum_into_and_out_of_a_buffer(gpu, orc):
     """FLOAT32 tensors into a FLOAT16 fusion buffer, pad bytes zeroed, and out again."""
     rng = np.random.default_rng(3)
