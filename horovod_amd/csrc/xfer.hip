@@ -61,7 +61,9 @@ struct Copy {
 };
 
 // out = (T)(factor * in): factor type TS is double for u8/i8/i32/i64/f64 and
-// float for f32 (ops/collective_operations.cc:119-140).
+// float for f32 (ops/collective_operations.cc:119-140).  A byte's product goes through 32
+// bits: straight to a byte it is undefined outside of the byte's range, and what the
+// compiler then left above eight bits ended up in the byte beside.
 template <typename T, typename TS>
 struct Scale {
   typedef T S;
@@ -70,8 +72,48 @@ struct Scale {
   struct P {
     TS s;
   };
-  static __device__ __forceinline__ D f(S x, P p) { return (T)(p.s * x); }
+  static __device__ __forceinline__ D f(S x, P p) {
+    if constexpr (sizeof(T) == 1) {
+      return (T)(int32_t)(p.s * x);
+    } else {
+      return (T)(p.s * x);
+    }
+  }
 };
+
+// What a lane does with its VEC elements.
+template <class Op>
+__device__ __forceinline__ Arr<typename Op::D, Op::VEC> apply(const Arr<typename Op::S, Op::VEC>& x, typename Op::P p) {
+  Arr<typename Op::D, Op::VEC> y;
+#pragma unroll
+  for (int j = 0; j < Op::VEC; ++j) y.v[j] = Op::f(x.v[j], p);
+  return y;
+}
+// Sixteen scaled bytes: the low bytes of four products are gathered by three permutes, without the masks and shifts that
+// the compiler makes of them (100 million uint8: 33.9 us with those, 32.5 so).
+template <typename T>
+__device__ __forceinline__ Arr<T, 16> apply_scale_bytes(const Arr<T, 16>& x, double s) {
+  uint32_t words[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t c[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = (uint32_t)(int32_t)(s * x.v[4 * w + j]);
+    const uint32_t lo = __builtin_amdgcn_perm(c[1], c[0], 0x0c0c0400), hi = __builtin_amdgcn_perm(c[3], c[2], 0x0c0c0400);
+    words[w] = __builtin_amdgcn_perm(hi, lo, 0x05040100);
+  }
+  return __builtin_bit_cast(Arr<T, 16>, words);
+}
+template <>
+__device__ __forceinline__ Arr<uint8_t, 16> apply<Scale<uint8_t, double>>(const Arr<uint8_t, 16>& x,
+                                                                         Scale<uint8_t, double>::P p) {
+  return apply_scale_bytes(x, p.s);
+}
+template <>
+__device__ __forceinline__ Arr<int8_t, 16> apply<Scale<int8_t, double>>(const Arr<int8_t, 16>& x,
+                                                                       Scale<int8_t, double>::P p) {
+  return apply_scale_bytes(x, p.s);
+}
 
 // fp16 scaled through fp32 with an fp32 factor, one rounding to nearest even
 // (ops/collective_operations.h:99-127).  When the host hands over a factor that a
@@ -163,20 +205,10 @@ __device__ __forceinline__ void stream_range(gptr<const typename Op::S> src,
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) x[u] = load(v + u * kWG);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      Arr<D, VEC> y;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) y.v[j] = Op::f(x[u].v[j], p);
-      stw<ST, D, VEC>(out, (v + u * kWG) * (uint32_t)(VEC * sizeof(D)), y);
-    }
+    for (int u = 0; u < kUnroll; ++u)
+      stw<ST, D, VEC>(out, (v + u * kWG) * (uint32_t)(VEC * sizeof(D)), apply<Op>(x[u], p));
   }
-  for (; v < nv; v += kWG) {
-    const Arr<S, VEC> x = load(v);
-    Arr<D, VEC> y;
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) y.v[j] = Op::f(x.v[j], p);
-    stw<ST, D, VEC>(out, v * (uint32_t)(VEC * sizeof(D)), y);
-  }
+  for (; v < nv; v += kWG) stw<ST, D, VEC>(out, v * (uint32_t)(VEC * sizeof(D)), apply<Op>(load(v), p));
   const uint32_t t = nv * VEC + threadIdx.x;  // fewer than VEC elements remain
   if (t < n) dst[t] = Op::f(src[t], p);
 }

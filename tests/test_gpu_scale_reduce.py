@@ -151,6 +151,31 @@ def test_tile_order_across_xcd_groups(gpu, orc, dtype, n_tiles):
     assert np.array_equal(gpu.download(d_v)[:n * es], orc.sum(_raw(p), _raw(v), dtype).view(np.uint8))
 
 
+@pytest.mark.parametrize("dtype", [U8, I8])
+@pytest.mark.parametrize("factor", [2.0, 3.7, -1.0, 1000.0])
+def test_scaled_bytes_beyond_their_range_leave_the_ones_beside_alone(gpu, orc, dtype, factor):
+    """A byte whose product leaves its range wraps as on the CPU, through the whole-buffer scale, the pack and the
+    unpack; no bit of it reaches another byte."""
+    rng = np.random.default_rng(7)
+    n = 5 * 256 + 3
+    v = rng.permutation(np.arange(n) % 256).astype(np.uint8).view(NP_OF[dtype])
+    want = orc.scale_buffer(v, factor, dtype)
+    src = gpu.upload(v)
+    out = gpu.empty(n)
+    gpu.H.scale_buffer(src.data_ptr(), out.data_ptr(), n, factor, dtype, gpu.stream)
+    assert np.array_equal(gpu.download(out), want.view(np.uint8))
+    back = gpu.empty(n)
+    plan = gpu.H.FusionPlan([src.data_ptr()], [back.data_ptr()], [n], dtype)
+    try:
+        buf = gpu.empty(plan.buffer_len)
+        plan.pack(buf.data_ptr(), factor, gpu.stream)
+        assert np.array_equal(gpu.download(buf)[:n], want.view(np.uint8))
+        plan.unpack(buf.data_ptr(), factor, gpu.stream)
+        assert np.array_equal(gpu.download(back), orc.scale_buffer(want, factor, dtype).view(np.uint8))
+    finally:
+        plan.destroy()
+
+
 @pytest.mark.parametrize("dtype", [U8, F16, F32, F64])
 @pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8])
 def test_reduce_sum_k_of_streams_split_over_wavefronts(gpu, orc, dtype, k):
