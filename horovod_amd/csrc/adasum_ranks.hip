@@ -174,7 +174,7 @@ __device__ __forceinline__ Arr<W, N> combined(double ca, const Arr<W, N>& a, dou
 }
 
 // Row: {elements, anything, rank 0, 1 ...}.  KEEP: whose tensors the loads leave in the Infinity Cache for the
-// pass that reads them again (0 nobody's, 1 every pair's first rank's, 2 all).
+// pass that reads them again (1 every pair's first rank's, 2 all).
 template <typename S, typename W, int KEEP>
 __global__ __launch_bounds__(kWG) void dots_k(Level l, Rows rows) {
   constexpr int VEC = kVec<S, W>;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kWG) void dots_k(Level l, Rows rows) {
     Arr<S, VEC> x[U], y[U];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-      x[i] = ldv<S, VEC, KEEP == 0>(a + (size_t)(v + i * kWG) * VEC);
+      x[i] = ldv<S, VEC, false>(a + (size_t)(v + i * kWG) * VEC);
       y[i] = ldv<S, VEC, KEEP != 2>(b + (size_t)(v + i * kWG) * VEC);
     }
 #pragma unroll

@@ -1,6 +1,8 @@
 """hvdhip_adasum_ranks against the oracle's pairwise combine, level by level, at the edges of its chunks (16 KiB of
-the wire type), of the partial sums that a consumer adds itself (512 per tensor), of the tensors one launch carries
-(44 of eight ranks) and of the ranks one launch reads (8)."""
+the wire type), of the partial sums that a consumer adds itself (512 per tensor; "long" at 8 and 16 ranks has every
+level read the coefficients of the launch in between), of the tensors one launch carries (44 of eight ranks), of the
+ranks one launch reads (8) and of what the first pass leaves in the Infinity Cache (all ranks up to 160 MiB in
+total, of 16 "long" ones every other)."""
 import numpy as np
 import pytest
 import torch
@@ -23,8 +25,8 @@ def _tree(orc, ranks, wire, pre, post):
 
 
 @pytest.mark.parametrize("dtype,wire", [(d, d) for d in NP] + [("float32", "float16")])
-@pytest.mark.parametrize("world,shape", [(2, "edges"), (4, "edges"), (8, "edges"), (32, "edges"), (4, "long"),
-                                         (8, "rows")])
+@pytest.mark.parametrize("world,shape", [(2, "edges"), (4, "edges"), (8, "edges"), (32, "edges"), (64, "edges"),
+                                         (128, "edges"), (4, "long"), (8, "long"), (16, "long"), (8, "rows")])
 def test_adasum_ranks_equals_the_pairwise_tree(gpu, orc, dtype, wire, world, shape):
     rng = np.random.default_rng(world)
     chunk = 16384 // np.dtype(NP[wire]).itemsize

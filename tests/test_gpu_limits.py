@@ -86,6 +86,54 @@ def test_contiguous_kernels_slice_beyond_one_launch(gpu):
     assert e.value.code == -4
 
 
+def _pattern(n):
+    """Bytes that differ from their neighbours and from those a launch further on."""
+    x = torch.arange(n, dtype=torch.int32, device="cuda") if n < (1 << 31) else None
+    if x is not None:
+        return ((x * 7) ^ (x >> 11) ^ (x >> 21)).to(torch.uint8)
+    return torch.cat([_pattern((1 << 30)).add_(3 * i) for i in range(n >> 30)] + [_pattern(n & ((1 << 30) - 1))])
+
+
+@pytest.mark.parametrize("world,gib", [(1, 32), (3, 16), (4, 8), (9, 32)])
+def test_sum_over_ranks_cuts_a_tensor_beyond_one_launch(gpu, world, gib):
+    """2^23 workgroups of 4 KiB (1, 2 and more than 8 ranks), 2 KiB or 1 KiB (3 to 8) are one launch's share; what is
+    left of the tensor goes on in the next, ahead of the tensors behind it.  In place, all ranks alike."""
+    n = (gib << 30) + 777
+    x = _pattern(n)
+    small = _pattern(5003)
+    out = torch.zeros_like(small)
+    want_small = small * (world % 256) if world > 1 else small.clone()
+    ends = [(0, 1 << 20), ((gib << 30) - (1 << 20), n)] + [((gib << 29) + 4096 * i, (gib << 29) + 4096 * i + 2048) for i in range(3)]
+    keep = [x[a:b].clone() for a, b in ends]
+    total = x[:n // 8 * 8].view(torch.int64)[::4097].clone()
+    y = x if world > 1 else torch.zeros_like(x)
+    torch.cuda.synchronize()
+    assert gpu.H.ranks_sum([y.data_ptr(), out.data_ptr()], [x.data_ptr(), small.data_ptr()] * world, [n, 5003], world, U8, U8,
+                           U8, 1.0, 1.0, gpu.stream)
+    gpu.sync()
+    assert torch.equal(out, want_small)
+    for (a, b), k in zip(ends, keep):
+        assert torch.equal(y[a:b], k * world), (a, b)
+    got = y[:n // 8 * 8].view(torch.int64)[::4097].contiguous().view(torch.uint8)
+    assert torch.equal(got, total.view(torch.uint8) * world)
+
+
+@pytest.mark.parametrize("k,gib", [(7, 8), (8, 16), (9, 4), (15, 4)])
+def test_split_sums_slice_beyond_one_launch(gpu, k, gib):
+    """2^23 workgroups of 1 or 2 KiB of every stream for 3 to 8 peers, 2^22 of 1 KiB for 9 to 15."""
+    n = (gib << 30) + 777
+    x = _pattern(n)
+    y = _pattern(n).add_(11)
+    want_end, want_mid = x[-5000:] + y[-5000:] * k, x[(gib << 29):(gib << 29) + 9000] + y[(gib << 29):(gib << 29) + 9000] * k
+    want = x[:n // 8 * 8].view(torch.int64)[::4097].contiguous().view(torch.uint8) + \
+        y[:n // 8 * 8].view(torch.int64)[::4097].contiguous().view(torch.uint8) * k
+    torch.cuda.synchronize()
+    gpu.H.reduce_sum_k(x.data_ptr(), [y.data_ptr()] * k, n, U8, gpu.stream)
+    gpu.sync()
+    assert torch.equal(x[-5000:], want_end) and torch.equal(x[(gib << 29):(gib << 29) + 9000], want_mid)
+    assert torch.equal(x[:n // 8 * 8].view(torch.int64)[::4097].contiguous().view(torch.uint8), want)
+
+
 def test_pipeline_replays_from_a_hip_graph(gpu, orc):
     """pack -> reduce -> unpack captured once and replayed: the entry points only launch kernels
     (no allocation, no memset), so they can be captured; every replay must equal the eager result."""

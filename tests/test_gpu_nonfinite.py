@@ -182,3 +182,63 @@ def test_adasum_layers_with_nonfinite_values(gpu, orc, dtype):
         s, e = starts[layer], starts[layer + 1]
         alone, _, _ = orc.adasum_pairwise(_raw(a[s:e]), _raw(b[s:e]), [e - s], dtype)
         assert np.array_equal(want[s:e], alone)
+
+
+@pytest.mark.parametrize("dtype", [F16, F32, F64])
+@pytest.mark.parametrize("world", [2, 3, 5, 8, 9, 20])
+@pytest.mark.parametrize("pre,post", [(1.0, 1.0), (0.3, 1e6)])
+def test_sums_over_ranks_with_nonfinite_values(gpu, orc, dtype, world, pre, post):
+    n = 20011
+    ranks = [_specials(dtype, n, 30 + r) for r in range(world)]
+    ranks[1][:200] = -ranks[0][:200]  # infinities that cancel, zeros of both signs
+    scaled = [orc.scale_buffer(_raw(v), pre, dtype) if pre != 1.0 else _raw(v) for v in ranks]
+    want = scaled[0].copy()
+    for v in scaled[1:]:
+        want = orc.sum(v, want, dtype)
+    want = orc.scale_buffer(want, post, dtype) if post != 1.0 else want
+    dev = [gpu.upload(v) for v in ranks]
+    out = gpu.empty(n * SIZE_OF[dtype])
+    assert gpu.H.ranks_sum([out.data_ptr()], [d.data_ptr() for d in dev], [n], world, dtype, dtype, dtype, pre, post,
+                           gpu.stream)
+    got = gpu.download(out, RAW_OF[dtype])
+    _same_but_for_nan_bits(got, want.view(RAW_OF[dtype]), NP_OF[dtype], "sum of %d ranks" % world)
+
+
+@pytest.mark.parametrize("dtype", [F32, F64, F16])
+@pytest.mark.parametrize("world", [2, 4, 8])
+def test_adasum_over_ranks_with_nonfinite_values(gpu, orc, dtype, world):
+    """As above for the tree over ranks: a NaN or an infinity in one rank's tensor comes out as pairwise combines on the
+    CPU leave it, and the tensors beside it are what they are without it."""
+    np_t = NP_OF[dtype]
+    counts = [1000, 20000, 17, 9000, 40000, 300, 5000]
+    rng = np.random.default_rng(6)
+    ranks = [[rng.standard_normal(c).astype(np_t) for c in counts] for _ in range(world)]
+    ranks[0][1][7] = np.nan
+    ranks[1][2][3] = np.nan
+    ranks[0][3][5] = ranks[world - 1][3][6] = np.nan
+    ranks[0][4][11] = np.inf
+    ranks[world - 1][5][1] = -np.inf
+    dev = [[gpu.upload(v) for v in rank] for rank in ranks]
+    out = [gpu.empty(v.nbytes) for v in ranks[0]]
+    need = gpu.H.adasum_ranks_workspace(counts, world, dtype)
+    work = gpu.empty(need + 256)
+    base = (work.data_ptr() + 255) // 256 * 256
+    assert gpu.H.adasum_ranks([o.data_ptr() for o in out], [d.data_ptr() for r in dev for d in r], counts, world, dtype,
+                              dtype, dtype, 1.0, 1.0, base, need, gpu.stream)
+    for i, c in enumerate(counts):
+        level = [_raw(r[i]) for r in ranks]
+        while len(level) > 1:
+            level = [orc.adasum_pairwise(a, b, [c], dtype)[0] for a, b in zip(level[::2], level[1::2])]
+        want, got = level[0].view(np_t), gpu.download(out[i], RAW_OF[dtype]).view(np_t)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), "tensor %d: NaN in other places" % i
+        inf = np.isinf(want)
+        assert np.array_equal(got[inf], want[inf]) and np.array_equal(np.isinf(got), inf), i
+        fin = np.isfinite(want)
+        if i in (0, 6):
+            assert fin.all()
+        # sums in another order move a coefficient by c units of 2^-53 and a rounding by an ulp a level (fp16: of
+        # values up to 2^3)
+        size = sum(np.abs(r[i].astype(np.float64)) for r in ranks)[fin]
+        ulp = {F16: 2.0 ** -10, F32: 2.0 ** -23, F64: 2.0 ** -52}[dtype]
+        diff = np.abs(got[fin].astype(np.float64) - want[fin].astype(np.float64))
+        assert np.all(diff <= 3 * (ulp + (c + 64) * 2.0 ** -53) * 1.5 ** 3 * size + 2.0 ** -24), (i, diff.max())

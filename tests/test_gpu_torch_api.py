@@ -484,3 +484,13 @@ def test_broadcast_in_the_simulated_world(hvd):
         hvd.broadcast_(t, root_rank=4)
     with pytest.raises(NotImplementedError):
         hvd.broadcast_optimizer_state(opt, root_rank=1)
+
+
+def test_the_producing_stream_is_the_one_that_is_current(gpu):
+    """The engine asks torch for the current stream's identifiers without the Stream object that the public call makes of
+    them: the same, on the default stream and on others."""
+    from horovod_amd.torch import engine
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.ExternalStream(gpu.stream.handle.value)):
+        with torch.cuda.stream(stream):
+            now = torch.cuda.current_stream()
+            assert tuple(engine._current_stream()) == (now.stream_id, now.device_index, now.device_type)
