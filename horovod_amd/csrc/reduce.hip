@@ -278,10 +278,11 @@ int launch_many(void* resident, const void* const* incoming, int k, int64_t n, h
 // reduce_k's whole grid at once and its longer way through LDS shows, above all where the streams still lie in the
 // Infinity Cache.  fp32, us of a launch over the same buffers again: 3 peers and 64 MiB 9.4 and 10.2 split, 128 MiB 20.2
 // and 21.1, 192 MiB 33.8 and 32.8; 5 peers and 48 MiB 7.2 and 7.5, 96 MiB 15.0 and 14.7; 6 peers and 64 MiB 9.6 and
-// 10.1; 8 peers and 64 MiB 9.7 and 10.5, 96 MiB the same; 7 peers and 64 MiB 9.5 and 9.3, 96 MiB 14.8 and 14.3.  Over
-// buffers that take turns: 3 peers and 64 MiB 12.2 and 12.6, 192 MiB 38.8 and 38.0; 7 peers and 96 MiB 17.8 and 17.3.
+// 10.1; 8 peers and 64 MiB 9.7 and 10.5, 96 MiB the same.  Over buffers that take turns: 3 peers and 64 MiB 12.2 and
+// 12.6, 192 MiB 38.8 and 38.0.  Seven peers have two streams for each of four wavefronts and one vector for each lane,
+// and gain first: 48 MiB the same either way, 64 MiB 9.5 and 9.3 (12.3 and 12.1 in turn), 96 MiB 14.8 and 14.3.
 template <int K>
-constexpr uint64_t kSplitFrom = (K == 3 ? 192ull : 96ull) << 20;
+constexpr uint64_t kSplitFrom = (K == 3 ? 192ull : K == 7 ? 48ull : 96ull) << 20;
 
 template <typename T, int K>
 int launch_k(void* resident, const void* const* incoming, int64_t n, hipStream_t stream) {

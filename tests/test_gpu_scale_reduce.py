@@ -179,11 +179,11 @@ def test_scaled_bytes_beyond_their_range_leave_the_ones_beside_alone(gpu, orc, d
 @pytest.mark.parametrize("dtype", [U8, F16, F32, F64])
 @pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8])
 def test_reduce_sum_k_of_streams_split_over_wavefronts(gpu, orc, dtype, k):
-    """From 96 MiB of all streams on (192 with three peers): tiles of 64 or 128 vectors, at a size that they divide,
+    """From 96 MiB of all streams on (192 with three peers, 48 with seven): tiles of 64 or 128 vectors, at a size that they divide,
     one element either side of it, and with a ragged end; the elements behind the chunk stay."""
     rng = np.random.default_rng(k)
     es = SIZE_OF[dtype]
-    base = (((192 if k == 3 else 96) << 20) // (k + 1) // es // (2048 // es) + 1) * (2048 // es)
+    base = (({3: 192, 7: 48}.get(k, 96) << 20) // (k + 1) // es // (2048 // es) + 1) * (2048 // es)
     host = [(rng.integers(0, 100, base + 80) * (1 if dtype == U8 else 0.37)).astype(NP_OF[dtype]) for _ in range(k + 1)]
     peers = [gpu.upload(h) for h in host[1:]]
     for n in (base - 1, base, base + 1, base + 77):
