@@ -11,11 +11,13 @@
 //            level and leaves the sums of the two                            (R + R/2, R/2 + R/4 ...)
 //   last_k   reads the last two, combines them, stores the result into the outputs            (2 + 1)
 //
-// 29 vectors for eight ranks, in 4 launches instead of 23.  Every pass is bound by memory: a BERT-large layer (16
-// tensors, 50 MB) of eight ranks takes 224 us, 6.5 TB/s over the 1.46 GB that the passes move (dots_k 62, level_k 88
-// and 44, last_k 23 us); the separate steps move 2.67 GB in 443 us.  What level_k stores goes through the Infinity
-// Cache to its reader (non-temporal stores: 248 us).  Sums of all pairs at once would spare the levels their own
-// (17 vectors), but a level's norm as a difference of the ranks' products has no digits left where ranks nearly cancel.
+// 29 vectors for eight ranks, in 4 launches instead of 23, and a launch of coeffs_k between two passes where a tensor has
+// more than 512 chunks.  Every pass is bound by memory: a BERT-large layer (16 tensors, 50 MB, four of them of 1,024
+// chunks) of eight ranks takes 230 us in 7 launches: dots_k 62, level_k 86 and 44, last_k 23.5 us, 6.8 TB/s over the 1.46
+// GB that the passes move, and 15 us of coeffs_k; the separate steps move 2.67 GB in 443 us.  What level_k stores goes
+// through the Infinity Cache to its reader (non-temporal stores take the passes 24 us more).  Sums of all pairs at once
+// would spare the levels their own (17 vectors), but a level's norm as a difference of the ranks' products has no digits
+// left where ranks nearly cancel.
 //
 // All roundings are those of the separate steps: to the wire type after the prescale, after every level's scaled add
 // and in the output.  The sums are taken in double in an order that depends on the tensor's size alone.

@@ -177,7 +177,7 @@ enum class Stores {
   kUnpackWidening = 4,  // fp16 -> fp32 unpack
   kContig = 5,      // whole-buffer scale
   kReduceFew = 6,   // reduce-sum of one or two peers
-  kReduceMany = 7,  // reduce-sum of three to eight peers
+  kReduceMany = 7,  // reduce-sum of three to fifteen peers
   kAdasum = 8,      // scaled add
 };
 int store_policy(Stores family);  // a StorePolicy value

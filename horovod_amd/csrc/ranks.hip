@@ -6,7 +6,7 @@
 // summed into the first, which is unpacked -- moves every byte three times (2 per packing rank,
 // world + 1 for the sum, 2 for the unpack: 27 passes over the tensors for 8 ranks where 9 do).
 // It is bound by memory in both forms: ResNet-50's gradients (102 MB) of 8 ranks took 222 us of
-// kernels and take 151 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 2.2 ms (8 read
+// kernels and take 152 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 1.95 ms (8 read
 // streams from HBM: 6.1-6.5 TB/s).  Results are the same to the bit: the same roundings in the
 // same order (to the wire type after the prescale and after every rank).
 //

@@ -149,8 +149,7 @@ constexpr int kSplitVecs = (K + 1) % kSplitWaves<K> == 0 ? 1 : 2;
 // w, w + WV ... (stream 0 is the resident chunk), all meet in LDS, and the first U wavefronts add them in peer order
 // and store.  It has a quarter of reduce_k's bytes under way (2,048 workgroups of 1 KiB per stream instead of 4), which
 // the memory serves faster once they are more than latency times bandwidth: 33 million fp32 and 7 peers 175 -> 170 us
-// (7.0 TB/s), 3 peers 95.5 -> 90.8, 5 peers 138 -> 129, 8 peers 194.5 -> 188, 15 peers 370 -> 357; fp16 and 7 peers
-// 88.6 -> 86.7.  A wavefront with one stream less than another waits for less, so there a lane takes two vectors.
+// (7.0 TB/s), 3 peers 95.5 -> 90.8, 5 peers 138 -> 129, 8 peers 194.5 -> 188; fp16 and 7 peers 88.6 -> 86.7.  A wavefront with one stream less than another waits for less, so there a lane takes two vectors.
 template <typename T, int K, int ST>
 __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* resident, uint64_t n, uint32_t shift,
                                                                       uint32_t ordered, const T* p0, const T* p1,
@@ -206,9 +205,10 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
 }
 
 // Nine to fifteen peers in one launch: half as many wavefronts as streams, two streams each (the last may have one).
-// In two launches of up to eight peers the resident chunk is written and read once more: 33 million fp32 and 9 peers
-// 242 us in two, 210 in one (6.9 TB/s), 10 peers 259 and 226, 15 peers 357 and 337, fp16 and 12 peers 154 and 137,
-// uint8 and 12 peers of 40 million 96 and 86; 300,000 fp32 and 9 peers 10 and 6.4.  (With eight wavefronts for any number 10 peers take 267 us.)
+// In two launches of reduce_k the resident chunk is written and read once more: 33 million fp32 and 9 peers 249 us in
+// two, 209 in one (6.9 TB/s), 10 peers 267 and 226, 15 peers 372 and 332, fp16 and 12 peers 158 and 137; 8 million uint8
+// and 15 peers 27.4 and 23.8; 300,000 fp32 and 9 peers 9.6 and 5.4.  (With eight wavefronts for any number 10 peers take
+// 267 us.)
 constexpr int kMostWaves = 8;
 constexpr int kManyStreams = 2 * kMostWaves;
 template <typename T>

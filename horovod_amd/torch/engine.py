@@ -17,8 +17,9 @@ this process is rank 0.  What ranks 1..size-1 contribute comes from ``peer_sourc
 tensor)``; by default every rank holds the same values, which is what the reference's own
 tests arrange by seeding all ranks alike (test/parallel/test_torch.py:251-445).  All of
 them sit in this GPU's memory, so a sum needs no fusion buffer: the kernel reads every rank's tensors
-where they are, with the roundings that packing, summing and unpacking would make.  Adasum packs
-every node's tensors into a buffer and combines the buffers pairwise.
+where they are, with the roundings that packing, summing and unpacking would make.  Adasum reads them
+so too, a pass per level of the pairwise tree; only where a node has several ranks are these summed into
+a buffer per node first.
 """
 import ctypes
 from ctypes import c_int, c_int64, c_void_p

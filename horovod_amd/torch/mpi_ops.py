@@ -10,7 +10,7 @@ pair of scale factors that reaches the kernels:
   does in non-ROCm builds (common/operations.cc:1394-1398).  The reference's ROCm build
   cannot do that (it has no scale kernels: ops/hip_operations.cc:150-153) and divides in the
   framework instead (mpi_ops.py:100-105, mpi_ops_v2.cc:69-77,118-120); with the kernels of
-  this library the division rides on the unpack.
+  this library the division rides on the pass that stores the result.
 * ``Adasum`` on the GPU averages over the ranks of a node the same way, ``postscale_factor /
   local_size()`` (common/operations.cc:1403-1408), and needs a power-of-two number of nodes.
 
@@ -248,7 +248,7 @@ class HorovodAllreduce(torch.autograd.Function):
 def allreduce(tensor, average=None, name=None, compression=Compression.none, op=None,
               prescale_factor=1.0, postscale_factor=1.0):
     """Allreduce into a new tensor; differentiable.  With Compression.fp16 on a float32 device
-    tensor the cast each way happens inside the pack and unpack kernels."""
+    tensor the cast each way happens inside the kernel that sums the ranks."""
     if _fused_fp16(compression, tensor):
         return HorovodAllreduce.apply(tensor, average, name, op, prescale_factor, postscale_factor, torch.float16)
     tensor_compressed, ctx = compression.compress(tensor)

@@ -16,8 +16,8 @@ the factory returns the delta-based variant (optimizer.py:333-503) instead.
 Two things differ from the reference on purpose.  The ROCm refusal of
 ``gradient_predivide_factor`` (optimizer.py:570-572) is gone, because the scale kernels it
 was waiting for exist here.  And ``Compression.fp16`` on float32 gradients allocates
-nothing: the request carries the gradient itself with float16 as the dtype of the fusion
-buffer, and the pack and unpack kernels do the two casts.
+nothing: the request carries the gradient itself with float16 as the dtype on the wire, and
+the kernel that sums the ranks does the two casts.
 """
 import warnings
 from contextlib import contextmanager

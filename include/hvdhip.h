@@ -55,7 +55,7 @@ enum hvdhip_dtype {
 /* A plan or batched copy needs more than 2^23 workgroups (32 GiB at 4 KiB each) in one launch.
  * Contiguous entry points (scale, reduce) have no such limit: they slice. */
 #define HVDHIP_ERR_TOO_LARGE (-4)
-/* hvdhip_ranks_sum(): an output overlaps another output or another entry's input. */
+/* hvdhip_ranks_sum(), hvdhip_adasum_ranks(): an output overlaps another output or another entry's input. */
 #define HVDHIP_ERR_OVERLAP (-5)
 
 /* Flags of hvdhip_fusion_pack(). */
