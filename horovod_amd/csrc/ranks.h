@@ -57,32 +57,42 @@ __device__ __forceinline__ half_t scaled<half_t>(half_t x, float s) {
   return (half_t)opaque(s * (float)x);
 }
 
+template <typename S, typename D, int N>
+__device__ __forceinline__ Arr<D, N> converted(const Arr<S, N>& x) {
+  if constexpr (std::is_same<S, D>::value) {
+    return x;
+  } else {
+    Arr<D, N> y;
+#pragma unroll
+    for (int j = 0; j < N; ++j) y.v[j] = (D)x.v[j];
+    return y;
+  }
+}
+
 // N elements on their way in (tensor type S to wire type W) and out (W to D): converted before or
 // after the wire, scaled on it (compress, then scale: horovod/torch/compression.py:49-55 before the
 // fp16 ScaleBuffer; the converting unpack scales the half and widens).  16-bit integers are summed and
 // copied but never scaled.
 template <typename W, int N>
 __device__ __forceinline__ void scale_all(Arr<W, N>& x, typename Factor<W>::type s) {
-  if constexpr (!std::is_same<W, uint16_t>::value) {
+  if constexpr (sizeof(W) == 1 && N == 16) {
+    asm volatile("");  // or the compiler scales in any case and picks one of the two
+    x = scaled_bytes(x, s);
+  } else if constexpr (!std::is_same<W, uint16_t>::value) {
 #pragma unroll
     for (int j = 0; j < N; ++j) x.v[j] = scaled<W>(x.v[j], s);
   }
 }
 template <typename S, typename W, int N>
 __device__ __forceinline__ Arr<W, N> to_wire(const Arr<S, N>& x, typename Factor<W>::type s, bool scale) {
-  Arr<W, N> y;
-#pragma unroll
-  for (int j = 0; j < N; ++j) y.v[j] = (W)x.v[j];
+  Arr<W, N> y = converted<S, W, N>(x);
   if (scale) scale_all(y, s);
   return y;
 }
 template <typename W, typename D, int N>
 __device__ __forceinline__ Arr<D, N> from_wire(Arr<W, N> x, typename Factor<W>::type s, bool scale) {
   if (scale) scale_all(x, s);
-  Arr<D, N> y;
-#pragma unroll
-  for (int j = 0; j < N; ++j) y.v[j] = (D)x.v[j];
-  return y;
+  return converted<W, D, N>(x);
 }
 
 template <typename S, typename D>

@@ -125,17 +125,14 @@ __global__ __launch_bounds__(kWG) void reduce_k(T* resident, uint64_t n, uint32_
   }
 }
 
-// Sixteen bytes of a stream on their way through LDS: one register quadruple for every type.  As an Arr of bytes the
-// compiler takes a load apart into sixteen registers wherever two branches meet, and waits for it to do so, one load
-// after the other: 512 MiB of uint8 streams, 5 peers 112 us and 86 in this form, 8 peers 142 and 86.
-typedef RawSel<16>::type Quad;
+// Vector v of a workgroup's `bytes` of a stream.
 template <typename T>
-__device__ __forceinline__ Quad load_quad(gptr<const T> p, uint32_t bytes, uint32_t v) {
+__device__ __forceinline__ Arr<T, 16 / (int)sizeof(T)> load_vec(gptr<const T> p, uint32_t bytes, uint32_t v) {
+  constexpr int VEC = 16 / (int)sizeof(T);
   if constexpr (sizeof(T) == 1) {
-    return __builtin_bit_cast(Quad, ldw<T, 16>(load_window(p, bytes), v * 16u));
+    return ldw<T, VEC>(load_window(p, bytes), v * 16u);
   } else {
-    constexpr int VEC = 16 / (int)sizeof(T);
-    return __builtin_bit_cast(Quad, ldv<T, VEC>(p + (size_t)v * VEC));
+    return ldv<T, VEC>(p + (size_t)v * VEC);
   }
 }
 
@@ -158,7 +155,7 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
   constexpr int VEC = 16 / (int)sizeof(T), WV = kSplitWaves<K>, U = kSplitVecs<K>, R = K + 1, L = (R + WV - 1) / WV;
   constexpr uint32_t kTile = 64 * U * VEC;
   typedef Arr<T, VEC> V;
-  __shared__ Quad lds[R][64 * U];
+  __shared__ V lds[R][64 * U];
   const T* const ps[kMaxK + 1] = {resident, p0, p1, p2, p3, p4, p5, p6, p7};
   const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
   const uint64_t left = n - start;
@@ -167,13 +164,13 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
 #pragma unroll
   for (int w = 0; w < WV; ++w) {  // a branch per wavefront keeps the streams' addresses in scalar registers
     if (wave != (uint32_t)w) continue;
-    Quad x[U][L];
+    V x[U][L];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int i = 0; i < L; ++i) {
         const uint32_t v = u * 64 + lane;
-        if (w + i * WV < R && v < nv) x[u][i] = load_quad<T>(as_global(ps[w + i * WV] + start), m, v);
+        if (w + i * WV < R && v < nv) x[u][i] = load_vec<T>(as_global(ps[w + i * WV] + start), m, v);
       }
     }
 #pragma unroll
@@ -190,9 +187,9 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void reduce_split_k(T* residen
   const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
   const uint32_t v = threadIdx.x;
   if (v < nv) {
-    V acc = __builtin_bit_cast(V, lds[0][v]);
+    V acc = lds[0][v];
 #pragma unroll
-    for (int k = 1; k < R; ++k) accumulate<T, VEC>(acc, __builtin_bit_cast(V, lds[k][v]));
+    for (int k = 1; k < R; ++k) accumulate<T, VEC>(acc, lds[k][v]);
     stw<ST, T, VEC>(out, v * 16u, acc);
   }
   const uint32_t t = nv * VEC + threadIdx.x;
@@ -221,7 +218,7 @@ __global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, ui
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr uint32_t kTile = 64 * VEC;
   typedef Arr<T, VEC> V;
-  __shared__ Quad lds[kManyStreams][64];
+  __shared__ V lds[kManyStreams][64];
   const uint64_t start = (uint64_t)xcd_tile(blockIdx.x, XcdOrder{shift, ordered}) * kTile;
   const uint64_t left = n - start;
   const uint32_t m = left < kTile ? (uint32_t)left : kTile;
@@ -232,8 +229,8 @@ __global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, ui
     // The last wavefront's second stream may be its first once more: a branch there has the compiler wait for
     // the first before it asks for the second.
     const uint32_t other = w + waves < streams ? w + waves : w;
-    const Quad x = load_quad<T>(as_global(s.p[w] + start), m, lane);
-    const Quad y = load_quad<T>(as_global(s.p[other] + start), m, lane);
+    const V x = load_vec<T>(as_global(s.p[w] + start), m, lane);
+    const V y = load_vec<T>(as_global(s.p[other] + start), m, lane);
     lds[w][lane] = x;
     lds[other][lane] = y;
   }
@@ -242,8 +239,8 @@ __global__ __launch_bounds__(64 * kMostWaves) void reduce_many_k(T* resident, ui
   gptr<T> r = as_global(resident + start);
   const Window out = store_window<ST>(r, m * (uint32_t)sizeof(T));
   if (lane < nv) {
-    V acc = __builtin_bit_cast(V, lds[0][lane]);
-    for (uint32_t k = 1; k < streams; ++k) accumulate<T, VEC>(acc, __builtin_bit_cast(V, lds[k][lane]));
+    V acc = lds[0][lane];
+    for (uint32_t k = 1; k < streams; ++k) accumulate<T, VEC>(acc, lds[k][lane]);
     stw<ST, T, VEC>(out, lane * 16u, acc);
   }
   const uint32_t t = nv * VEC + lane;

@@ -155,8 +155,10 @@ def test_contiguous_kernels_reach_their_first_load_without_a_scalar_branch(kerne
         first = next(i for i, op in enumerate(ops) if op.startswith(("global_load", "buffer_load")))
         head = ops[:first]
         assert not any(op.startswith("s_cbranch_scc") for op in head), name
-        # the compatibility prologue for firmware that does not preload waits once, the kernel proper at most once
-        assert sum(op == "s_waitcnt" for op in head) <= 2, (name, head)
+        # the compatibility prologue for firmware that does not preload waits once, the kernel proper at most once, and a
+        # wavefront of the split sums once more for the addresses of its own streams
+        split = re.search(r"reduce_(split|many)_k", name) is not None
+        assert sum(op == "s_waitcnt" for op in head) <= 2 + split, (name, head)
         checked += 1
     assert checked >= 100, checked
 
