@@ -159,7 +159,15 @@ struct UnpackF16F32 {
   }
 };
 
-constexpr int kUnroll = 4;  // 16-byte loads in flight per lane, for chunks of more than one vector per lane
+// 16-byte loads in flight per lane, for chunks of more than one vector per lane.  Two for scaled bytes, whose sixteen
+// products in double take registers: with four the kernel has 90 of them, and fewer wavefronts fit beside each other
+// (1 GiB of uint8 from tensor to tensor 440 us with four, 390 with two).
+template <class Op>
+constexpr int kUnroll = 4;
+template <>
+constexpr int kUnroll<Scale<uint8_t, double>> = 2;
+template <>
+constexpr int kUnroll<Scale<int8_t, double>> = 2;
 
 // Streams n elements from src to dst through Op::f with the whole workgroup.
 template <class Op, int ST>
@@ -184,13 +192,14 @@ __device__ __forceinline__ void stream_range(gptr<const typename Op::S> src,
       return ldv<S, VEC>(src + (size_t)vec * VEC);
     }
   };
+  constexpr int U = kUnroll<Op>;
   uint32_t v = threadIdx.x;
-  for (; v + (kUnroll - 1) * kWG < nv; v += kUnroll * kWG) {
-    Arr<S, VEC> x[kUnroll];
+  for (; v + (U - 1) * kWG < nv; v += U * kWG) {
+    Arr<S, VEC> x[U];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) x[u] = load(v + u * kWG);
+    for (int u = 0; u < U; ++u) x[u] = load(v + u * kWG);
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+    for (int u = 0; u < U; ++u)
       stw<ST, D, VEC>(out, (v + u * kWG) * (uint32_t)(VEC * sizeof(D)), apply<Op>(x[u], p));
   }
   for (; v < nv; v += kWG) stw<ST, D, VEC>(out, v * (uint32_t)(VEC * sizeof(D)), apply<Op>(load(v), p));
