@@ -164,7 +164,8 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
 // 85.8 -> 83.7, 5 ranks 106 -> 99, 6 ranks 123 -> 118, below 16 MiB per rank no difference.  With an odd number of
 // ranks a wavefront has one load to wait for, so a lane takes two vectors of each (5 ranks, one vector: 112 us); more
 // per workgroup in a loop that loads ahead is slower (4 tiles: 161 us, 8: 176).  Runs of 256 KiB per XCD gain 1-4 % at
-// 3 to 6 ranks; with 8 ResNet-50's take 155 us in them.
+// 3 to 6 ranks; with 8 they lose 2-5 % on the responses of ResNet-50, BERT-large and GPT-2 XL and on single tensors from
+// 64 MiB a rank on (200 MiB 288 and 304 us), and gain up to 16 MiB (4 MiB 9.1 and 7.9).
 template <typename S, typename W, typename D, int K, int ST>
 __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t shift, uint32_t ordered, uint32_t nrows,
                                                                      double pre, double post, uint32_t flags,
