@@ -17,12 +17,16 @@
 // rounded once.  In the combine, when no layer has more than 512 triples, pass 2
 // does pass 1b's work itself (every workgroup re-adds its layer's triples in that
 // same fixed order under the shadow of its data loads) and pass 1b is not launched.
+// Layers that fit the registers of one workgroup are combined in one launch
+// (combine_held_k), with the same operations in the same order.
 //
 // Products of two fp32 (or fp16) values are exact in double, so only the
 // order of the double additions differs from the reference's sequential
 // loop.  Bandwidth-bound: 3 double fmas per 8 bytes read in pass 1.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <cstring>
 #include <list>
 #include <mutex>
 
@@ -278,6 +282,150 @@ __global__ __launch_bounds__(kWG) void scaled_add_k(const Chunk* __restrict__ ch
   if (t < n) pa[t] = Axpby<T>::f(ca, pa[t], cb, pb[t]);
 }
 
+// A layer's place in the vectors, for the kernel that takes whole layers.
+struct Span {
+  uint64_t start;  // first element
+  uint32_t n;
+  uint32_t chunks;
+};
+
+// A chunk of at most kAdasumChunkBytes of both vectors in the registers of 256 lanes, with the order of operations of
+// dot_partials_k: a lane with four vectors takes them over two chains, one with fewer over the first chain alone, and
+// the elements behind the last whole vector go to the second.
+// The vectors stay as they were loaded: pinned() hides that both uses widen the same elements, or the compiler keeps
+// those of 16 bits in four times the registers from one use to the next.
+template <typename T>
+struct Held {
+  static constexpr int VEC = 16 / (int)sizeof(T);
+  typedef Arr<T, VEC> V;
+  typedef RawSel<16>::type R;
+  gptr<T> pa;
+  uint32_t n, nv, lane;
+  R x[kUnroll], y[kUnroll];
+  T xt, yt;
+
+  static __device__ __forceinline__ V pinned(R& r) {
+    asm("" : "+v"(r));
+    return __builtin_bit_cast(V, r);
+  }
+
+  __device__ __forceinline__ void load(T* a, const T* b, uint64_t start, uint32_t count, uint32_t lane_) {
+    pa = as_global(a + start);
+    const gptr<const T> pb = as_global(b + start);
+    n = count;
+    nv = n / VEC;
+    lane = lane_;
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      if (lane + u * kWG < nv) {
+        x[u] = __builtin_bit_cast(R, ldv<T, VEC>(gptr<const T>(pa) + (size_t)(lane + u * kWG) * VEC));
+        y[u] = __builtin_bit_cast(R, ldv<T, VEC>(pb + (size_t)(lane + u * kWG) * VEC));
+      }
+    }
+    if (nv * VEC + lane < n) {
+      xt = pa[nv * VEC + lane];
+      yt = pb[nv * VEC + lane];
+    }
+  }
+
+  __device__ __forceinline__ Triple sums() {
+    double d[2] = {0., 0.}, p[2] = {0., 0.}, q[2] = {0., 0.};
+    auto add = [&](int chain, T xe, T ye) {
+      const double xd = (double)xe, yd = (double)ye;
+      d[chain] = fma(xd, yd, d[chain]);
+      p[chain] = fma(xd, xd, p[chain]);
+      q[chain] = fma(yd, yd, q[chain]);
+    };
+    if (lane + (kUnroll - 1) * kWG < nv) {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const V xv = pinned(x[u]), yv = pinned(y[u]);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) add(j & 1, xv.v[j], yv.v[j]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kUnroll - 1; ++u) {
+        if (lane + u * kWG >= nv) break;
+        const V xv = pinned(x[u]), yv = pinned(y[u]);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) add(0, xv.v[j], yv.v[j]);
+      }
+    }
+    if (nv * VEC + lane < n) add(1, xt, yt);
+    return Triple{d[0] + d[1], p[0] + p[1], q[0] + q[1]};
+  }
+
+  __device__ __forceinline__ void add(double ca, double cb) {
+    const Window out = store_window<kStoreNT>(pa, n * (uint32_t)sizeof(T));
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      if (lane + u * kWG >= nv) break;
+      V r = pinned(x[u]);
+      const V yv = pinned(y[u]);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) r.v[j] = Axpby<T>::f(ca, r.v[j], cb, yv.v[j]);
+      stw<kStoreNT, T, VEC>(out, (lane + u * kWG) * 16u, r);
+    }
+    if (nv * VEC + lane < n) pa[nv * VEC + lane] = Axpby<T>::f(ca, xt, cb, yt);
+  }
+};
+
+// The whole combine of layers that fit the registers of a workgroup, one workgroup each: both vectors are read once,
+// kept while the sums go through LDS, and written from there: three vectors of traffic in one launch instead of five in
+// two.  G groups of 256 lanes have C chunks each.  Bound by the chain of one workgroup (load, sums, two trips through
+// LDS and lanes, divide, store: about 3 us with the launch) where the device holds all of them, by memory beyond: 61 fp16
+// layers of a few hundred to 19,000 elements 6.4 -> 4.4 us, 1,000 fp32 layers of 16 KB 13.7 -> 9.5.
+template <typename T, int G, int C>
+__global__ __launch_bounds__(G * kWG) void combine_held_k(const Span* __restrict__ spans, T* a,
+                                                          const T* __restrict__ b, double* __restrict__ normdots,
+                                                          double* __restrict__ coeffs, double guard) {
+  constexpr uint32_t kUnits = kAdasumChunkBytes / (uint32_t)sizeof(T);
+  const Span s = spans[blockIdx.x];
+  const uint32_t group = threadIdx.x / kWG, lane = threadIdx.x % kWG, l64 = threadIdx.x & 63;
+  Held<T> held[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const uint32_t k = group + c * G;  // chunks are cut at multiples of their size from the vectors' start
+    const uint64_t cut = (s.start / kUnits + k) * kUnits, end = s.start + s.n;
+    const uint64_t from = k == 0 ? s.start : cut, to = cut + kUnits < end ? cut + kUnits : end;
+    held[c].load(a, b, from, k < s.chunks ? (uint32_t)(to - from) : 0, lane);
+  }
+  __shared__ double red[C * G][3][kWG / 64];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    Triple t = held[c].sums();
+    t.d = wave_sum(t.d);
+    t.a = wave_sum(t.a);
+    t.b = wave_sum(t.b);
+    if (l64 == 63) {
+      double(&to)[3][kWG / 64] = red[group + c * G];
+      to[0][lane / 64] = t.d;
+      to[1][lane / 64] = t.a;
+      to[2][lane / 64] = t.b;
+    }
+  }
+  __syncthreads();
+  // Every wavefront adds the chunks' sums for itself, with the bits that finalize_k gets: there lane i has triple i, and
+  // those of a layer of at most 16 meet in the first row of 16 lanes.  Here each of the three sums has a row.
+  const uint32_t chunk = l64 & 15, which = l64 / 16;
+  double r = 0.;
+  if (which < 3 && chunk < s.chunks) {
+#pragma unroll
+    for (int w = 0; w < kWG / 64; ++w) r += red[chunk][which][w];
+  }
+  if (C * G > 1) r = row_sum(r);
+  constexpr int kAt = C * G > 1 ? 15 : 0;
+  const Triple t = {0. + lane_value(r, kAt), 0. + lane_value(r, 16 + kAt), 0. + lane_value(r, 32 + kAt)};
+  double ca, cb;
+  layer_coeffs(t, guard, &ca, &cb);
+  if (threadIdx.x < 3)
+    normdots[3 * (uint64_t)blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? t.d : threadIdx.x == 1 ? t.a : t.b;
+  if (threadIdx.x < 2) coeffs[2 * (uint64_t)blockIdx.x + threadIdx.x] = threadIdx.x ? cb : ca;
+#pragma unroll
+  for (int c = 0; c < C; ++c) held[c].add(ca, cb);
+}
+
 // Writes the chunk and layer tables of a single layer of `count` elements, as
 // hvdhip_adasum_plan_create lays them out for one layer: chunk c starts at element
 // c * chunk_units and sits at table position xcd_slot(c).
@@ -317,7 +465,8 @@ struct hvdhip_adasum_plan {
   uint32_t max_layer_chunks = 0;
   DevTables tables;
   Layer* layers = nullptr;    // device, nlayers entries
-  double* results = nullptr;  // one allocation: partials | normdots | coeffs | layer table
+  Span* spans = nullptr;      // device, nlayers entries; NULL in a view of the static scratch
+  double* results = nullptr;  // one allocation: partials | normdots | coeffs | spans | layer table
   double* partials = nullptr;
   double* normdots = nullptr;
   double* coeffs = nullptr;
@@ -405,6 +554,48 @@ int plan_scaled_add(hvdhip_adasum_plan* p, void* a, const void* b, const double*
 // 64 layers of 2^25 elements, 3.5 % at 1,000 layers, 9 % at 2^22 elements).
 bool fused_coeffs(const hvdhip_adasum_plan* p) {
   return p->tables.nchunks > 0 && p->max_layer_chunks <= 2 * (uint32_t)kWG;
+}
+
+// Whether the combine is one launch of combine_held_k, with as many lanes for every layer as the longest one needs.
+// Measured against the two passes, us, fp32 (fp16 and fp64 alike): one layer of 1 chunk 3.6 and 7.3, of 4 chunks 4.8 and
+// 7.5; 256 layers of 1 chunk 4.6 and 8.6, of 3 chunks 6.7 and 10.1, of 7 chunks 13.2 and 24.4; 1,000 layers of 4 chunks
+// 36.7 and 49.3.  The lines: what the device holds at once costs one workgroup's time however little a layer has (400
+// layers of up to 4 chunks, most of them short, 5.4 and 6.0; 800: 8.8 and 6.0); beyond, and for the eight chunks that a
+// compute unit takes 6 us over (8 layers of 7 chunks 7.2 and 7.4, fp16 9.7 and 7.7), the lanes have to be used: 2,000
+// layers of up to 2 chunks 10.1 and 8.8 with 500 bytes each, 12.2 and 11.8 with 6.5 KB, 18.9 and 31.8 with 16 KB.
+bool held_layers(const hvdhip_adasum_plan* p) {
+  const uint64_t layers = (uint64_t)p->nlayers;
+  if (!p->spans || layers > kMaxWorkgroups / 4 || chunk_bytes(Family::kAdasum) != kAdasumChunkBytes) return false;
+  const uint64_t bytes = (uint64_t)p->total * (uint64_t)dtype_size(p->dtype);
+  const uint64_t chunk = kAdasumChunkBytes;
+  if (p->max_layer_chunks <= 2) return layers <= 1000 || bytes >= layers * chunk / 2;
+  if (p->max_layer_chunks <= 4) return layers <= 400 || bytes >= layers * chunk * 2;
+  return p->max_layer_chunks <= 8 && layers >= 200 && bytes >= layers * chunk * 4;
+}
+
+template <typename T, int G, int C>
+hipError_t launch_held(hvdhip_adasum_plan* p, void* a, const void* b, hipStream_t s) {
+  return launch_shaped(nullptr, combine_held_k<T, G, C>, (uint32_t)p->nlayers, G * kWG, s, p->spans, static_cast<T*>(a),
+                       static_cast<const T*>(b), p->normdots, p->coeffs, std::sqrt(DBL_MIN));
+}
+template <typename T>
+hipError_t launch_held(hvdhip_adasum_plan* p, void* a, const void* b, hipStream_t s) {
+  if (p->max_layer_chunks <= 1) return launch_held<T, 1, 1>(p, a, b, s);
+  if (p->max_layer_chunks <= 2) return launch_held<T, 2, 1>(p, a, b, s);
+  if (p->max_layer_chunks <= 4) return launch_held<T, 4, 1>(p, a, b, s);
+  return launch_held<T, 4, 2>(p, a, b, s);
+}
+
+int plan_combine_held(hvdhip_adasum_plan* p, void* a, const void* b, hipStream_t s) {
+  if (p->nlayers == 0) return 0;
+  hipError_t status;
+  switch (p->dtype) {
+  case HVDHIP_FLOAT16: status = launch_held<half_t>(p, a, b, s); break;
+  case HVDHIP_FLOAT32: status = launch_held<float>(p, a, b, s); break;
+  default: status = launch_held<double>(p, a, b, s); break;
+  }
+  HVDHIP_CHECK_LAUNCH("combine_held_k", status);
+  return 0;
 }
 
 int check_vectors(const hvdhip_adasum_plan* p, const void* a, const void* b) {
@@ -519,6 +710,7 @@ int hvdhip_adasum_plan_create(const int* tensor_counts, int nlayers, int dtype,
     return fail(HVDHIP_ERR_UNSUPPORTED_DTYPE, "Adasum supports FLOAT16, FLOAT32 and FLOAT64, not dtype %d", dtype);
   const uint32_t chunk_units = chunk_bytes(Family::kAdasum) / (uint32_t)dtype_size(dtype);
   std::vector<Layer> layers((size_t)nlayers);
+  std::vector<Span> spans((size_t)nlayers);
   std::vector<Chunk> chunks;
   uint64_t off = 0;
   uint32_t max_layer_chunks = 0;
@@ -544,6 +736,7 @@ int hvdhip_adasum_plan_create(const int* tensor_counts, int nlayers, int dtype,
       chunks[c].output |= (uint64_t)layers[(size_t)i].first << 32;
       chunks[c].pad = layers[(size_t)i].count;
     }
+    spans[(size_t)i] = Span{off, (uint32_t)n, layers[(size_t)i].count};
     if (layers[(size_t)i].count > max_layer_chunks) max_layer_chunks = layers[(size_t)i].count;
     if (chunks.size() > kMaxWorkgroups) return fail(HVDHIP_ERR_TOO_LARGE, "the vectors need more than 2^23 workgroups");
     off += n;
@@ -566,11 +759,15 @@ int hvdhip_adasum_plan_create(const int* tensor_counts, int nlayers, int dtype,
     return rc;
   }
   const size_t ndoubles = 3 * (size_t)p->tables.nchunks + 5 * (size_t)nlayers + 8;
-  const size_t layer_bytes = (size_t)nlayers * sizeof(Layer);
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->results), ndoubles * sizeof(double) + layer_bytes);
+  const size_t layer_bytes = (size_t)nlayers * sizeof(Layer), span_bytes = (size_t)nlayers * sizeof(Span);
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->results), ndoubles * sizeof(double) + span_bytes + layer_bytes);
+  unsigned char* const tables_at = reinterpret_cast<unsigned char*>(p->results + ndoubles);
   if (e == hipSuccess) e = hipMemset(p->results, 0, ndoubles * sizeof(double));
-  if (e == hipSuccess && nlayers > 0)
-    e = hipMemcpy(p->results + ndoubles, layers.data(), layer_bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess && nlayers > 0) {
+    spans.resize((size_t)nlayers * (1 + (sizeof(Layer) + sizeof(Span) - 1) / sizeof(Span)));  // both tables in one copy
+    std::memcpy(reinterpret_cast<unsigned char*>(spans.data()) + span_bytes, layers.data(), layer_bytes);
+    e = hipMemcpy(tables_at, spans.data(), span_bytes + layer_bytes, hipMemcpyHostToDevice);
+  }
   // the fill above may return before the device has done it; the plan is used on other streams
   if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   if (e != hipSuccess) {
@@ -581,7 +778,8 @@ int hvdhip_adasum_plan_create(const int* tensor_counts, int nlayers, int dtype,
     return fail(e == hipErrorOutOfMemory ? HVDHIP_ERR_OUT_OF_MEMORY : (int)e,
                 "allocating Adasum results failed: %s", hipGetErrorString(e));
   }
-  p->layers = reinterpret_cast<Layer*>(p->results + ndoubles);
+  p->spans = reinterpret_cast<Span*>(tables_at);
+  p->layers = reinterpret_cast<Layer*>(tables_at + span_bytes);
   p->partials = p->results;
   p->normdots = p->partials + 3 * (size_t)p->tables.nchunks;
   p->coeffs = p->normdots + 3 * (size_t)nlayers;
@@ -617,6 +815,10 @@ int hvdhip_adasum_combine(hvdhip_adasum_plan* plan, void* a, const void* b, void
   int rc = check_vectors(plan, a, b);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (held_layers(plan)) {
+    rc = plan_combine_held(plan, a, b, s);
+    return rc ? rc : ok();
+  }
   const bool fused = fused_coeffs(plan);
   rc = plan_dot_norms(plan, a, b, s, !fused);
   if (rc) return rc;

@@ -24,17 +24,27 @@ __device__ __forceinline__ double dpp_add(double x) {
   return x + __hiloint2double(hi2, lo2);
 }
 
-// Sum over the 64 lanes of a wavefront in a fixed order; the total arrives in lane 63.  Within
-// each row of 16 lanes a shifted-add scan (by 1, 2, 4, 8), then lane 15 of rows 0 and 2 into rows
-// 1 and 3, then lane 31 into rows 2 and 3.
-__device__ __forceinline__ double wave_sum(double x) {
+// Sum over each row of 16 lanes by a shifted-add scan; the totals arrive in lanes 15, 31, 47 and 63.
+__device__ __forceinline__ double row_sum(double x) {
   x = dpp_add<0x111, 0xf>(x);  // row_shr:1
   x = dpp_add<0x112, 0xf>(x);  // row_shr:2
   x = dpp_add<0x114, 0xf>(x);  // row_shr:4
-  x = dpp_add<0x118, 0xf>(x);  // row_shr:8
+  return dpp_add<0x118, 0xf>(x);  // row_shr:8
+}
+
+// Sum over the 64 lanes of a wavefront in a fixed order; the total arrives in lane 63.  First the rows of 16
+// lanes, then lane 15 of rows 0 and 2 into rows 1 and 3, then lane 31 into rows 2 and 3.
+__device__ __forceinline__ double wave_sum(double x) {
+  x = row_sum(x);
   x = dpp_add<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
   x = dpp_add<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
   return x;
+}
+
+// A lane's value in every lane.
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                          __builtin_amdgcn_readlane(__double2loint(x), lane));
 }
 
 __device__ __forceinline__ Triple wg_reduce(Triple t) {

@@ -282,6 +282,53 @@ def test_combine_equals_split_sequence_bit_for_bit(gpu, dtype, big):
         plan2.destroy()
 
 
+def _held_counts(chunk, longest):
+    """Layers of which the longest touches `longest` chunks of the vectors: around the ends of chunks and of a lane's
+    vectors, empty ones, single elements, and enough long ones for the eight-chunk kernel to be taken."""
+    if longest == 1:  # one layer, which starts and ends within a chunk, and several in one chunk
+        return [3, 0, 255, 1, chunk // 2 - 300, 17]
+    if longest == 2:
+        return [chunk, 1, chunk - 1, chunk // 2 + 1, 0, 7, chunk + 5 - 8, 1000, 1]
+    if longest <= 4:
+        return [0, (longest - 1) * chunk + 1, 3 * (16 // 8), 1, (longest - 1) * chunk - 3, 2 * chunk, 5, 255, chunk]
+    return [(longest - 1) * chunk - (i * 37) % 911 if i % 40 else i % 7 for i in range(210)]
+
+
+@pytest.mark.parametrize("dtype", [F32, F64, F16])
+@pytest.mark.parametrize("longest", [1, 2, 3, 4, 6, 8])
+@pytest.mark.parametrize("shift", [0, 1])  # vectors on a 16-byte boundary and one element behind it
+def test_layers_that_fit_a_workgroup_equal_the_two_passes_bit_for_bit(gpu, dtype, longest, shift):
+    """combine() takes layers of few chunks in one launch; dot_norms() followed by scaled_add() never does."""
+    rng = np.random.default_rng(longest)
+    np_t, es = NP_OF[dtype], SIZE_OF[dtype]
+    counts = _held_counts(16384 // es, longest)
+    n = sum(counts)
+    a, b = _pair(rng, n, np_t)
+    if dtype != F16:
+        a[:2], b[:2] = [np.inf, np.nan], [-np.inf, 1.0]  # the first layer's sums are not finite
+    pad = np.zeros(8, np_t)
+    d_a1, d_a2 = (gpu.upload(np.concatenate([pad[:shift], a, pad])) for _ in range(2))
+    d_b = gpu.upload(np.concatenate([pad[:shift], b, pad]))
+    plan1, plan2 = gpu.H.AdasumPlan(counts, dtype), gpu.H.AdasumPlan(counts, dtype)
+    try:
+        at = shift * es
+        plan1.dot_norms(d_a1.data_ptr() + at, d_b.data_ptr() + at, gpu.stream)
+        plan1.scaled_add(d_a1.data_ptr() + at, d_b.data_ptr() + at, gpu.stream)
+        first = plan1.read(gpu.stream)
+        plan2.combine(d_a2.data_ptr() + at, d_b.data_ptr() + at, gpu.stream)
+        second = plan2.read(gpu.stream)
+        for x, y in zip(first, second):
+            assert np.array_equal(np.array(x).view(np.uint64), np.array(y).view(np.uint64))
+        raw = np.uint16 if np_t == np.float16 else np_t
+        g1, g2 = gpu.download(d_a1, raw), gpu.download(d_a2, raw)
+        assert np.array_equal(g1.view(np.uint8), g2.view(np.uint8))
+        assert not g2[shift + n:].any() and not g2[:shift].any(), "wrote outside the vector"
+        assert not np.array_equal(g2[shift:shift + n].view(np.uint8), _raw(a).view(np.uint8))
+    finally:
+        plan1.destroy()
+        plan2.destroy()
+
+
 def test_rejects_integer_dtypes(gpu):
     import horovod_amd
     with pytest.raises(horovod_amd.HvdHipError) as e:
