@@ -169,7 +169,8 @@ __global__ __launch_bounds__(kWG) void finalize_k(const Layer* __restrict__ laye
 // bit; the layer's first workgroup also stores the sums and coefficients for readers.
 template <typename T, bool FUSED, int ST>
 __global__ __launch_bounds__(kWG) void scaled_add_k(const Chunk* __restrict__ chunks, T* a,
-                                                    const T* __restrict__ b,
+                                                    const T* __restrict__ b, uint32_t turn,
+                                                    uint32_t workgroups, uint32_t nchunks,
                                                     const double* __restrict__ coeffs,
                                                     double ca_arg, double cb_arg,
                                                     const Layer* __restrict__ layers,
@@ -179,7 +180,9 @@ __global__ __launch_bounds__(kWG) void scaled_add_k(const Chunk* __restrict__ ch
                                                     uint32_t nlayers) {
   constexpr int VEC = 16 / (int)sizeof(T);
   typedef Arr<T, VEC> V;
-  const Chunk c = chunks[blockIdx.x];
+  const uint32_t turned = blockIdx.x + turn, at = turned < workgroups ? turned : turned - workgroups;
+  if (at >= nchunks) return;  // the grid is a multiple of eight, so that every chunk stays on its XCD
+  const Chunk c = chunks[at];
   const uint32_t n = c.n;
   gptr<T> pa = as_global(a + c.tensor);
   gptr<const T> pb = as_global(b + c.tensor);
@@ -518,13 +521,24 @@ int plan_dot_norms(hvdhip_adasum_plan* p, const void* a, const void* b, hipStrea
   return 0;
 }
 
+// The scaled add of long vectors begins with the last 24 MiB of each, which the first pass read last: part of them still
+// lies in the eight L2s (4 MB each), on the XCDs that ask again, and the rest of the way is the first pass's.  Cold, us:
+// 2 x 64 MiB 51.4 -> 51.0, 2 x 128 MiB 97.4 -> 96.1, 2 x 192 MiB 144.6 -> 142.9 (8 MiB: 98.0, 16 MiB 96.9, 32 MiB 96.0);
+// up to 2 x 48 MiB nothing or a little worse.  On other XCDs than the first pass's the data is as good as gone: 2 x 12
+// MiB, which the L2s hold whole, 9.8 us, and 16.4 with every chunk on a neighbour.
+constexpr uint32_t kTurnChunks = 1536, kTurnFrom = 4096;
+inline uint32_t add_turn(uint32_t nchunks) {
+  return nchunks >= kTurnFrom ? (nchunks - kTurnChunks) / kXcds * kXcds : 0;
+}
+
 template <typename T, bool FUSED>
 hipError_t launch_scaled_add(hvdhip_adasum_plan* p, void* a, const void* b, const double* coeffs,
                              double ca, double cb, hipStream_t s) {
   const DevTables& t = p->tables;
+  const uint32_t workgroups = (t.nchunks + kXcds - 1) / kXcds * kXcds;
   return with_store_policy(Stores::kAdasum, [&](auto st) {
-    return launch(scaled_add_k<T, FUSED, decltype(st)::value>, t.nchunks, s, t.chunks, static_cast<T*>(a),
-                  static_cast<const T*>(b), coeffs, ca, cb, p->layers, p->partials, p->normdots, p->coeffs,
+    return launch(scaled_add_k<T, FUSED, decltype(st)::value>, workgroups, s, t.chunks, static_cast<T*>(a),
+                  static_cast<const T*>(b), add_turn(t.nchunks), workgroups, t.nchunks, coeffs, ca, cb, p->layers, p->partials, p->normdots, p->coeffs,
                   std::sqrt(DBL_MIN), (uint32_t)p->nlayers);
   });
 }

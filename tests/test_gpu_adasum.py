@@ -329,6 +329,32 @@ def test_layers_that_fit_a_workgroup_equal_the_two_passes_bit_for_bit(gpu, dtype
         plan2.destroy()
 
 
+@pytest.mark.parametrize("cut", [4093, 4094, 4097, 4102])  # two chunks more in the table
+def test_scaled_add_takes_every_chunk_once_wherever_it_begins(gpu, cut):
+    """From 4,096 chunks on the scaled add begins in the middle of its table, whose length need not be a multiple of
+    eight.  With the device's own coefficients the result is two rounded products and their sum in double."""
+    import torch
+    chunk = 16384 // 4
+    counts = [5, chunk * (cut // 2) - 5, 0, chunk // 2, chunk * (cut - cut // 2) - chunk - 3]
+    n = sum(counts)
+    gen = torch.Generator(device="cuda").manual_seed(cut)
+    a, b = (torch.empty(n + 8, dtype=torch.float32, device="cuda").normal_(generator=gen) for _ in range(2))
+    before = a.clone()
+    torch.cuda.synchronize()
+    plan = gpu.H.AdasumPlan(counts, F32)
+    try:
+        plan.combine(a.data_ptr(), b.data_ptr(), gpu.stream)
+        _, co = plan.read(gpu.stream)
+        want, off = before.clone(), 0
+        for i, c in enumerate(counts):
+            part = slice(off, off + c)
+            want[part] = (before[part].double() * co[2 * i] + b[part].double() * co[2 * i + 1]).float()
+            off += c
+        assert torch.equal(a.view(torch.int32), want.view(torch.int32))
+    finally:
+        plan.destroy()
+
+
 def test_rejects_integer_dtypes(gpu):
     import horovod_amd
     with pytest.raises(horovod_amd.HvdHipError) as e:
