@@ -46,6 +46,7 @@ _PROTOTYPES = {
     "hvdhip_stream_forget": (c_int, [c_void_p]),
     "hvdhip_stream_synchronize": (c_int, [c_void_p]),
     "hvdhip_stream_wait_event": (c_int, [c_void_p, c_void_p]),
+    "hvdhip_stream_idle": (c_int, [c_void_p, POINTER(c_int)]),
     "hvdhip_event_acquire": (c_int, [c_void_p, _PV]),
     "hvdhip_event_record": (c_int, [c_void_p, c_void_p]),
     "hvdhip_event_query": (c_int, [c_void_p, POINTER(c_int)]),
@@ -139,6 +140,27 @@ def adapter_lib():
     cdll.hvd_adapter_fuse_keyed.argtypes = [POINTER(c_int64), POINTER(c_int), c_int, c_int64, c_int, POINTER(c_int)]
     _adapter = cdll
     return _adapter
+
+
+_front = None
+
+
+def front():
+    """lib/_front.so: the per-tensor part of horovod_amd.torch, an extension module over torch's own headers."""
+    global _front
+    if _front is not None:
+        return _front
+    import importlib.util
+    import torch  # noqa: F401  the module links torch's libraries
+    path = os.path.join(_HERE, "lib", "_front.so")
+    if not os.path.exists(path):
+        raise RuntimeError("%s is missing: build it with `make -C horovod_amd/csrc`; "
+                           "there is no fallback path" % path)
+    spec = importlib.util.spec_from_file_location("horovod_amd.torch._front", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    _front = module
+    return _front
 
 
 def check(code, what):

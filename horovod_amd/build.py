@@ -1,5 +1,5 @@
-"""Builds the in-tree native libraries with make (hipcc for gfx950, g++ for the adapter, gcc for the
-C99 example client)."""
+"""Builds the in-tree native libraries with make (hipcc for gfx950, g++ for the adapter and the front
+end's extension module, gcc for the C99 example client)."""
 import os
 import subprocess
 
@@ -17,6 +17,7 @@ def build(force=False, jobs=8):
 
 def ensure_built():
     """Builds the libraries only if one of them is missing; never replaces an existing build."""
-    need = [os.path.join(_HERE, "lib", n) for n in ("libhvdhip.so", "libhvdhip_tuning.so", "libhvdhip_adapter.so", "c_client", "cache_stress")]
+    need = [os.path.join(_HERE, "lib", n) for n in ("libhvdhip.so", "libhvdhip_tuning.so", "libhvdhip_adapter.so", "_front.so", "c_client",
+                                                  "cache_stress")]
     if not all(os.path.exists(p) for p in need):
         build()

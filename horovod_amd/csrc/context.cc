@@ -317,6 +317,24 @@ int hvdhip_stream_wait_event(void* stream, void* event) {
   return ok();
 }
 
+int hvdhip_stream_idle(void* stream, int* idle) {
+  if (!idle) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "idle is NULL");
+  *idle = 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  HVDHIP_CHECK(hipStreamIsCapturing(s, &capture));
+  if (capture != hipStreamCaptureStatusNone) return ok();  // a query would end the capture
+  const hipError_t before = hipPeekAtLastError();
+  const hipError_t e = hipStreamQuery(s);
+  if (e == hipErrorNotReady) {
+    if (before == hipSuccess) (void)hipGetLastError();  // not an error: leave none behind
+    return ok();
+  }
+  HVDHIP_CHECK(e);
+  *idle = 1;
+  return ok();
+}
+
 int hvdhip_event_acquire(void* stream, void** event) {
   if (!event) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "event is NULL");
   int dev = 0;

@@ -12,8 +12,8 @@ from ._lib import DTYPE, check, lib
 
 def _ptr_array(values):
     """A C array of addresses; through array.array, which converts a list several times faster
-    than filling a ctypes array element by element."""
-    raw = array.array("Q", values)
+    than filling a ctypes array element by element and is taken as it is where the caller has one."""
+    raw = values if isinstance(values, array.array) else array.array("Q", values)
     return (c_void_p * len(raw)).from_buffer(raw) if len(raw) else (c_void_p * 0)()
 
 
@@ -23,7 +23,7 @@ def _size_array(values):
 
 
 def _count_array(values):
-    raw = array.array("q", values)
+    raw = values if isinstance(values, array.array) else array.array("q", values)
     return (c_int64 * len(raw)).from_buffer(raw) if len(raw) else (c_int64 * 0)()
 
 

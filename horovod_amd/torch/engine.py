@@ -22,12 +22,12 @@ so too, a pass per level of the pairwise tree; only where a node has several ran
 a buffer per node first.
 """
 import ctypes
-from ctypes import c_int, c_int64, c_void_p
+from ctypes import c_int, c_void_p
 
 import torch
 
 from .. import host as H
-from .._lib import adapter_lib, check, dtype_size, lib
+from .._lib import adapter_lib, check, dtype_size, front, lib
 
 SUM = 1      # ReduceOp values, common/operations.h:35-40
 ADASUM = 2
@@ -45,47 +45,47 @@ def _current_stream():
     return torch._C._cuda_getCurrentStream(torch._C._cuda_getDevice())
 
 
+def _stream_of(producer):
+    stream_id, device_index, device_type = producer
+    return torch.cuda.Stream(stream_id=stream_id, device_index=device_index, device_type=device_type)
+
+
 class HorovodInternalError(RuntimeError):
     """An error of the op layer surfacing in the caller (horovod/common/exceptions.py:18-23)."""
 
 
-class Entry:
-    __slots__ = ("name", "tensor", "output", "count", "parts")
-
-    def __init__(self, name, tensor, output):
-        self.name, self.tensor, self.output, self.count = name, tensor, output, tensor.numel()
-        self.parts = None  # allgather: what every rank contributes, rank 0 first
-
-
-class Request:
-    __slots__ = ("kind", "entries", "op", "prescale", "postscale", "divisor", "tensor_dtype", "wire_dtype", "device",
-                 "producer", "markers", "submitted", "error", "grouped")
-
-    def __init__(self, entries, op, prescale, postscale, divisor, tensor_dtype, wire_dtype, device,
-                 kind="allreduce", grouped=False):
-        self.kind = kind
-        self.entries = entries
-        self.op, self.prescale, self.postscale, self.divisor = op, float(prescale), float(postscale), divisor
-        self.tensor_dtype, self.wire_dtype, self.device = tensor_dtype, wire_dtype, device
-        self.producer = None     # the framework stream that was current at enqueue (torch's identifiers)
-        self.markers = []        # one Marker per fused response that carries one of the entries
-        self.submitted = False
-        self.error = None
-        self.grouped = grouped
-
-    def key(self):
-        return (self.kind, self.op, self.device, self.tensor_dtype, self.wire_dtype, self.prescale, self.postscale)
+# The records that travel through a cycle, and the loops over tensors and ranks, are native (csrc/front/front.cc):
+#   Entry(name, tensor, output)        count = elements; parts = what every rank contributes to an allgather
+#   Request(entries, op, prescale, postscale, tensor_dtype, wire_dtype, device, kind, grouped)
+#       producer = the framework stream that was current at enqueue (torch's identifiers); markers = one Marker per
+#       fused response that carries one of the entries; submitted, error
+#   Marker(stream, event, refs, keepalive)   completion event of one fused response, shared by the requests it carried
+#       (ops/gpu_operations.cc:50-56 records one per response); done; keepalive = the other ranks' tensors until then
+_front = front()
+Entry, Request, Marker = _front.Entry, _front.Request, _front.Marker
 
 
-class Marker:
-    """Completion event of one fused response, shared by the requests it carried
-    (ops/gpu_operations.cc:50-56 records one per response)."""
-    __slots__ = ("stream", "event", "refs", "done", "keepalive")
+def _is_peer(t, tensor, count):
+    """Whether t can stand for another rank's `tensor`: for those that the native check leaves open."""
+    return (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == tensor.dtype and t.numel() == count
+            and t.is_contiguous())
 
-    def __init__(self, stream, event, refs, keepalive):
-        self.stream, self.event, self.refs = stream, event, refs
-        self.done = False
-        self.keepalive = keepalive  # the other ranks' tensors, until the response has completed
+
+def _peer_address(t, e):
+    if not _is_peer(t, e.tensor, e.count):
+        raise ValueError("peer_source must return a contiguous device tensor of the shape and dtype of %r" % e.name)
+    return t.data_ptr()
+
+
+def _is_part(t, e):
+    """Whether t can stand for another rank's rows of an allgather (first dimensions may differ)."""
+    return (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == e.tensor.dtype and t.dim() == e.tensor.dim()
+            and t.shape[1:] == e.tensor.shape[1:] and t.is_contiguous())
+
+
+# Cycles for which a framework stream that was found busy is waited for without another look.  A look costs 0.1 us at an
+# idle stream and saves the event and the wait, 15 us of host time; at a busy one it costs 6 us on top of them.
+_BUSY_CYCLES = 16
 
 
 class Engine:
@@ -104,6 +104,7 @@ class Engine:
         self.cycles = 0
         self.responses = 0       # fused responses executed so far
         self.ready = {}          # framework stream -> event recorded during the current cycle
+        self.busy = {}           # framework stream -> cycle up to which it is taken to be busy
 
     # ---- queueing -------------------------------------------------------
 
@@ -137,46 +138,26 @@ class Engine:
                 self.inflight.pop(e.name, None)
                 # common/controller.cc:575-579
                 raise HorovodInternalError("Rank zero tried to allgather a rank-zero tensor.")
-            parts = [e.tensor]
-            for rank in range(1, self.size):
-                t = e.tensor if self.peer_source is None else self.peer_source(rank, e.name, e.tensor)
-                if (not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != e.tensor.dtype
-                        or t.dim() != e.tensor.dim() or t.shape[1:] != e.tensor.shape[1:] or not t.is_contiguous()):
-                    self.inflight.pop(e.name, None)
-                    raise HorovodInternalError(
-                        "Mismatched allgather tensor shapes: ranks may differ in the first dimension only "
-                        "(tensor %r)." % e.name)
-                parts.append(t)
-            e.parts = parts
-            e.output.resize_((sum(t.shape[0] for t in parts),) + tuple(e.tensor.shape[1:]))
+            found = _front.parts(e, self.size, self.peer_source, _is_part)
+            if found is None:
+                self.inflight.pop(e.name, None)
+                raise HorovodInternalError(
+                    "Mismatched allgather tensor shapes: ranks may differ in the first dimension only "
+                    "(tensor %r)." % e.name)
+            e.parts, rows = found
+            e.output.resize_((rows,) + tuple(e.tensor.shape[1:]))
 
     def run_cycle(self):
         """Fuses and queues everything enqueued so far (one pass of RunLoopOnce,
         common/operations.cc:593-717, with every request already agreed upon)."""
-        pending, self.queue = self.queue, []
+        pending = list(self.queue)
+        self.queue.clear()
         if not pending:
             return
         self.cycles += 1
         self.ready = {}
-        flat, sizes, keys, classes = [], [], [], {}
-        for r in pending:
-            key = classes.setdefault(r.key(), len(classes))
-            gathers = r.kind == "allgather"
-            es = dtype_size(r.tensor_dtype if gathers else r.wire_dtype)
-            for e in r.entries:
-                nbytes = (e.output.numel() if gathers else e.count) * es
-                if self.batch_d2d_memcopies and not gathers:  # no padding on that path
-                    nbytes = (nbytes + 15) // 16 * 16
-                flat.append((r, e))
-                sizes.append(nbytes)
-                keys.append(key)
-        n = len(flat)
-        group_of = (c_int * n)()
-        ngroups = adapter_lib().hvd_adapter_fuse_keyed((c_int64 * n)(*sizes), (c_int * n)(*keys), n,
-                                                       self.fusion_threshold, 0, group_of)
-        groups = [[] for _ in range(ngroups)]
-        for i in range(n):
-            groups[group_of[i]].append(flat[i])
+        fuse = ctypes.cast(adapter_lib().hvd_adapter_fuse_keyed, c_void_p).value
+        groups = _front.plan(pending, self.batch_d2d_memcopies, self.fusion_threshold, fuse)
         for g in groups:
             try:
                 if g[0][0].kind == "allgather":
@@ -200,39 +181,18 @@ class Engine:
             self.buffers[(slot, what)] = t
         return t.data_ptr()
 
-    def _peers(self, group, addresses):
-        """The tensors that the other ranks pass for a group's entries; their addresses are appended rank by rank."""
-        source, dtype, peers = self.peer_source, group[0][1].tensor.dtype, []
-        for rank in range(1, self.size):
-            for _, e in group:
-                t = source(rank, e.name, e.tensor)
-                if (not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != dtype or t.numel() != e.count
-                        or not t.is_contiguous()):
-                    raise ValueError("peer_source must return a contiguous device tensor of the shape and dtype of %r"
-                                     % e.name)
-                peers.append(t)
-                addresses.append(t.data_ptr())
-        return peers
-
     # ---- one fused response --------------------------------------------
 
     def _execute(self, group):
         first = group[0][0]
-        counts = [e.count for _, e in group]
-        inputs = [e.tensor.data_ptr() for _, e in group]  # rank-major: inputs[rank * len(group) + entry]
-        peers = made = None
-        if self.peer_source is None:
-            inputs *= self.size
-        elif self.size > 1:
-            # the other ranks' tensors (framework stream); this response's stream waits for them, which
-            # covers what that stream did before
-            peers = self._peers(group, inputs)
-            made = _current_stream()
-            peers.append(self._record(made))
+        # rank-major: inputs[rank * len(group) + entry]
+        inputs, outputs, counts, peers = _front.addresses(group, self.size, self.peer_source, _peer_address)
+        # the other ranks' tensors (framework stream): this response's stream waits for them, which covers what
+        # that stream did before
+        made = _current_stream() if peers else None
         slot, s, requests = self._begin(group, made)
         if made is not None:
-            self._wait_for(s, peers[-1])
-        outputs = [e.output.data_ptr() for _, e in group]
+            peers.append(self._wait_for(s, made))
         event = self._acquire(s)
         try:
             plain = first.wire_dtype == first.tensor_dtype
@@ -326,37 +286,42 @@ class Engine:
             H.ranks_sum([out], [buf + o], [n], 1, wire, wire, tdt, 1.0, req.postscale, s)
         check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
 
-    @staticmethod
-    def _record(producer):
-        ev = torch.cuda.Event()
-        stream_id, device_index, device_type = producer
-        ev.record(torch.cuda.Stream(stream_id=stream_id, device_index=device_index, device_type=device_type))
-        return ev
+    def _wait_for(self, s, producer, event=None):
+        """Makes the stream wait for what the framework's stream `producer` holds now, if there is anything, or for
+        `event`, which was recorded there.  Returns the event that it waits for."""
+        if event is None:
+            if self.busy.get(producer, 0) < self.cycles:
+                if producer == _current_stream():
+                    handle = torch._C._cuda_getCurrentRawStream(producer[1])
+                else:
+                    handle = _stream_of(producer).cuda_stream
+                idle = c_int()
+                check(lib().hvdhip_stream_idle(handle, ctypes.byref(idle)), "hvdhip_stream_idle")
+                if idle.value:
+                    return None
+                if len(self.busy) > 64:
+                    self.busy.clear()
+                self.busy[producer] = self.cycles + _BUSY_CYCLES
+            event = torch.cuda.Event()
+            event.record(_stream_of(producer))
+        check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(event.cuda_event)), "hvdhip_stream_wait_event")
+        return event
 
-    @staticmethod
-    def _wait_for(s, ev):
-        check(lib().hvdhip_stream_wait_event(s.handle, c_void_p(ev.cuda_event)), "hvdhip_stream_wait_event")
-
-    def _begin(self, group, covered=None):
-        """Picks the stream slot of a fused response and makes it wait for the framework's streams, all but
-        the one that the caller makes it wait for."""
+    def _begin(self, group, made=None):
+        """Picks the stream slot of a fused response and makes it wait for the framework's streams that its requests were
+        enqueued on, all but the one that the caller makes it wait for (`made`)."""
         self.responses += 1
         slot, self.slot = self.slot, (self.slot + 1) % len(self.streams)
         s = self.streams[slot]
-        requests = list(dict.fromkeys(r for r, _ in group))
-        for producer in {r.producer for r in requests}:
-            if producer == covered:
-                continue
-            if producer not in self.ready:
-                self.ready[producer] = self._record(producer)
-            self._wait_for(s, self.ready[producer])
+        requests, producers = _front.requests(group)
+        for producer in producers:
+            if producer != made:
+                self.ready[producer] = self._wait_for(s, producer, self.ready.get(producer))
         return slot, s, requests
 
     @staticmethod
     def _finish(s, requests, event, keepalive=None):
-        marker = Marker(s, event, len(requests), keepalive)
-        for r in requests:
-            r.markers.append(marker)
+        _front.attach(requests, Marker(s, event, len(requests), keepalive))
 
     def _execute_allgather(self, group):
         """The fusion-buffer side of a fused allgather (AllgatherOp::MemcpyInFusionBuffer /
@@ -366,16 +331,7 @@ class Engine:
         slot, s, requests = self._begin(group)
         dtype = group[0][0].tensor_dtype
         es = dtype_size(dtype)
-        sources, places, counts = [], [], []
-        for _, e in group:
-            at = e.output.data_ptr()
-            for part in e.parts:
-                n = part.numel()
-                if n:
-                    sources.append(part.data_ptr())
-                    places.append(at)
-                    counts.append(n)
-                    at += n * es
+        places, sources, counts = _front.places(group, es)
         if any(p % es for p in sources):  # foreign memory that no element type fits: bytes
             counts, dtype = [n * es for n in counts], TORCH_TO_HVD[torch.uint8]
         event = self._acquire(s)
@@ -421,6 +377,10 @@ class Engine:
 
     # ---- completion -----------------------------------------------------
 
+    @staticmethod
+    def _release(marker):
+        check(lib().hvdhip_event_release(marker.stream.handle, marker.event), "hvdhip_event_release")
+
     def poll(self, request):
         if not request.submitted:
             self.run_cycle()
@@ -445,7 +405,7 @@ class Engine:
             for m in request.markers:
                 m.refs -= 1
                 if m.refs == 0:  # the last request of the response hands the event back to its pool
-                    check(lib().hvdhip_event_release(m.stream.handle, m.event), "hvdhip_event_release")
+                    self._release(m)
             request.markers = []
             for e in request.entries:
                 self.inflight.pop(e.name, None)

@@ -23,7 +23,7 @@ import warnings
 import torch
 
 from .compression import Compression
-from .engine import ADASUM, SUM, Engine, Entry, HorovodInternalError, Request, TORCH_TO_HVD
+from .engine import ADASUM, SUM, Engine, Entry, HorovodInternalError, Request, TORCH_TO_HVD, _front
 
 # ReduceOp values handed out by horovod_reduce_op_*(), common/operations.h:35-40
 Average = 0
@@ -31,6 +31,7 @@ Sum = 1
 Adasum = 2
 
 _engine = None
+_state_of_front = None  # what the native half of submission and completion works on, while there is an engine
 _handle_map = {}
 _next_handle = [0]
 _noname = [0]
@@ -44,7 +45,7 @@ def init(size=1, local_size=1, peer_source=None, fusion_threshold=None, num_stre
     HOROVOD_FUSION_THRESHOLD (bytes, 64 MiB) and HOROVOD_NUM_NCCL_STREAMS, the knobs of
     common/operations.cc:419-441,475-481; without the variable there are two stream slots (the
     reference has one): consecutive fused responses then overlap each other's start-up and drain."""
-    global _engine
+    global _engine, _state_of_front
     if _engine is not None:
         return
     if not torch.cuda.is_available():
@@ -56,13 +57,15 @@ def init(size=1, local_size=1, peer_source=None, fusion_threshold=None, num_stre
         num_streams = int(os.environ.get("HOROVOD_NUM_NCCL_STREAMS", 2))
     batch = os.environ.get("HOROVOD_BATCH_D2D_MEMCOPIES", "1") != "0"
     _engine = Engine(size, local_size, peer_source, fusion_threshold, num_streams, batch)
+    _state_of_front = _front.State(size, local_size, _engine.inflight, _engine.queue, _handle_map, _next_handle, _noname,
+                                   _engine._release)
 
 
 def shutdown():
-    global _engine
+    global _engine, _state_of_front
     if _engine is not None:
         _engine.shutdown()
-        _engine = None
+        _engine = _state_of_front = None
     _handle_map.clear()
 
 
@@ -187,7 +190,7 @@ def _submit(tensors, outputs, names, op, prescale_factor, postscale_factor, wire
     red, pre, post = _factors(op, prescale_factor, postscale_factor, torch.float16 if wire_dtype is not None else dtype)
     tdt = TORCH_TO_HVD[dtype]
     wire = tdt if wire_dtype is None else TORCH_TO_HVD[wire_dtype]
-    req = Request([Entry(n, t, o) for n, t, o in zip(names, tensors, outputs)], red, pre, post, 1, tdt, wire,
+    req = Request([Entry(n, t, o) for n, t, o in zip(names, tensors, outputs)], red, pre, post, tdt, wire,
                   device.index, grouped=grouped)
     try:
         eng.enqueue(req)
@@ -199,14 +202,22 @@ def _submit(tensors, outputs, names, op, prescale_factor, postscale_factor, wire
 
 
 def _allreduce_async(tensor, output, name, op, prescale_factor, postscale_factor, wire_dtype=None):
+    if _state_of_front is not None:
+        handle = _state_of_front.submit(tensor, output, name, op, prescale_factor, postscale_factor, wire_dtype)
+        if handle is not None:
+            return handle
     return _submit([tensor], [output], [_name(name, 'allreduce')], op, prescale_factor, postscale_factor, wire_dtype)
 
 
 def _grouped_allreduce_async(tensors, outputs, name, op, prescale_factor, postscale_factor, wire_dtype=None):
     base = _name(name, 'grouped_allreduce')
-    n = len(tensors)
+    tensors, outputs, n = list(tensors), list(outputs), len(tensors)
+    if _state_of_front is not None and type(base) is str:
+        handle = _state_of_front.submit_group(tensors, outputs, base, op, prescale_factor, postscale_factor, wire_dtype)
+        if handle is not None:
+            return handle
     names = ['%s_%dof%d' % (base, i + 1, n) for i in range(n)]  # horovod/torch/mpi_ops_v2.cc:207
-    return _submit(list(tensors), list(outputs), names, op, prescale_factor, postscale_factor, wire_dtype,
+    return _submit(tensors, outputs, names, op, prescale_factor, postscale_factor, wire_dtype,
                    grouped=True)
 
 
@@ -310,7 +321,7 @@ def allgather_async(tensor, name=None):
     eng = _state()
     _check(tensor)
     output = tensor.new()
-    req = Request([Entry(_name(name, 'allgather'), tensor, output)], SUM, 1.0, 1.0, 1, TORCH_TO_HVD[tensor.dtype],
+    req = Request([Entry(_name(name, 'allgather'), tensor, output)], SUM, 1.0, 1.0, TORCH_TO_HVD[tensor.dtype],
                   TORCH_TO_HVD[tensor.dtype], tensor.device.index, kind="allgather")
     try:
         eng.enqueue(req)
@@ -440,6 +451,10 @@ def poll(handle):
 
 def synchronize(handle):
     """Waits for the operation and returns its output (a list for grouped operations)."""
+    if _state_of_front is not None:
+        output = _state_of_front.finish(handle)
+        if output is not _front.PENDING:
+            return output
     if handle not in _handle_map:
         return None
     req = _handle_map.pop(handle)

@@ -137,6 +137,10 @@ int hvdhip_stream_synchronize(void* stream);
 /* The framework's ready event is waited for on the Horovod stream, without a
  * host synchronisation: ops/nccl_operations.cc:140-154. */
 int hvdhip_stream_wait_event(void* stream, void* event);
+/* *idle = 1 if everything that was queued on the stream (any stream of the caller's, NULL for the null
+ * stream) has completed, so that nothing need wait for it; 0 if not, or while the stream is being captured.
+ * No counterpart in the reference, which records a ready event on a stream that is idle as well. */
+int hvdhip_stream_idle(void* stream, int* idle);
 
 /* GetGpuEvent, ops/cuda_operations.cc:28-63: takes an event from the pool
  * kept per (current device, stream); the pool is filled with 128

@@ -1,0 +1,163 @@
+"""The native half of the torch front end on the GPU: tensors and peers that are not the plain case take the Python path
+and give the same, work of busy streams is waited for whether or not the engine looks, and nothing is left behind."""
+import ctypes
+import gc
+
+import pytest
+import torch
+
+import horovod_amd
+from horovod_amd._lib import check, front
+
+pytestmark = pytest.mark.gpu
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+@pytest.fixture
+def hvd():
+    import horovod_amd.torch as hvd
+    hvd.shutdown()
+    yield hvd
+    hvd.shutdown()
+
+
+KINDS = {"plain": lambda t: t, "parameter": lambda t: torch.nn.Parameter(t, requires_grad=False),
+         "subclass": lambda t: t.as_subclass(Sub)}
+
+
+@pytest.mark.parametrize("peer", KINDS)
+@pytest.mark.parametrize("own", KINDS)
+def test_every_kind_of_tensor_is_summed(hvd, own, peer):
+    hvd.init(size=3, peer_source=lambda rank, name, t: KINDS[peer](torch.full_like(t.data, float(rank)).as_subclass(torch.Tensor)))
+    t = KINDS[own](torch.arange(1000, dtype=torch.float32, device="cuda"))
+    out = hvd.synchronize(hvd.allreduce_async(t, op=hvd.Sum))
+    assert torch.equal(out.as_subclass(torch.Tensor), t.as_subclass(torch.Tensor) + 3)
+    rows = hvd.synchronize(hvd.allgather_async(t.reshape(10, 100), name="rows"))
+    assert rows.shape == (30, 100) and torch.equal(rows.as_subclass(torch.Tensor)[10:], torch.cat(
+        [torch.full((10, 100), float(r), device="cuda") for r in (1, 2)]))
+
+
+@pytest.mark.parametrize("odd", [None, 0, 1, 2])
+def test_a_group_is_summed_whatever_its_tensors_are(hvd, odd):
+    """One that is no plain tensor takes the whole group through Python; the names and results are the same."""
+    names = []
+
+    def source(rank, name, t):
+        names.append(name)
+        return torch.full_like(t, float(rank))
+
+    hvd.init(size=2, peer_source=source)
+    tensors = [torch.arange(n, dtype=torch.float32, device="cuda") for n in (5, 1000, 1)]
+    if odd is not None:
+        tensors[odd] = tensors[odd].as_subclass(Sub)
+    for out, t in zip(hvd.synchronize(hvd.grouped_allreduce_async(tensors, name="g", op=hvd.Sum)), tensors):
+        assert torch.equal(out.as_subclass(torch.Tensor), t.as_subclass(torch.Tensor) + 1)
+    assert names == ["grouped_allreduce.g_%dof3" % i for i in (1, 2, 3)]
+    first = hvd.grouped_allreduce_async(tensors, name="g")
+    with pytest.raises(hvd.HorovodInternalError, match="same name"):
+        hvd.grouped_allreduce_async(tensors, name="g")
+    hvd.synchronize(first)
+    with pytest.raises(ValueError, match="share dtype and device"):
+        hvd.grouped_allreduce_async([tensors[0], tensors[1].double()])
+
+
+@pytest.mark.parametrize("wrong", [lambda t: t.double(), lambda t: t[:-1], lambda t: t.cpu(), lambda t: None,
+                                   lambda t: torch.stack([t, t], 1)[:, 0], lambda t: t.double().as_subclass(Sub)])
+def test_a_peer_that_does_not_fit_is_an_error_of_its_response(hvd, wrong):
+    hvd.init(size=2, peer_source=lambda rank, name, t: wrong(t) if name.endswith("bad") else t)
+    t = torch.ones(100, device="cuda")
+    handle = hvd.allreduce_async(t, name="bad")
+    with pytest.raises(hvd.HorovodInternalError, match="peer_source must return"):
+        hvd.synchronize(handle)
+    assert torch.equal(hvd.allreduce(t, name="good"), t)
+
+
+@pytest.mark.parametrize("peers", [True, False])
+@pytest.mark.parametrize("stream", ["default", "side", "another than at the cycle"])
+def test_work_of_a_busy_stream_is_waited_for(hvd, stream, peers):
+    """The tensor (and in turn the peer's) is written behind a long wait on the device: in cycles in which the engine looks
+    at the stream and finds it busy, in those after, in which it does not look, and among idle ones."""
+    y = torch.zeros(1 << 16, device="cuda")
+    hvd.init(size=2, peer_source=(lambda rank, name, t: y) if peers else None)
+    other = torch.cuda.current_stream() if stream == "default" else torch.cuda.Stream()
+    x = torch.zeros(1 << 16, device="cuda")
+    torch.cuda.synchronize()
+    for i in range(40):
+        with torch.cuda.stream(other):
+            if i % 20 < 4 or i % 3 == 0:
+                torch.cuda._sleep(2000000)
+            x.fill_(i)
+            y.fill_(2 * i if peers else i)
+            handle = hvd.allreduce_async(x, op=hvd.Sum)
+            if stream != "another than at the cycle":
+                out = hvd.synchronize(handle)
+        if stream == "another than at the cycle":
+            if peers:  # they are made on the stream of the cycle, which here waits for the other
+                torch.cuda.current_stream().wait_stream(other)
+            out = hvd.synchronize(handle)
+        assert float(out[0]) == float(out[-1]) == (3 * i if peers else 2 * i), i
+        other.synchronize()
+
+
+def test_idle_is_said_of_idle_streams_only():
+    L = horovod_amd.lib()
+
+    def idle(s):
+        out = ctypes.c_int(-1)
+        check(L.hvdhip_stream_idle(s.cuda_stream, ctypes.byref(out)), "hvdhip_stream_idle")
+        return out.value
+
+    for s in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        torch.cuda.synchronize()
+        assert idle(s) == 1
+        with torch.cuda.stream(s):
+            torch.cuda._sleep(20000000)
+        assert idle(s) == 0
+        assert float((torch.ones(8, device="cuda") + 1)[0]) == 2.0  # no stale error is left for the next launch
+        s.synchronize()
+        assert idle(s) == 1
+    assert L.hvdhip_stream_idle(None, None) == -1
+    x, g, s = torch.zeros(64, device="cuda"), torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        x.add_(1)
+        assert idle(s) == 0  # and the capture goes on
+        x.add_(1)
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert float(x[0]) == 2 * (i + 1)
+
+
+def test_the_stream_of_a_request_is_the_current_one(hvd, gpu):
+    from horovod_amd.torch import engine, mpi_ops
+    hvd.init(size=2)
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.ExternalStream(gpu.stream.handle.value)):
+        with torch.cuda.stream(stream):
+            assert mpi_ops._state_of_front.producer() == tuple(engine._current_stream())
+
+
+def test_nothing_is_left_of_finished_requests(hvd):
+    t = [torch.ones(1000, device="cuda") for _ in range(20)]
+    hvd.init(size=4, peer_source=lambda rank, name, x: torch.ones_like(x))
+
+    def step(i):
+        handles = [hvd.allreduce_async(x, name="%d" % k if i % 2 else None) for k, x in enumerate(t)]
+        for h in handles:
+            hvd.synchronize(h)
+
+    def counts():
+        gc.collect()
+        torch.cuda.synchronize()
+        kinds = (front().Request, front().Entry, front().Marker)
+        return torch.cuda.memory_allocated(), sum(type(o) in kinds for o in gc.get_objects())
+
+    for i in range(4):
+        step(i)
+    before = counts()
+    for i in range(50):
+        step(i)
+    assert counts() == before and before[1] == 0
