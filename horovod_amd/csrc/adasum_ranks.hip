@@ -11,6 +11,8 @@
 //            level and leaves the sums of the two                            (R + R/2, R/2 + R/4 ...)
 //   last_k   reads the last two, combines them, stores the result into the outputs            (2 + 1)
 //
+// A response of rows that fit the registers of a workgroup goes through the tree in one launch (tree_held_k).
+//
 // 29 vectors for eight ranks, in 4 launches instead of 23, and a launch of coeffs_k between two passes where a tensor has
 // more than 512 chunks.  Every pass is bound by memory: a BERT-large layer (16 tensors, 50 MB, four of them of 1,024
 // chunks) of eight ranks takes 230 us in 7 launches: dots_k 62, level_k 86 and 44, last_k 23.5 us, 6.8 TB/s over the 1.46
@@ -319,6 +321,128 @@ __global__ __launch_bounds__(kWG) void coeffs_k(const double* __restrict__ sums,
   }
 }
 
+// ---- rows that fit a workgroup -----------------------------------------------------------------
+
+// A chunk of every rank in the registers of 256 lanes.  The vectors are pinned where they are used: the compiler would
+// keep widened halves from the sums to the scaled add, in four times the registers.
+template <typename W, int WORLD>
+struct HeldRanks {
+  static constexpr int VEC = 16 / (int)sizeof(W), kVecs = (int)(kChunkBytes / 16 / kWG);
+  typedef RawSel<16>::type R;
+  uint32_t m, nv, lane;
+  R x[WORLD][kVecs];
+  W t[WORLD];  // the element behind the last whole vector
+
+  static __device__ __forceinline__ Arr<W, VEC> pinned(R& r) {
+    asm("" : "+v"(r));
+    return __builtin_bit_cast(Arr<W, VEC>, r);
+  }
+  __device__ __forceinline__ bool has_tail() const { return nv * VEC + lane < m; }
+
+  __device__ __forceinline__ void load(const uint64_t* ranks, uint64_t start, uint32_t elements, uint32_t lane_,
+                                       typename Factor<W>::type fin, bool scale_in) {
+    m = elements;
+    nv = m / VEC;
+    lane = lane_;
+#pragma unroll
+    for (int r = 0; r < WORLD; ++r) {
+      const gptr<const W> p = as_global<const W>(ranks[r]) + start;
+#pragma unroll
+      for (int u = 0; u < kVecs; ++u)
+        if (lane + u * kWG < nv) x[r][u] = __builtin_bit_cast(R, ldv<W, VEC>(p + (size_t)(lane + u * kWG) * VEC));
+      if (has_tail()) t[r] = p[nv * VEC + lane];
+    }
+    if (!scale_in) return;
+#pragma unroll
+    for (int r = 0; r < WORLD; ++r) {
+#pragma unroll
+      for (int u = 0; u < kVecs; ++u)
+        if (lane + u * kWG < nv) x[r][u] = __builtin_bit_cast(R, to_wire<W, W, VEC>(pinned(x[r][u]), fin, true));
+      if (has_tail()) t[r] = to_wire<W, W, 1>(Arr<W, 1>{t[r]}, fin, true).v[0];
+    }
+  }
+};
+
+// The levels of the tree from PAIRS pairs on, the vectors in the first 2 * PAIRS places; the result ends in the first.
+template <int PAIRS, typename W, int WORLD, int G>
+__device__ __forceinline__ void held_levels(HeldRanks<W, WORLD>& h, uint32_t group, double guard,
+                                            double (*red)[WORLD / 2][3][kWG / 64]) {
+  constexpr int VEC = HeldRanks<W, WORLD>::VEC, kVecs = HeldRanks<W, WORLD>::kVecs;
+  const uint32_t l64 = threadIdx.x & 63;
+#pragma unroll
+  for (int p = 0; p < PAIRS; ++p) {
+    Sums sums;
+#pragma unroll
+    for (int u = 0; u < kVecs; ++u)
+      if (h.lane + u * kWG < h.nv) sums.add(h.pinned(h.x[2 * p][u]), h.pinned(h.x[2 * p + 1][u]));
+    if (h.has_tail()) sums.add(Arr<W, 1>{h.t[2 * p]}, Arr<W, 1>{h.t[2 * p + 1]});
+    const double d = wave_sum(sums.d[0] + sums.d[1]), a = wave_sum(sums.a[0] + sums.a[1]),
+                 b = wave_sum(sums.b[0] + sums.b[1]);
+    if (l64 == 63) {
+      red[group][p][0][h.lane / 64] = d;
+      red[group][p][1][h.lane / 64] = a;
+      red[group][p][2][h.lane / 64] = b;
+    }
+  }
+  __syncthreads();
+  // Every wavefront adds the chunks' sums for itself, a lane per coefficient, with the bits of wg_reduce and
+  // short_row_sum.
+  const uint32_t k = l64 < 2 * PAIRS ? l64 : 0;
+  double d = 0., n = 0., c, other;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    double rd = 0., rn = 0.;
+#pragma unroll
+    for (int w = 0; w < kWG / 64; ++w) {
+      rd += red[g][k / 2][0][w];
+      rn += red[g][k / 2][1 + k % 2][w];
+    }
+    d += rd;
+    n += rn;
+  }
+  layer_coeffs(Triple{d, n, n}, guard, &c, &other);
+#pragma unroll
+  for (int p = 0; p < PAIRS; ++p) {
+    const double ca = lane_value(c, 2 * p), cb = lane_value(c, 2 * p + 1);
+#pragma unroll
+    for (int u = 0; u < kVecs; ++u)
+      if (h.lane + u * kWG < h.nv)
+        h.x[p][u] = __builtin_bit_cast(typename HeldRanks<W, WORLD>::R,
+                                       combined<W, VEC>(ca, h.pinned(h.x[2 * p][u]), cb, h.pinned(h.x[2 * p + 1][u])));
+    if (h.has_tail()) h.t[p] = combined<W, 1>(ca, Arr<W, 1>{h.t[2 * p]}, cb, Arr<W, 1>{h.t[2 * p + 1]}).v[0];
+  }
+  if constexpr (PAIRS > 1) held_levels<PAIRS / 2, W, WORLD, G>(h, group, guard, red + G);
+}
+
+// The whole tree of rows of at most G chunks, a workgroup each: G groups of 256 lanes have a chunk of every rank.  Row:
+// {elements, output, rank 0, 1 ...}.  The operations and their order are those of the launches it stands for, four of
+// them for eight ranks, each of which costs the stream 4 to 5 us however little it does.  Bound by the chain of one
+// workgroup: a level's sums, two trips through LDS and a divide, 1 us, and what a compute unit takes to load the ranks.
+// fp32, us: 8 ranks of 10 rows of 1,000 elements 15.7 -> 6.6, of 44 rows of one chunk 19.6 -> 9.7, of two 20.2 -> 13.4,
+// 2 ranks of 44 rows of two chunks 7.8 -> 4.4.  The lines: 8 ranks of two chunks are 182 registers at 512 lanes, and one
+// row of them takes as long in fp16 (16.7) as level by level; with a narrower type on the wire the levels' lanes have
+// other elements than the ranks', and a row's bits would depend on whether a longer row is beside it.
+template <typename W, int WORLD, int G>
+__global__ __launch_bounds__(G * kWG) void tree_held_k(Level l, Rows rows) {
+  constexpr int VEC = HeldRanks<W, WORLD>::VEC, kVecs = HeldRanks<W, WORLD>::kVecs;
+  const uint64_t* q = rows.q + blockIdx.x * l.words;
+  const typename Factor<W>::type fin = (typename Factor<W>::type)l.pre, fout = (typename Factor<W>::type)l.post;
+  const uint32_t group = threadIdx.x / kWG, count = (uint32_t)q[0], start = group * kChunk<W>;
+  const uint32_t left = start < count ? count - start : 0;
+  HeldRanks<W, WORLD> h;
+  h.load(q + 2, start, left < kChunk<W> ? left : kChunk<W>, threadIdx.x % kWG, fin, l.flags & kScaleIn);
+  __shared__ double red[(WORLD == 8 ? 3 : WORLD == 4 ? 2 : 1) * G][WORLD / 2][3][kWG / 64];
+  held_levels<WORLD / 2, W, WORLD, G>(h, group, l.guard, red);
+  const bool scale_out = l.flags & kScaleOut;
+  const gptr<W> to = as_global<W>(q[1]) + start;
+  const Window out = store_window<kStoreNT>(to, h.m * (uint32_t)sizeof(W));
+#pragma unroll
+  for (int u = 0; u < kVecs; ++u)
+    if (h.lane + u * kWG < h.nv)
+      stw<kStoreNT, W, VEC>(out, (h.lane + u * kWG) * 16u, from_wire<W, W, VEC>(h.pinned(h.x[0][u]), fout, scale_out));
+  if (h.has_tail()) to[h.nv * VEC + h.lane] = from_wire<W, W, 1>(Arr<W, 1>{h.t[0]}, fout, scale_out).v[0];
+}
+
 // ---- host side ---------------------------------------------------------------------------------
 
 uint64_t up256(uint64_t bytes) { return (bytes + 255) / 256 * 256; }
@@ -401,6 +525,17 @@ class Tree {
     l_.guard = std::sqrt(DBL_MIN);
     const uint32_t world = c_.world, at_once = std::min(world, kRanksAtOnce);
     double* sums[2] = {reinterpret_cast<double*>(ws_ + g_.sums_at[0]), reinterpret_cast<double*>(ws_ + g_.sums_at[1])};
+    if constexpr (std::is_same<S, W>::value && std::is_same<W, D>::value) {
+      if (g_.max_row_chunks <= 2 && world <= kRanksAtOnce) {
+        fill(0, world, true);
+        const bool one = g_.max_row_chunks == 1;
+        const hipError_t status = world == 2   ? (one ? held<2, 1>(completion) : held<2, 2>(completion))
+                                  : world == 4 ? (one ? held<4, 1>(completion) : held<4, 2>(completion))
+                                               : (one ? held<8, 1>(completion) : held<8, 2>(completion));
+        HVDHIP_CHECK_LAUNCH("tree_held_k", status);
+        return 0;
+      }
+    }
     // the ranks' sums, pairwise
     l_.out_sums = sums[0];
     for (uint32_t r = 0; r < world; r += at_once) {
@@ -441,6 +576,11 @@ class Tree {
     fill(0, 0, true);
     HVDHIP_CHECK_LAUNCH("last_k", launch_with(completion, last_k<W, W, D, false>, dim3(columns()), c_.stream, l_, rows_));
     return 0;
+  }
+
+  template <int WORLD, int G>
+  hipError_t held(hipEvent_t completion) const {
+    return launch_shaped(completion, tree_held_k<W, WORLD, G>, dim3(g_.nrows), G * kWG, c_.stream, l_, rows_);
   }
 
   // Workgroups along a launch's chunks: a multiple of the XCDs, so that a chunk is on the same one for every pair and in

@@ -98,6 +98,54 @@ def test_adasum_ranks_does_not_depend_on_the_other_tensors(gpu, world):
         assert torch.equal(combine([i])[0].view(torch.int64), together[i].view(torch.int64)), counts[i]
 
 
+@pytest.mark.parametrize("dtype", NP)
+@pytest.mark.parametrize("world", [2, 4, 8])
+@pytest.mark.parametrize("chunks", [1, 2])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_short_rows_give_the_same_bits_in_one_launch(gpu, dtype, world, chunks, scaled):
+    """Rows of up to two chunks go through the tree in one launch when all of a response's are so short; beside a row of
+    three chunks they go level by level.  Rows at the ends of vectors and chunks, one element into their allocations;
+    more rows than a launch carries; sums that are not finite; ranks that cancel."""
+    es = np.dtype(NP[dtype]).itemsize
+    chunk, code = 16384 // es, DTYPE[dtype]
+    counts = [1, 0, 16 // es - 1, 255 * 16 // es, 3 * 4096 // es + 5, chunk - 1, chunk, 7]
+    if chunks == 2:
+        counts += [chunk + 1, 2 * chunk - 1, 2 * chunk, chunk + 16 // es]
+    counts += [33 + i for i in range(44)]  # more than a launch carries; the long row below comes first of all
+    gen = torch.Generator(device="cuda").manual_seed(world)
+    kind = getattr(torch, dtype)
+
+    def draw(n):
+        return torch.empty(n + 1, dtype=kind, device="cuda").normal_(0.0, 0.1, generator=gen)
+
+    long_row = 2 * chunk + 1
+    base = [draw(n) for n in counts]
+    ranks = [[b * 0.5 + draw(n) for b, n in zip(base, counts)] for _ in range(world)]
+    longs = [draw(long_row) for _ in range(world)]
+    ranks[1][7][:] = -ranks[0][7]                     # a pair that cancels
+    ranks[0][5][3], ranks[1][6][2] = float("nan"), float("inf")
+    pre, post = (0.3, 1.7) if scaled else (1.0, 1.0)
+
+    def run(beside_a_long_row, in_place):
+        sizes = [long_row] * beside_a_long_row + counts
+        ins = [[t.clone() for t in [row] * beside_a_long_row + r] for row, r in zip(longs, ranks)]
+        outs = ins[0] if in_place else [torch.zeros_like(t) for t in ins[0]]
+        need = H.adasum_ranks_workspace(sizes, world, code)
+        work = torch.empty(max(need, 256), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        assert H.adasum_ranks([t.data_ptr() + es for t in outs], [t.data_ptr() + es for r in ins for t in r], sizes, world,
+                              code, code, code, pre, post, work.data_ptr(), need, gpu.stream)
+        gpu.stream.synchronize()
+        return outs[beside_a_long_row:]
+
+    alone, in_place, general = run(False, False), run(False, True), run(True, False)
+    for i, n in enumerate(counts):
+        want = general[i].view(torch.uint8)
+        assert torch.equal(alone[i].view(torch.uint8), want), (i, n)
+        assert torch.equal(in_place[i][1:].view(torch.uint8), want[es:]), (i, n)
+        assert torch.equal(in_place[i][:1].view(torch.uint8), ranks[0][i][:1].view(torch.uint8)), (i, n)
+
+
 def test_adasum_ranks_refuses(gpu):
     t = torch.zeros(8192, dtype=torch.float32, device="cuda")
     work = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
