@@ -161,3 +161,16 @@ def test_nothing_is_left_of_finished_requests(hvd):
     for i in range(50):
         step(i)
     assert counts() == before and before[1] == 0
+
+
+def test_a_large_response_is_followed_on_its_own_stream(hvd, monkeypatch):
+    from horovod_amd.torch import engine, mpi_ops
+    hvd.init(size=2, num_streams=2)
+    monkeypatch.setattr(engine, "_BYTES_OF_ITS_OWN", 2 * 4 * 1000)
+    slots = []
+    for n in (999, 999, 1000, 4000, 1, 1000):
+        t = torch.full((n,), 1.5, device="cuda")
+        handle = hvd.allreduce_async(t, op=hvd.Sum)
+        slots.append(mpi_ops._engine.slot)
+        assert torch.equal(hvd.synchronize(handle), 2 * t)
+    assert slots == [0, 1, 0, 0, 0, 1]
