@@ -6,12 +6,12 @@
 // summed into the first, which is unpacked -- moves every byte three times (2 per packing rank,
 // world + 1 for the sum, 2 for the unpack: 27 passes over the tensors for 8 ranks where 9 do).
 // It is bound by memory in both forms: ResNet-50's gradients (102 MB) of 8 ranks took 222 us of
-// kernels and take 152 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 1.95 ms (8 read
+// kernels and take 146 us in this one, BERT-large's with fp16 on the wire 4.2 ms and 1.95 ms (8 read
 // streams from HBM: 6.1-6.5 TB/s).  Results are the same to the bit: the same roundings in the
 // same order (to the wire type after the prescale and after every rank).
 //
-// There is no table in device memory.  A launch carries the addresses of up to kMaxRows tensors
-// (what fits in 4 KiB of kernel arguments: 44 tensors of 8 ranks), a response of more is several
+// There is no table in device memory.  A launch carries the addresses of up to 128 tensors
+// (what fits in 4 KiB of kernel arguments: 86 tensors of 8 ranks), a response of more is several
 // launches.  A table would have to be built and copied for every new set of addresses, and new
 // outputs are what an out-of-place call brings each time: with a cache of tables, BERT-large's
 // step spent 16 ms on rebuilding them whenever more sets rotated than it held.
@@ -93,6 +93,54 @@ __device__ __forceinline__ void add_ranks(Arr<W, N>& acc, uint32_t rank, uint32_
   if constexpr (B > 1) add_ranks<B / 2, W, N>(acc, rank, world, load, wire);
 }
 
+// The rows of up to eight ranks: addresses as 32-bit distances, in elements, from the lowest one of each rank (and of the
+// outputs), half the size of Rows', so that a launch carries up to 128 tensors (86 of eight ranks, where 64-bit addresses
+// leave room for 44).  Each launch more costs the stream 4 to 5 us between one's drain and the next one's start: of eight
+// ranks, ResNet-50's 161 gradients 153 -> 146.5 us, 320 tensors of 8 million elements in all 77 -> 62, 200 of 2 million
+// 47.5 -> 38.5.
+constexpr uint32_t kMaxShortRows = 128;  // two per lane of a wavefront
+constexpr uint32_t kShortWords = 864;
+struct ShortRows {
+  uint32_t first[kMaxShortRows];  // as in Rows
+  uint64_t base[9];               // outputs, rank 0, 1 ...
+  uint32_t d[kShortWords];        // per row: output, elements, rank 0, 1 ...
+};
+static_assert(sizeof(ShortRows) + 48 <= 4096, "kernel arguments");
+
+// What a workgroup needs of its row, of K ranks (more than eight: `world` of them).
+template <typename S, typename D, int K>
+struct ShortRow {
+  const ShortRows& rows;
+  const uint32_t* d;
+  uint32_t row;
+  __device__ __forceinline__ ShortRow(const ShortRows& r, uint32_t nrows, uint32_t chunk, uint32_t) : rows(r), row(0) {
+    if (nrows > 1) {
+      const uint32_t lane = threadIdx.x & 63, low = r.first[lane], high = r.first[64 + lane];
+      row = (uint32_t)__popcll(__ballot(low <= chunk)) + (uint32_t)__popcll(__ballot(high <= chunk)) - 1;
+    }
+    d = r.d + row * (K + 2);
+  }
+  __device__ __forceinline__ uint64_t elements() const { return d[1]; }
+  __device__ __forceinline__ gptr<D> output() const { return as_global<D>(rows.base[0]) + d[0]; }
+  __device__ __forceinline__ gptr<const S> input(uint32_t r) const { return as_global<const S>(rows.base[1 + r]) + d[2 + r]; }
+};
+template <typename S, typename D>
+struct LongRow {
+  const uint64_t* q;  // {output, elements, input of rank 0, 1 ...}
+  uint32_t row;
+  __device__ __forceinline__ LongRow(const Rows& r, uint32_t nrows, uint32_t chunk, uint32_t world)
+      : row(row_of(r, nrows, chunk)) {
+    q = r.q + row * (world + 2);
+  }
+  __device__ __forceinline__ uint64_t elements() const { return q[1]; }
+  __device__ __forceinline__ gptr<D> output() const { return as_global<D>(q[0]); }
+  __device__ __forceinline__ gptr<const S> input(uint32_t r) const { return as_global<const S>(q[2 + r]); }
+};
+template <int K>
+using RowsOf = typename std::conditional<K == kTogether, Rows, ShortRows>::type;  // of ranks_sum_k
+template <typename S, typename D, int K>
+using RowOf = typename std::conditional<K == kTogether, LongRow<S, D>, ShortRow<S, D, K>>::type;
+
 // For 1, 2 and more than 8 ranks.  One workgroup per chunk of kWG * kVec elements: 4 KiB of the wider side, one 16-byte
 // access per lane and rank, the loads of the first K ranks (K = min(world, 8)) all in flight before the first add.  The
 // arguments stay in the scalar cache, so a workgroup waits for one vector load (the search) and one batch of scalar
@@ -101,21 +149,20 @@ __device__ __forceinline__ void add_ranks(Arr<W, N>& acc, uint32_t rank, uint32_
 // XCD measure within 2 % of each other.
 template <typename S, typename W, typename D, int K, int ST>
 __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t ordered, uint32_t nrows, uint32_t world,
-                                                   double pre, double post, uint32_t flags, Rows rows) {
+                                                   double pre, double post, uint32_t flags, RowsOf<K> rows) {
   constexpr int VEC = kVec<S, D>;
   constexpr uint32_t kTile = kWG * VEC;
   constexpr bool kBytes = sizeof(S) == 1;  // byte elements are read through windows (vecmem.h)
   const uint32_t chunk = xcd_tile(blockIdx.x, XcdOrder{shift, ordered});
-  const uint32_t row = row_of(rows, nrows, chunk);
-  const uint64_t* q = rows.q + row * (world + 2);  // {output, elements, input of rank 0, 1 ...}
-  const uint64_t start = (uint64_t)(chunk - rows.first[row]) * kTile;
-  const uint64_t left = q[1] - start;
+  const RowOf<S, D, K> row(rows, nrows, chunk, world);
+  const uint64_t start = (uint64_t)(chunk - rows.first[row.row]) * kTile;
+  const uint64_t left = row.elements() - start;
   const uint32_t m = left < kTile ? (uint32_t)left : kTile;
-  gptr<D> out = as_global<D>(q[0]) + start;
+  gptr<D> out = row.output() + start;
   const Window win = store_window<ST>(out, m * (uint32_t)sizeof(D));
   const typename Factor<W>::type fin = (typename Factor<W>::type)pre, fout = (typename Factor<W>::type)post;
   const bool scale_in = flags & kScaleIn, scale_out = flags & kScaleOut;
-  auto source = [&](uint32_t rank) { return as_global<const S>(q[2 + rank]) + start; };
+  auto source = [&](uint32_t rank) { return row.input(rank) + start; };
   gptr<const S> src[K];  // all at once, ahead of the branch
 #pragma unroll
   for (int k = 0; k < K; ++k) src[k] = source(k);
@@ -149,8 +196,8 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
     out[t] = from_wire<W, D, 1>(acc, fout, scale_out).v[0];
   }
   if constexpr (ST == kStoreWT) {  // into a fusion buffer: zeros up to the next 16-byte boundary
-    const uint32_t pad = (uint32_t)(0u - (uint32_t)q[1] * (uint32_t)sizeof(D)) & 15u;
-    if (left <= kTile && threadIdx.x < pad) as_global<uint8_t>(q[0])[q[1] * sizeof(D) + threadIdx.x] = 0;
+    const uint32_t pad = (uint32_t)(0u - (uint32_t)row.elements() * (uint32_t)sizeof(D)) & 15u;
+    if (left <= kTile && threadIdx.x < pad) as_global<uint8_t>(win.base)[left * sizeof(D) + threadIdx.x] = 0;
   }
 }
 
@@ -169,22 +216,21 @@ __global__ __launch_bounds__(kWG) void ranks_sum_k(uint32_t shift, uint32_t orde
 template <typename S, typename W, typename D, int K, int ST>
 __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t shift, uint32_t ordered, uint32_t nrows,
                                                                      double pre, double post, uint32_t flags,
-                                                                     Rows rows) {
+                                                                     ShortRows rows) {
   constexpr int VEC = kVec<S, D>, WV = kSplitWaves<K>, U = kSplitVecs<K>;
   constexpr uint32_t kTile = 64 * U * VEC;
   constexpr bool kBytes = sizeof(S) == 1;
   static_assert(U <= WV, "a wavefront per 64 vectors of the sum");
   __shared__ Arr<W, VEC> lds[K][64 * U];
   const uint32_t chunk = xcd_tile(blockIdx.x, XcdOrder{shift, ordered});
-  const uint32_t row = row_of(rows, nrows, chunk);
-  const uint64_t* q = rows.q + row * (K + 2);  // {output, elements, input of rank 0, 1 ...}
-  const uint64_t start = (uint64_t)(chunk - rows.first[row]) * kTile;
-  const uint64_t left = q[1] - start;
+  const ShortRow<S, D, K> row(rows, nrows, chunk, K);
+  const uint64_t start = (uint64_t)(chunk - rows.first[row.row]) * kTile;
+  const uint64_t left = row.elements() - start;
   const uint32_t m = left < kTile ? (uint32_t)left : kTile;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const typename Factor<W>::type fin = (typename Factor<W>::type)pre, fout = (typename Factor<W>::type)post;
   const bool scale_in = flags & kScaleIn, scale_out = flags & kScaleOut;
-  auto source = [&](uint32_t rank) { return as_global<const S>(q[2 + rank]) + start; };
+  auto source = [&](uint32_t rank) { return row.input(rank) + start; };
   const bool second = K == 2 * WV || wave + WV < K;
   const gptr<const S> src[2] = {source(wave), source(second ? wave + WV : wave)};
   const uint32_t nv = m / VEC;
@@ -213,7 +259,7 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t sh
     }
   }
   __syncthreads();
-  gptr<D> out = as_global<D>(q[0]) + start;
+  gptr<D> out = row.output() + start;
   const Window win = store_window<ST>(out, m * (uint32_t)sizeof(D));
   const uint32_t v = threadIdx.x;
   if (v < nv) {
@@ -230,8 +276,8 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t sh
     out[t] = from_wire<W, D, 1>(acc, fout, scale_out).v[0];
   }
   if constexpr (ST == kStoreWT) {  // into a fusion buffer: zeros up to the next 16-byte boundary
-    const uint32_t pad = (uint32_t)(0u - (uint32_t)q[1] * (uint32_t)sizeof(D)) & 15u;
-    if (left <= kTile && threadIdx.x < pad) as_global<uint8_t>(q[0])[q[1] * sizeof(D) + threadIdx.x] = 0;
+    const uint32_t pad = (uint32_t)(0u - (uint32_t)row.elements() * (uint32_t)sizeof(D)) & 15u;
+    if (left <= kTile && threadIdx.x < pad) as_global<uint8_t>(win.base)[left * sizeof(D) + threadIdx.x] = 0;
   }
 }
 
@@ -241,27 +287,101 @@ __global__ __launch_bounds__(64 * kSplitWaves<K>) void ranks_split_k(uint32_t sh
 template <int K>
 constexpr bool kSplit = K >= 3;
 
-template <typename S, typename W, typename D, int K, int ST>
-hipError_t launch_rows(const RanksCall& c, const Rows& rows, uint32_t nrows, uint32_t chunks, bool last) {
+// The rows of one launch.  add() refuses one that it has no room for.
+class LongTable {
+ public:
+  explicit LongTable(uint32_t world) : world_(world), max_(std::min(kMaxRows, kQwords / (world + 2))) {}
+  uint32_t rows() const { return n_; }
+  // Elements that a row can have, a multiple of `tile`.
+  static uint64_t most(uint64_t) { return ~0ull; }
+  template <typename Input>
+  bool add(uint32_t first, uint64_t output, uint64_t elements, Input&& input) {
+    if (n_ == max_) return false;
+    uint64_t* q = table_.q + n_ * (world_ + 2);
+    *q++ = output;
+    *q++ = elements;
+    for (uint32_t r = 0; r < world_; ++r) *q++ = input(r);
+    table_.first[n_++] = first;
+    return true;
+  }
+  const Rows& finished() {
+    for (uint32_t i = n_; i < kMaxRows; ++i) table_.first[i] = ~0u;
+    n_ = 0;
+    return table_;
+  }
+
+ private:
+  const uint32_t world_, max_;
+  uint32_t n_ = 0;
+  Rows table_;
+};
+
+// IS and OS: bytes of an element on either side, which every address is a multiple of.
+template <int K, uint32_t IS, uint32_t OS>
+class ShortTable {
+ public:
+  explicit ShortTable(uint32_t) {}
+  uint32_t rows() const { return n_; }
+  static uint64_t most(uint64_t tile) { return 0xffffffffull / tile * tile; }
+  template <typename Input>
+  bool add(uint32_t first, uint64_t output, uint64_t elements, Input&& input) {
+    constexpr uint32_t max = std::min(kMaxShortRows, kShortWords / (K + 2));
+    if (n_ == max) return false;
+    uint64_t* at = at_[n_];
+    at[0] = output;
+    for (uint32_t r = 0; r < K; ++r) at[1 + r] = input(r);
+    uint64_t lo[K + 1], hi[K + 1];
+    for (uint32_t r = 0; r <= K; ++r) {
+      lo[r] = n_ ? std::min(lo_[r], at[r]) : at[r];
+      hi[r] = n_ ? std::max(hi_[r], at[r]) : at[r];
+      if ((hi[r] - lo[r]) / (r ? IS : OS) > 0xffffffffull) return false;  // never the first row of a launch
+    }
+    std::copy(lo, lo + K + 1, lo_);
+    std::copy(hi, hi + K + 1, hi_);
+    table_.d[n_ * (K + 2) + 1] = (uint32_t)elements;
+    table_.first[n_++] = first;
+    return true;
+  }
+  const ShortRows& finished() {
+    for (uint32_t i = 0; i < n_; ++i) {
+      uint32_t* d = table_.d + i * (K + 2);
+      d[0] = (uint32_t)((at_[i][0] - lo_[0]) / OS);
+      for (uint32_t r = 0; r < K; ++r) d[2 + r] = (uint32_t)((at_[i][1 + r] - lo_[1 + r]) / IS);
+    }
+    std::copy(lo_, lo_ + K + 1, table_.base);
+    for (uint32_t i = n_; i < kMaxShortRows; ++i) table_.first[i] = ~0u;
+    n_ = 0;
+    return table_;
+  }
+
+ private:
+  uint32_t n_ = 0;
+  uint64_t lo_[K + 1], hi_[K + 1], at_[kMaxShortRows][K + 1];
+  ShortRows table_;
+};
+
+template <typename S, typename W, typename D, int K, int ST, typename Table>
+hipError_t launch_rows(const RanksCall& c, Table& table, uint32_t chunks, bool last) {
   constexpr uint32_t kVecBytes = kVec<S, D> * (uint32_t)(sizeof(S) > sizeof(D) ? sizeof(S) : sizeof(D));
   hipEvent_t completion = last ? c.completion : nullptr;
+  const uint32_t nrows = table.rows();
   if constexpr (kSplit<K>) {
     const XcdOrder order = K < 8 ? xcd_order(chunks, 64 * kSplitVecs<K> * kVecBytes) : XcdOrder{0, 0};
     return launch_shaped(completion, ranks_split_k<S, W, D, K, ST>, chunks, 64 * kSplitWaves<K>, c.stream, order.shift,
-                         order.ordered, nrows, c.pre, c.post, c.flags, rows);
+                         order.ordered, nrows, c.pre, c.post, c.flags, table.finished());
   } else {
     const XcdOrder order = xcd_order(chunks, kWG * kVecBytes);
     return launch_with(completion, ranks_sum_k<S, W, D, K ? K : kTogether, ST>, chunks, c.stream, order.shift,
-                       order.ordered, nrows, c.world, c.pre, c.post, c.flags, rows);
+                       order.ordered, nrows, c.world, c.pre, c.post, c.flags, table.finished());
   }
 }
 
 // Fills launches with as many rows as their arguments hold.  A tensor that would take a launch beyond
-// kMaxWorkgroups chunks is cut there and goes on in the next one.
+// kMaxWorkgroups chunks, or has more elements than a row can say, is cut there and goes on in the next one.
 template <typename S, typename W, typename D, int K>
 int run_ranks(const RanksCall& c) {
   constexpr uint64_t kTile = (uint64_t)(kSplit<K> ? 64 * kSplitVecs<K> : kWG) * kVec<S, D>;
-  const uint32_t max_rows = std::min(kMaxRows, kQwords / (c.world + 2));
+  typedef typename std::conditional<K != 0, ShortTable<K ? K : 1, sizeof(S), sizeof(D)>, LongTable>::type Table;
   int entry = 0;
   uint64_t done = 0;  // elements of the current entry that earlier launches took
   // One rank's tensor that is its own output and changes neither type nor scale is left where it is.
@@ -274,19 +394,16 @@ int run_ranks(const RanksCall& c) {
     if (c.completion) HVDHIP_CHECK(hipEventRecord(c.completion, c.stream));
     return 0;
   }
-  Rows rows;
+  Table table(c.world);
   while (entry < c.n) {
-    uint32_t nrows = 0;
     uint64_t chunks = 0;
-    uint64_t* q = rows.q;
-    while (entry < c.n && nrows < max_rows && chunks < kMaxWorkgroups) {
+    while (entry < c.n && chunks < kMaxWorkgroups) {
       const uint64_t left = (uint64_t)c.counts[entry] - done;
-      const uint64_t take = std::min(left, (kMaxWorkgroups - chunks) * kTile);
-      rows.first[nrows++] = (uint32_t)chunks;
-      *q++ = (uint64_t)(uintptr_t)c.outputs[entry] + done * sizeof(D);
-      *q++ = take;
-      for (uint32_t r = 0; r < c.world; ++r)
-        *q++ = (uint64_t)(uintptr_t)c.inputs[(size_t)r * (size_t)c.n + (size_t)entry] + done * sizeof(S);
+      const uint64_t take = std::min(std::min(left, Table::most(kTile)), (kMaxWorkgroups - chunks) * kTile);
+      auto input = [&](uint32_t r) {
+        return (uint64_t)(uintptr_t)c.inputs[(size_t)r * (size_t)c.n + (size_t)entry] + done * sizeof(S);
+      };
+      if (!table.add((uint32_t)chunks, (uint64_t)(uintptr_t)c.outputs[entry] + done * sizeof(D), take, input)) break;
       chunks += (take + kTile - 1) / kTile;
       done += take;
       if (take == left) {
@@ -295,11 +412,10 @@ int run_ranks(const RanksCall& c) {
         skip_idle();
       }
     }
-    for (uint32_t i = nrows; i < kMaxRows; ++i) rows.first[i] = ~0u;
     const bool last = entry == c.n;
     const hipError_t status = c.flags & kPadOut
-                                  ? launch_rows<S, W, D, K, kStoreWT>(c, rows, nrows, (uint32_t)chunks, last)
-                                  : launch_rows<S, W, D, K, kStoreNT>(c, rows, nrows, (uint32_t)chunks, last);
+                                  ? launch_rows<S, W, D, K, kStoreWT>(c, table, (uint32_t)chunks, last)
+                                  : launch_rows<S, W, D, K, kStoreNT>(c, table, (uint32_t)chunks, last);
     HVDHIP_CHECK_LAUNCH("ranks_sum_k", status);
   }
   return 0;

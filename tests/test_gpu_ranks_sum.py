@@ -181,6 +181,72 @@ def test_ranks_sum_refuses_overlap(gpu):
     assert not call([p, p + 400], [p, p + 400, p + 400, p], [100, 100], 2)     # output over another entry's input
 
 
+# tensors that one launch carries, by the number of ranks
+CARRIED = {1: 128, 2: 128, 3: 128, 5: 123, 8: 86, 9: 40}
+
+
+@pytest.mark.parametrize("world", CARRIED)
+@pytest.mark.parametrize("more", [-1, 0, 1, None])
+def test_as_many_tensors_as_a_launch_carries_and_more(gpu, world, more):
+    """Wherever they lie: each rank's tensors, and the outputs, in an order of their own within one allocation."""
+    n = 2 * CARRIED[world] + 3 if more is None else CARRIED[world] + more
+    rng = np.random.default_rng(n)
+    counts = [int(x) for x in rng.choice([1, 3, 256, 1023, 1025], n)]
+
+    def scattered():
+        whole = torch.empty(1030 * n, dtype=torch.float32, device="cuda").normal_()
+        return whole, [whole[1030 * int(k):1030 * int(k) + c] for k, c in zip(rng.permutation(n), counts)]
+
+    ranks = [scattered() for _ in range(world)]
+    whole, outs = scattered()
+    want = whole.clone()
+    for i, o in enumerate(outs):
+        acc = ranks[0][1][i].clone()
+        for r in range(1, world):
+            acc += ranks[r][1][i]
+        at = o.storage_offset()
+        want[at:at + counts[i]] = acc
+    torch.cuda.synchronize()
+    f32 = DTYPE["float32"]
+    assert H.ranks_sum([o.data_ptr() for o in outs], [t.data_ptr() for _, r in ranks for t in r], counts, world, f32, f32,
+                       f32, 1.0, 1.0, gpu.stream)
+    gpu.stream.synchronize()
+    assert torch.equal(whole, want)
+
+
+@pytest.mark.parametrize("world", [1, 2, 3])
+def test_tensors_that_32_bits_do_not_span(gpu, world):
+    """Bytes more than 2^32 apart in one rank or in the outputs, and a tensor of more than 2^32 of them."""
+    u8, far = DTYPE["uint8"], (1 << 32) + 70001
+    big = [torch.empty(far, dtype=torch.uint8, device="cuda").random_() for _ in range(world)]
+    out = torch.zeros(far + 16, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert H.ranks_sum([out.data_ptr()], [b.data_ptr() for b in big], [far], world, u8, u8, u8, 1.0, 1.0, gpu.stream)
+    gpu.stream.synchronize()
+    acc = big[0].clone()
+    for b in big[1:]:
+        acc += b
+    assert torch.equal(out[:far], acc) and not out[far:].any()
+    del acc
+    # the first rank's tensors far apart, the others' close together; then the outputs
+    n = 5000
+    ends = [big[0][:n], big[0][-n:], big[0][n:2 * n]]
+    near = [[torch.empty(n, dtype=torch.uint8, device="cuda").random_() for _ in ends] for _ in range(world - 1)]
+    small = [torch.empty_like(e) for e in ends]
+    spread = [out[:n], out[far - n:far], out[n:2 * n]]
+    torch.cuda.synchronize()
+    for outs, first in ((small, ends), (spread, near[0] if near else ends)):
+        ranks = [first] + near
+        assert H.ranks_sum([o.data_ptr() for o in outs], [t.data_ptr() for r in ranks for t in r], [n] * 3, len(ranks), u8,
+                           u8, u8, 1.0, 1.0, gpu.stream)
+        gpu.stream.synchronize()
+        for i, o in enumerate(outs):
+            acc = ranks[0][i].clone()
+            for r in ranks[1:]:
+                acc += r[i]
+            assert torch.equal(o, acc), i
+
+
 @pytest.mark.parametrize("case", ["peers_are_outputs", "same_output_twice", "more_ranks_than_one_pass"])
 def test_engine_sums_through_a_buffer_where_one_pass_cannot(monkeypatch, case):
     import horovod_amd.torch as hvd
