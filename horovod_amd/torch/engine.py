@@ -83,8 +83,8 @@ def _is_part(t, e):
             and t.shape[1:] == e.tensor.shape[1:] and t.is_contiguous())
 
 
-# A response that reads this many bytes, all ranks together, is followed by the next one on its own stream: each has the
-# memory to itself then, where two at a time stream 3 to 5 % slower between them and the first completes with the second.
+# Behind a response that reads this many bytes, all ranks together, the others of its cycle stay on its stream: each has
+# the memory to itself then, where two at a time stream 3 to 5 % slower between them and the first completes with the second.
 # Below, the start and the end of a response hide in the other's work.  Four responses on one stream and on two, us: 8
 # ranks, 256 MB each 199 and 197, 320 MB 241 and 242, 512 MB 367 and 371, 1,280 MB 890 and 920; 2 ranks, 128 MB 141 and
 # 133, 320 MB 314 and 316, 960 MB 882 and 911; 16 ranks, 320 MB 242 and 250.
@@ -111,6 +111,7 @@ class Engine:
         self.cycles = 0
         self.responses = 0       # fused responses executed so far
         self.ready = {}          # framework stream -> event recorded during the current cycle
+        self.staying = 0         # the last cycle with a response whose stream the others behind it keep to
         self.busy = {}           # framework stream -> cycle up to which it is taken to be busy
 
     # ---- queueing -------------------------------------------------------
@@ -319,7 +320,9 @@ class Engine:
         enqueued on, all but the one that the caller makes it wait for (`made`).  nbytes: what it reads."""
         self.responses += 1
         slot = self.slot
-        if nbytes < _BYTES_OF_ITS_OWN:
+        if nbytes >= _BYTES_OF_ITS_OWN:
+            self.staying = self.cycles
+        if self.staying != self.cycles:
             self.slot = (slot + 1) % len(self.streams)
         s = self.streams[slot]
         requests, producers = _front.requests(group)

@@ -163,14 +163,21 @@ def test_nothing_is_left_of_finished_requests(hvd):
     assert counts() == before and before[1] == 0
 
 
-def test_a_large_response_is_followed_on_its_own_stream(hvd, monkeypatch):
+def test_behind_a_large_response_a_cycle_keeps_its_stream(hvd, monkeypatch):
     from horovod_amd.torch import engine, mpi_ops
-    hvd.init(size=2, num_streams=2)
+    hvd.init(size=2, num_streams=2, fusion_threshold=0)  # a response per tensor
     monkeypatch.setattr(engine, "_BYTES_OF_ITS_OWN", 2 * 4 * 1000)
-    slots = []
-    for n in (999, 999, 1000, 4000, 1, 1000):
-        t = torch.full((n,), 1.5, device="cuda")
-        handle = hvd.allreduce_async(t, op=hvd.Sum)
-        slots.append(mpi_ops._engine.slot)
-        assert torch.equal(hvd.synchronize(handle), 2 * t)
-    assert slots == [0, 1, 0, 0, 0, 1]
+    slots, begin = [], engine.Engine._begin
+
+    def recorded(self, group, made=None, nbytes=0):
+        found = begin(self, group, made, nbytes)
+        slots.append(found[0])
+        return found
+
+    monkeypatch.setattr(engine.Engine, "_begin", recorded)
+    for sizes in ((999, 999, 5), (4, 1000, 5, 4000, 1), (7,), (7,)):
+        tensors = [torch.full((n,), 1.5, device="cuda") for n in sizes]
+        handles = [hvd.allreduce_async(t, op=hvd.Sum) for t in tensors]
+        for h, t in zip(handles, tensors):
+            assert torch.equal(hvd.synchronize(h), 2 * t)
+    assert slots == [0, 1, 0] + [1, 0, 0, 0, 0] + [0] + [1]
