@@ -48,30 +48,41 @@ constexpr uint32_t kChunk = kChunkBytes / (uint32_t)sizeof(W);
 struct Level {
   uint32_t nrows;
   uint32_t chunks;
-  uint32_t words;  // per row in Rows::q
+  uint32_t words;  // per row in ShortRows::d
   uint32_t first;  // pair (dots_k) or group of four vectors (level_k) that blockIdx.y = 0 works on
   uint32_t flags;
   uint64_t in_stride, out_stride;
   double pre, post, guard;
   const double* in_sums;
-  const double* coeffs;  // [(pair * kMaxRows + row) * 2], or NULL: from in_sums
+  const double* coeffs;  // [(pair * kMaxShortRows + row) * 2], or NULL: from in_sums
   double* out_sums;
 };
 
+// A row: {distance from base[0], elements in two words, distances from base[1], base[2] ...}.
+constexpr uint32_t kRowHead = 3;
+static_assert(sizeof(ShortRows) + sizeof(Level) <= 4096, "kernel arguments");
+
 struct Place {
-  const uint64_t* q;
+  const uint32_t* d;
   uint32_t row, chunk;
-  uint64_t start;  // element within the row
-  uint32_t m;      // elements of this chunk
+  uint64_t elements, start;  // of the row; element within it
+  uint32_t m;                // elements of this chunk
+  // What base[k] is the lowest one of.
+  template <typename T>
+  __device__ __forceinline__ gptr<T> at(const ShortRows& rows, uint32_t k) const {
+    return as_global<T>(rows.base[k]) + (k == 0 ? d[0] : d[kRowHead - 1 + k]);
+  }
 };
+__device__ __forceinline__ uint64_t row_elements(const uint32_t* d) { return d[1] | (uint64_t)d[2] << 32; }
 template <typename W>
-__device__ __forceinline__ Place place(const Rows& rows, const Level& l) {
+__device__ __forceinline__ Place place(const ShortRows& rows, const Level& l) {
   Place p;
   p.chunk = blockIdx.x;
   p.row = row_of(rows, l.nrows, p.chunk);
-  p.q = rows.q + p.row * l.words;
+  p.d = rows.d + p.row * l.words;
+  p.elements = row_elements(p.d);
   p.start = (uint64_t)(p.chunk - rows.first[p.row]) * kChunk<W>;
-  const uint64_t left = p.q[0] - p.start;
+  const uint64_t left = p.elements - p.start;
   p.m = left < kChunk<W> ? (uint32_t)left : kChunk<W>;
   return p;
 }
@@ -149,11 +160,11 @@ template <int NP>
 __device__ __forceinline__ void row_coeffs(const Level& l, const Place& p, uint32_t first_chunk, uint32_t chunks,
                                            uint32_t pair, double (&c)[2 * NP]) {
   if (l.coeffs) {
-    const double* t = l.coeffs + 2 * ((uint64_t)pair * kMaxRows + p.row);
+    const double* t = l.coeffs + 2 * ((uint64_t)pair * kMaxShortRows + p.row);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      c[2 * k] = t[2 * kMaxRows * k];
-      c[2 * k + 1] = t[2 * kMaxRows * k + 1];
+      c[2 * k] = t[2 * kMaxShortRows * k];
+      c[2 * k + 1] = t[2 * kMaxShortRows * k + 1];
     }
     return;
   }
@@ -177,15 +188,15 @@ __device__ __forceinline__ Arr<W, N> combined(double ca, const Arr<W, N>& a, dou
   return y;
 }
 
-// Row: {elements, anything, rank 0, 1 ...}.  KEEP: whose tensors the loads leave in the Infinity Cache for the
+// Bases: anything, rank 0, 1 ...  KEEP: whose tensors the loads leave in the Infinity Cache for the
 // pass that reads them again (1 every pair's first rank's, 2 all).
 template <typename S, typename W, int KEEP>
-__global__ __launch_bounds__(kWG) void dots_k(Level l, Rows rows) {
+__global__ __launch_bounds__(kWG) void dots_k(Level l, ShortRows rows) {
   constexpr int VEC = kVec<S, W>;
   if (blockIdx.x >= l.chunks) return;
   const Place p = place<W>(rows, l);
-  const gptr<const S> a = as_global<const S>(p.q[2 + 2 * blockIdx.y]) + p.start;
-  const gptr<const S> b = as_global<const S>(p.q[3 + 2 * blockIdx.y]) + p.start;
+  const gptr<const S> a = p.at<const S>(rows, 1 + 2 * blockIdx.y) + p.start;
+  const gptr<const S> b = p.at<const S>(rows, 2 + 2 * blockIdx.y) + p.start;
   const typename Factor<W>::type fin = (typename Factor<W>::type)l.pre;
   const bool scale_in = l.flags & kScaleIn;
   Sums sums;
@@ -207,30 +218,31 @@ __global__ __launch_bounds__(kWG) void dots_k(Level l, Rows rows) {
   sums.store(l, l.first + blockIdx.y, p.chunk);
 }
 
-// LEAVES, row: {elements, workspace, rank 0, 1 ...}; else {elements, workspace}, and the vectors are in_stride
-// apart in the workspace, where the two results take the places of two of the four.
+// LEAVES, bases: workspace, rank 0, 1 ...; else the workspace alone, and the vectors are in_stride
+// apart in it, where the two results take the places of two of the four.
 template <typename S, typename W, bool LEAVES>
-__global__ __launch_bounds__(kWG) void level_k(Level l, Rows rows) {
+__global__ __launch_bounds__(kWG) void level_k(Level l, ShortRows rows) {
   constexpr int VEC = kVec<S, W>;
   if (blockIdx.x >= l.chunks) return;
   const Place p = place<W>(rows, l);
   const uint32_t quad = l.first + blockIdx.y;
   const typename Factor<W>::type fin = (typename Factor<W>::type)l.pre;
   const bool scale_in = LEAVES && (l.flags & kScaleIn);
+  const uint64_t work = reinterpret_cast<uint64_t>(p.at<W>(rows, 0));
   gptr<const S> in[4];
 #pragma unroll
   for (uint32_t k = 0; k < 4; ++k)
-    in[k] = as_global<const S>(LEAVES ? p.q[2 + 4 * blockIdx.y + k] : p.q[1] + (uint64_t)(4 * quad + k) * l.in_stride) +
-            p.start;
+    in[k] = (LEAVES ? p.at<const S>(rows, 1 + 4 * blockIdx.y + k)
+                    : as_global<const S>(work + (uint64_t)(4 * quad + k) * l.in_stride)) + p.start;
   Window out[2];
   gptr<W> to[2];
 #pragma unroll
   for (uint32_t k = 0; k < 2; ++k) {
-    to[k] = as_global<W>(p.q[1] + (uint64_t)(2 * quad + k) * l.out_stride) + p.start;
+    to[k] = as_global<W>(work + (uint64_t)(2 * quad + k) * l.out_stride) + p.start;
     out[k] = store_window<kStoreWT>(to[k], p.m * (uint32_t)sizeof(W));
   }
   double c[4];
-  row_coeffs<2>(l, p, rows.first[p.row], (uint32_t)((p.q[0] + kChunk<W> - 1) / kChunk<W>), 2 * quad, c);
+  row_coeffs<2>(l, p, rows.first[p.row], (uint32_t)((p.elements + kChunk<W> - 1) / kChunk<W>), 2 * quad, c);
   Sums sums;
   over_vectors<2>(p.m / VEC, [&](auto u, uint32_t v) {
     constexpr int U = decltype(u)::value;
@@ -264,20 +276,21 @@ __global__ __launch_bounds__(kWG) void level_k(Level l, Rows rows) {
   sums.store(l, quad, p.chunk);
 }
 
-// LEAVES (two ranks), row: {elements, output, rank 0, rank 1}; else {elements, output, workspace}.
+// LEAVES (two ranks), bases: output, rank 0, rank 1; else output, workspace.
 template <typename S, typename W, typename D, bool LEAVES>
-__global__ __launch_bounds__(kWG) void last_k(Level l, Rows rows) {
+__global__ __launch_bounds__(kWG) void last_k(Level l, ShortRows rows) {
   constexpr int VEC = kVec<S, D>;
   if (blockIdx.x >= l.chunks) return;
   const Place p = place<W>(rows, l);
   const typename Factor<W>::type fin = (typename Factor<W>::type)l.pre, fout = (typename Factor<W>::type)l.post;
   const bool scale_in = LEAVES && (l.flags & kScaleIn), scale_out = l.flags & kScaleOut;
-  const gptr<const S> a = as_global<const S>(p.q[2]) + p.start;
-  const gptr<const S> b = as_global<const S>(LEAVES ? p.q[3] : p.q[2] + l.in_stride) + p.start;
-  const gptr<D> to = as_global<D>(p.q[1]) + p.start;
+  const gptr<const S> a = p.at<const S>(rows, 1) + p.start;
+  const gptr<const S> b = LEAVES ? p.at<const S>(rows, 2) + p.start
+                                 : as_global<const S>(reinterpret_cast<uint64_t>(a) + l.in_stride);
+  const gptr<D> to = p.at<D>(rows, 0) + p.start;
   const Window out = store_window<kStoreNT>(to, p.m * (uint32_t)sizeof(D));
   double c[2];
-  row_coeffs<1>(l, p, rows.first[p.row], (uint32_t)((p.q[0] + kChunk<W> - 1) / kChunk<W>), 0, c);
+  row_coeffs<1>(l, p, rows.first[p.row], (uint32_t)((p.elements + kChunk<W> - 1) / kChunk<W>), 0, c);
   over_vectors<4>(p.m / VEC, [&](auto u, uint32_t v) {
     constexpr int U = decltype(u)::value;
     Arr<S, VEC> x[U], y[U];
@@ -303,14 +316,14 @@ __global__ __launch_bounds__(kWG) void last_k(Level l, Rows rows) {
 
 // One workgroup per row and pair of a level: the coefficients, where some row has more chunks than kReaddMax.
 struct RowStarts {
-  uint32_t first[kMaxRows + 1];
+  uint32_t first[kMaxShortRows + 1];
 };
 __global__ __launch_bounds__(kWG) void coeffs_k(const double* __restrict__ sums, double* __restrict__ coeffs,
                                                 uint32_t chunks, double guard, RowStarts rows) {
   const uint32_t row = blockIdx.x, pair = blockIdx.y;
   const uint32_t first = rows.first[row], count = rows.first[row + 1] - first;
   const double* s = sums + 3 * ((uint64_t)pair * chunks + first);
-  double* c = coeffs + 2 * ((uint64_t)pair * kMaxRows + row);
+  double* c = coeffs + 2 * ((uint64_t)pair * kMaxShortRows + row);
   if (count <= kReaddMax) {
     if (threadIdx.x >= 64) return;
     const Triple r = short_row_sum(s, count, threadIdx.x);
@@ -339,14 +352,14 @@ struct HeldRanks {
   }
   __device__ __forceinline__ bool has_tail() const { return nv * VEC + lane < m; }
 
-  __device__ __forceinline__ void load(const uint64_t* ranks, uint64_t start, uint32_t elements, uint32_t lane_,
+  __device__ __forceinline__ void load(const ShortRows& rows, const Place& at, uint32_t lane_,
                                        typename Factor<W>::type fin, bool scale_in) {
-    m = elements;
+    m = at.m;
     nv = m / VEC;
     lane = lane_;
 #pragma unroll
     for (int r = 0; r < WORLD; ++r) {
-      const gptr<const W> p = as_global<const W>(ranks[r]) + start;
+      const gptr<const W> p = at.at<const W>(rows, 1 + r) + at.start;
 #pragma unroll
       for (int u = 0; u < kVecs; ++u)
         if (lane + u * kWG < nv) x[r][u] = __builtin_bit_cast(R, ldv<W, VEC>(p + (size_t)(lane + u * kWG) * VEC));
@@ -414,8 +427,8 @@ __device__ __forceinline__ void held_levels(HeldRanks<W, WORLD>& h, uint32_t gro
   if constexpr (PAIRS > 1) held_levels<PAIRS / 2, W, WORLD, G>(h, group, guard, red + G);
 }
 
-// The whole tree of rows of at most G chunks, a workgroup each: G groups of 256 lanes have a chunk of every rank.  Row:
-// {elements, output, rank 0, 1 ...}.  The operations and their order are those of the launches it stands for, four of
+// The whole tree of rows of at most G chunks, a workgroup each: G groups of 256 lanes have a chunk of every rank.
+// Bases: output, rank 0, 1 ...  The operations and their order are those of the launches it stands for, four of
 // them for eight ranks, each of which costs the stream 4 to 5 us however little it does.  Bound by the chain of one
 // workgroup: a level's sums, two trips through LDS and a divide, 1 us, and what a compute unit takes to load the ranks.
 // fp32, us: 8 ranks of 10 rows of 1,000 elements 15.7 -> 6.6, of 44 rows of one chunk 19.6 -> 9.7, of two 20.2 -> 13.4,
@@ -423,18 +436,23 @@ __device__ __forceinline__ void held_levels(HeldRanks<W, WORLD>& h, uint32_t gro
 // row of them takes as long in fp16 (16.7) as level by level; with a narrower type on the wire the levels' lanes have
 // other elements than the ranks', and a row's bits would depend on whether a longer row is beside it.
 template <typename W, int WORLD, int G>
-__global__ __launch_bounds__(G * kWG) void tree_held_k(Level l, Rows rows) {
+__global__ __launch_bounds__(G * kWG) void tree_held_k(Level l, ShortRows rows) {
   constexpr int VEC = HeldRanks<W, WORLD>::VEC, kVecs = HeldRanks<W, WORLD>::kVecs;
-  const uint64_t* q = rows.q + blockIdx.x * l.words;
   const typename Factor<W>::type fin = (typename Factor<W>::type)l.pre, fout = (typename Factor<W>::type)l.post;
-  const uint32_t group = threadIdx.x / kWG, count = (uint32_t)q[0], start = group * kChunk<W>;
-  const uint32_t left = start < count ? count - start : 0;
+  const uint32_t group = threadIdx.x / kWG;
+  Place p;
+  p.row = blockIdx.x;
+  p.d = rows.d + p.row * l.words;
+  p.elements = row_elements(p.d);
+  p.start = group * kChunk<W>;
+  const uint32_t left = p.start < p.elements ? (uint32_t)(p.elements - p.start) : 0;
+  p.m = left < kChunk<W> ? left : kChunk<W>;
   HeldRanks<W, WORLD> h;
-  h.load(q + 2, start, left < kChunk<W> ? left : kChunk<W>, threadIdx.x % kWG, fin, l.flags & kScaleIn);
+  h.load(rows, p, threadIdx.x % kWG, fin, l.flags & kScaleIn);
   __shared__ double red[(WORLD == 8 ? 3 : WORLD == 4 ? 2 : 1) * G][WORLD / 2][3][kWG / 64];
   held_levels<WORLD / 2, W, WORLD, G>(h, group, l.guard, red);
   const bool scale_out = l.flags & kScaleOut;
-  const gptr<W> to = as_global<W>(q[1]) + start;
+  const gptr<W> to = p.at<W>(rows, 0) + p.start;
   const Window out = store_window<kStoreNT>(to, h.m * (uint32_t)sizeof(W));
 #pragma unroll
   for (int u = 0; u < kVecs; ++u)
@@ -457,7 +475,7 @@ struct Group {
 };
 
 int next_group(const int64_t* counts, int n, int begin, uint32_t world, uint32_t wire_size, Group* out) {
-  const uint32_t max_rows = std::min(kMaxRows, kQwords / (2 + std::min(world, kRanksAtOnce)));
+  const uint32_t max_rows = std::min(kMaxShortRows, kShortWords / (kRowHead + std::min(world, kRanksAtOnce)));
   const uint64_t chunk = kChunkBytes / wire_size;
   const uint64_t max_chunks = kMaxWorkgroups / std::max(1u, world / 2);
   Group g = {begin, begin, 0, 0, 0, 0, {0, 0}, 0, 0};
@@ -475,7 +493,7 @@ int next_group(const int64_t* counts, int n, int begin, uint32_t world, uint32_t
   g.sums_at[0] = world >= 4 ? world / 2 * g.vector_bytes : 0;
   g.sums_at[1] = g.sums_at[0] + up256(world / 2 * triples);
   g.coeffs_at = g.sums_at[1] + up256(world / 4 * triples);
-  g.bytes = g.coeffs_at + up256(g.max_row_chunks > kReaddMax ? world / 2 * (uint64_t)kMaxRows * 2 * sizeof(double) : 0);
+  g.bytes = g.coeffs_at + up256(g.max_row_chunks > kReaddMax ? world / 2 * (uint64_t)kMaxShortRows * 2 * sizeof(double) : 0);
   *out = g;
   return 0;
 }
@@ -505,11 +523,15 @@ class Tree {
       return 0;
     }
     for (int at = 0; at < last;) {
-      int rc = next_group(c_.counts, last, at, c_.world, sizeof(W), &g_);
+      Group whole;  // what the workspace was sized for
+      int rc = next_group(c_.counts, last, at, c_.world, sizeof(W), &whole);
       if (rc) return rc;
-      rc = group(g_.end == last ? c_.completion : nullptr);
-      if (rc) return rc;
-      at = g_.end;
+      for (; at < whole.end; at = g_.end) {
+        rc = next_group(c_.counts, within_reach(at, whole.end), at, c_.world, sizeof(W), &g_);
+        if (rc) return rc;
+        rc = group(g_.end == last ? c_.completion : nullptr);
+        if (rc) return rc;
+      }
     }
     return 0;
   }
@@ -604,27 +626,60 @@ class Tree {
     return 0;
   }
 
-  // Rows of {elements, workspace or output, the tensors of `ranks` ranks from `first` on}, or without ranks
-  // {elements, workspace} and {elements, output, workspace}.
+  // The end of the entries from `begin` on, at most `end`, whose addresses lie close enough together for 32-bit distances.
+  int within_reach(int begin, int end) const {
+    auto reach = [&](auto&& address, uint64_t unit) {  // of one base, and never short of the first entry with elements
+      uint64_t lo = ~0ull, hi = 0;
+      for (int e = begin; e < end; ++e) {
+        if (c_.counts[e] == 0) continue;
+        const uint64_t at = address(e);
+        lo = std::min(lo, at);
+        hi = std::max(hi, at);
+        if ((hi - lo) / unit > kMaxDistance) end = e;
+      }
+    };
+    reach([&](int e) { return (uint64_t)(uintptr_t)c_.outputs[e]; }, sizeof(D));
+    for (uint32_t r = 0; r < c_.world; ++r)
+      reach([&](int e) { return (uint64_t)(uintptr_t)c_.inputs[(size_t)r * (size_t)c_.n + (size_t)e]; }, sizeof(S));
+    uint64_t next = 0;
+    reach([&](int e) { const uint64_t at = next; next += up256((uint64_t)c_.counts[e] * sizeof(W)); return at; }, sizeof(W));
+    return end;
+  }
+
+  // Rows from the bases workspace or output and the tensors of `ranks` ranks from `first` on, or without ranks
+  // workspace alone and output and workspace.
   void fill(uint32_t first, uint32_t ranks, bool to_output) {
-    uint64_t* q = rows_.q;
-    uint64_t base = (uint64_t)(uintptr_t)ws_;
+    const bool work_too = to_output && ranks == 0;
+    const uint32_t bases = 1 + (work_too ? 1 : ranks);
+    const uint64_t work = (uint64_t)(uintptr_t)ws_;
+    uint64_t at[kMaxShortRows][1 + kRanksAtOnce];
+    uint64_t* base = rows_.base;
+    std::fill(base, base + bases, ~0ull);
+    l_.words = kRowHead - 1 + bases;
     uint32_t row = 0, chunks = 0;
+    uint64_t offset = 0;
     for (int e = g_.begin; e < g_.end; ++e) {
       const uint64_t count = (uint64_t)c_.counts[e];
       if (count == 0) continue;
+      at[row][0] = to_output ? (uint64_t)(uintptr_t)c_.outputs[e] : work + offset;
+      if (work_too) at[row][1] = work + offset;
+      for (uint32_t r = 0; r < ranks; ++r)
+        at[row][1 + r] = (uint64_t)(uintptr_t)c_.inputs[(size_t)(first + r) * (size_t)c_.n + (size_t)e];
+      for (uint32_t k = 0; k < bases; ++k) base[k] = std::min(base[k], at[row][k]);
+      uint32_t* d = rows_.d + row * l_.words;
+      d[1] = (uint32_t)count;
+      d[2] = (uint32_t)(count >> 32);
       rows_.first[row++] = chunks;
       chunks += (uint32_t)((count + kChunk<W> - 1) / kChunk<W>);
-      const uint64_t* start = q;
-      *q++ = count;
-      if (to_output) *q++ = (uint64_t)(uintptr_t)c_.outputs[e];
-      if (!to_output || ranks == 0) *q++ = base;
-      for (uint32_t r = first; r < first + ranks; ++r)
-        *q++ = (uint64_t)(uintptr_t)c_.inputs[(size_t)r * (size_t)c_.n + (size_t)e];
-      l_.words = (uint32_t)(q - start);
-      base += up256(count * sizeof(W));
+      offset += up256(count * sizeof(W));
     }
-    for (; row < kMaxRows; ++row) rows_.first[row] = ~0u;
+    for (uint32_t i = 0; i < row; ++i) {
+      uint32_t* d = rows_.d + i * l_.words;
+      d[0] = (uint32_t)((at[i][0] - base[0]) / (to_output ? sizeof(D) : sizeof(W)));
+      for (uint32_t k = 1; k < bases; ++k)
+        d[kRowHead - 1 + k] = (uint32_t)((at[i][k] - base[k]) / (work_too ? sizeof(W) : sizeof(S)));
+    }
+    for (; row < kMaxShortRows; ++row) rows_.first[row] = ~0u;
   }
 
   // Largest total of the ranks' tensors that the first pass leaves in the Infinity Cache whole: keeping all, half or
@@ -636,7 +691,7 @@ class Tree {
   unsigned char* ws_;
   Group g_;
   Level l_;
-  Rows rows_;
+  ShortRows rows_;
 };
 
 template <typename S, typename W, typename D>

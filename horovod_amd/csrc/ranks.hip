@@ -11,7 +11,7 @@
 // same order (to the wire type after the prescale and after every rank).
 //
 // There is no table in device memory.  A launch carries the addresses of up to 128 tensors
-// (what fits in 4 KiB of kernel arguments: 86 tensors of 8 ranks), a response of more is several
+// (what fits in 4 KiB of kernel arguments: 85 tensors of 8 ranks), a response of more is several
 // launches.  A table would have to be built and copied for every new set of addresses, and new
 // outputs are what an out-of-place call brings each time: with a cache of tables, BERT-large's
 // step spent 16 ms on rebuilding them whenever more sets rotated than it held.
@@ -93,31 +93,15 @@ __device__ __forceinline__ void add_ranks(Arr<W, N>& acc, uint32_t rank, uint32_
   if constexpr (B > 1) add_ranks<B / 2, W, N>(acc, rank, world, load, wire);
 }
 
-// The rows of up to eight ranks: addresses as 32-bit distances, in elements, from the lowest one of each rank (and of the
-// outputs), half the size of Rows', so that a launch carries up to 128 tensors (86 of eight ranks, where 64-bit addresses
-// leave room for 44).  Each launch more costs the stream 4 to 5 us between one's drain and the next one's start: of eight
-// ranks, ResNet-50's 161 gradients 153 -> 146.5 us, 320 tensors of 8 million elements in all 77 -> 62, 200 of 2 million
-// 47.5 -> 38.5.
-constexpr uint32_t kMaxShortRows = 128;  // two per lane of a wavefront
-constexpr uint32_t kShortWords = 864;
-struct ShortRows {
-  uint32_t first[kMaxShortRows];  // as in Rows
-  uint64_t base[9];               // outputs, rank 0, 1 ...
-  uint32_t d[kShortWords];        // per row: output, elements, rank 0, 1 ...
-};
-static_assert(sizeof(ShortRows) + 48 <= 4096, "kernel arguments");
-
-// What a workgroup needs of its row, of K ranks (more than eight: `world` of them).
+// What a workgroup needs of its row: of K ranks {output, elements, rank 0, 1 ...}, or of `world` ranks, more than eight.
+static_assert(sizeof(ShortRows) + 40 <= 4096, "kernel arguments");
 template <typename S, typename D, int K>
 struct ShortRow {
   const ShortRows& rows;
   const uint32_t* d;
   uint32_t row;
-  __device__ __forceinline__ ShortRow(const ShortRows& r, uint32_t nrows, uint32_t chunk, uint32_t) : rows(r), row(0) {
-    if (nrows > 1) {
-      const uint32_t lane = threadIdx.x & 63, low = r.first[lane], high = r.first[64 + lane];
-      row = (uint32_t)__popcll(__ballot(low <= chunk)) + (uint32_t)__popcll(__ballot(high <= chunk)) - 1;
-    }
+  __device__ __forceinline__ ShortRow(const ShortRows& r, uint32_t nrows, uint32_t chunk, uint32_t)
+      : rows(r), row(row_of(r, nrows, chunk)) {
     d = r.d + row * (K + 2);
   }
   __device__ __forceinline__ uint64_t elements() const { return d[1]; }
@@ -322,7 +306,7 @@ class ShortTable {
  public:
   explicit ShortTable(uint32_t) {}
   uint32_t rows() const { return n_; }
-  static uint64_t most(uint64_t tile) { return 0xffffffffull / tile * tile; }
+  static uint64_t most(uint64_t tile) { return kMaxDistance / tile * tile; }
   template <typename Input>
   bool add(uint32_t first, uint64_t output, uint64_t elements, Input&& input) {
     constexpr uint32_t max = std::min(kMaxShortRows, kShortWords / (K + 2));
@@ -334,7 +318,7 @@ class ShortTable {
     for (uint32_t r = 0; r <= K; ++r) {
       lo[r] = n_ ? std::min(lo_[r], at[r]) : at[r];
       hi[r] = n_ ? std::max(hi_[r], at[r]) : at[r];
-      if ((hi[r] - lo[r]) / (r ? IS : OS) > 0xffffffffull) return false;  // never the first row of a launch
+      if ((hi[r] - lo[r]) / (r ? IS : OS) > kMaxDistance) return false;  // never the first row of a launch
     }
     std::copy(lo, lo + K + 1, lo_);
     std::copy(hi, hi + K + 1, hi_);

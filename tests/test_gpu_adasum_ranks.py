@@ -1,6 +1,6 @@
 """hvdhip_adasum_ranks against the oracle's pairwise combine, level by level, at the edges of its chunks (16 KiB of
 the wire type), of the partial sums that a consumer adds itself (512 per tensor; "long" at 8 and 16 ranks has every
-level read the coefficients of the launch in between), of the tensors one launch carries (44 of eight ranks), of the
+level read the coefficients of the launch in between), of the tensors one launch carries (77 of eight ranks), of the
 ranks one launch reads (8) and of what the first pass leaves in the Infinity Cache (all ranks up to 160 MiB in
 total, of 16 "long" ones every other)."""
 import numpy as np
@@ -111,7 +111,7 @@ def test_short_rows_give_the_same_bits_in_one_launch(gpu, dtype, world, chunks, 
     counts = [1, 0, 16 // es - 1, 255 * 16 // es, 3 * 4096 // es + 5, chunk - 1, chunk, 7]
     if chunks == 2:
         counts += [chunk + 1, 2 * chunk - 1, 2 * chunk, chunk + 16 // es]
-    counts += [33 + i for i in range(44)]  # more than a launch carries; the long row below comes first of all
+    counts += [33 + i for i in range(100)]  # more than a launch carries; the long row below comes first of all
     gen = torch.Generator(device="cuda").manual_seed(world)
     kind = getattr(torch, dtype)
 
@@ -144,6 +144,33 @@ def test_short_rows_give_the_same_bits_in_one_launch(gpu, dtype, world, chunks, 
         assert torch.equal(alone[i].view(torch.uint8), want), (i, n)
         assert torch.equal(in_place[i][1:].view(torch.uint8), want[es:]), (i, n)
         assert torch.equal(in_place[i][:1].view(torch.uint8), ranks[0][i][:1].view(torch.uint8)), (i, n)
+
+
+@pytest.mark.parametrize("world", [2, 8])
+def test_rows_that_32_bits_do_not_span(gpu, world):
+    """Halves more than 2^32 elements apart, in a rank and then in the outputs: in groups of their own, with the bits
+    that the rows give close together; beside a row of three chunks, so that levels and workspace are used."""
+    code, far, n = DTYPE["float16"], (1 << 32) + 4096, 3 * 8192 + 5
+    gen = torch.Generator(device="cuda").manual_seed(world)
+    wide = torch.empty(far + n, dtype=torch.float16, device="cuda")
+    ends = [wide[:n], wide[far:], wide[n:2 * n]]
+    ranks = [[torch.empty(n, dtype=torch.float16, device="cuda").normal_(generator=gen) for _ in ends] for _ in range(world)]
+    need = H.adasum_ranks_workspace([n] * 3, world, code)
+    work = torch.empty(need, dtype=torch.uint8, device="cuda")
+
+    def run(outs, ins):
+        torch.cuda.synchronize()
+        assert H.adasum_ranks([o.data_ptr() for o in outs], [t.data_ptr() for r in ins for t in r], [n] * 3, world, code,
+                              code, code, 1.0, 1.0, work.data_ptr(), need, gpu.stream)
+        gpu.stream.synchronize()
+        return [o.clone() for o in outs]
+
+    want = run([torch.zeros_like(t) for t in ranks[0]], ranks)
+    for e, t in zip(ends, ranks[1]):
+        e.copy_(t)
+    for got in (run([torch.zeros_like(t) for t in ranks[0]], ranks[:1] + [ends] + ranks[2:]), run(ends, ranks)):
+        for g, w in zip(got, want):
+            assert torch.equal(g.view(torch.int16), w.view(torch.int16))
 
 
 def test_adasum_ranks_refuses(gpu):
