@@ -91,8 +91,10 @@ def _is_part(t, e):
 _BYTES_OF_ITS_OWN = 320 << 20
 
 # Cycles for which a framework stream that was found busy is waited for without another look.  A look costs 0.1 us at an
-# idle stream and saves the event and the wait, 15 us of host time; at a busy one it costs 6 us on top of them.
-_BUSY_CYCLES = 16
+# idle stream and saves the event and the wait, 15 us of host time for every response; at a busy one it costs 6 to 8 us on
+# top of them.  Few, so that a script whose stream is idle again soon has what the look saves, and more than none for one
+# that averages a value it has just computed.
+_BUSY_CYCLES = 4
 
 
 class Engine:
