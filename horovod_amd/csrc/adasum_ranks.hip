@@ -49,6 +49,7 @@ struct Level {
   uint32_t nrows;
   uint32_t chunks;
   uint32_t words;  // per row in ShortRows::d
+  uint32_t high;   // where in it the words of high bits start
   uint32_t first;  // pair (dots_k) or group of four vectors (level_k) that blockIdx.y = 0 works on
   uint32_t flags;
   uint64_t in_stride, out_stride;
@@ -58,19 +59,21 @@ struct Level {
   double* out_sums;
 };
 
-// A row: {distance from base[0], elements in two words, distances from base[1], base[2] ...}.
+// A row: {distance from base[0], elements in two words, distances from base[1], base[2] ...; wide_words() of them if they
+// are wide}.
 constexpr uint32_t kRowHead = 3;
 static_assert(sizeof(ShortRows) + sizeof(Level) <= 4096, "kernel arguments");
 
 struct Place {
   const uint32_t* d;
+  uint32_t high;  // where the row's words of high bits are
   uint32_t row, chunk;
   uint64_t elements, start;  // of the row; element within it
   uint32_t m;                // elements of this chunk
   // What base[k] is the lowest one of.
   template <typename T>
   __device__ __forceinline__ gptr<T> at(const ShortRows& rows, uint32_t k) const {
-    return as_global<T>(rows.base[k]) + (k == 0 ? d[0] : d[kRowHead - 1 + k]);
+    return as_global<T>(rows.base[k]) + distance(rows, d, k == 0 ? 0 : kRowHead - 1 + k, high, k);
   }
 };
 __device__ __forceinline__ uint64_t row_elements(const uint32_t* d) { return d[1] | (uint64_t)d[2] << 32; }
@@ -80,6 +83,7 @@ __device__ __forceinline__ Place place(const ShortRows& rows, const Level& l) {
   p.chunk = blockIdx.x;
   p.row = row_of(rows, l.nrows, p.chunk);
   p.d = rows.d + p.row * l.words;
+  p.high = l.high;
   p.elements = row_elements(p.d);
   p.start = (uint64_t)(p.chunk - rows.first[p.row]) * kChunk<W>;
   const uint64_t left = p.elements - p.start;
@@ -443,6 +447,7 @@ __global__ __launch_bounds__(G * kWG) void tree_held_k(Level l, ShortRows rows) 
   Place p;
   p.row = blockIdx.x;
   p.d = rows.d + p.row * l.words;
+  p.high = l.high;
   p.elements = row_elements(p.d);
   p.start = group * kChunk<W>;
   const uint32_t left = p.start < p.elements ? (uint32_t)(p.elements - p.start) : 0;
@@ -527,7 +532,7 @@ class Tree {
       int rc = next_group(c_.counts, last, at, c_.world, sizeof(W), &whole);
       if (rc) return rc;
       for (; at < whole.end; at = g_.end) {
-        rc = next_group(c_.counts, within_reach(at, whole.end), at, c_.world, sizeof(W), &g_);
+        rc = next_group(c_.counts, within_reach(at, whole.end, &wide_), at, c_.world, sizeof(W), &g_);
         if (rc) return rc;
         rc = group(g_.end == last ? c_.completion : nullptr);
         if (rc) return rc;
@@ -626,8 +631,22 @@ class Tree {
     return 0;
   }
 
-  // The end of the entries from `begin` on, at most `end`, whose addresses lie close enough together for 32-bit distances.
-  int within_reach(int begin, int end) const {
+  // The end of the entries from `begin` on, at most `end`, that a group of short or of wide distances reaches, whichever
+  // is further; of the wide ones fewer fit a launch's arguments.
+  int within_reach(int begin, int end, bool* wide) const {
+    const int narrow = within(begin, end, kShortReach);
+    *wide = false;
+    if (narrow == end) return end;
+    const uint32_t bases = 1 + std::min(c_.world, kRanksAtOnce);
+    uint32_t room = std::min(kMaxShortRows, kShortWords / (kRowHead - 1 + bases + wide_words(bases)));
+    int most = begin;
+    for (; most < end; ++most)
+      if (c_.counts[most] && room-- == 0) break;
+    const int far = within(begin, most, kWideReach);
+    *wide = far > narrow;
+    return std::max(far, narrow);
+  }
+  int within(int begin, int end, uint64_t most) const {
     auto reach = [&](auto&& address, uint64_t unit) {  // of one base, and never short of the first entry with elements
       uint64_t lo = ~0ull, hi = 0;
       for (int e = begin; e < end; ++e) {
@@ -635,7 +654,7 @@ class Tree {
         const uint64_t at = address(e);
         lo = std::min(lo, at);
         hi = std::max(hi, at);
-        if ((hi - lo) / unit > kMaxDistance) end = e;
+        if ((hi - lo) / unit > most) end = e;
       }
     };
     reach([&](int e) { return (uint64_t)(uintptr_t)c_.outputs[e]; }, sizeof(D));
@@ -655,7 +674,9 @@ class Tree {
     uint64_t at[kMaxShortRows][1 + kRanksAtOnce];
     uint64_t* base = rows_.base;
     std::fill(base, base + bases, ~0ull);
-    l_.words = kRowHead - 1 + bases;
+    l_.high = kRowHead - 1 + bases;
+    l_.words = l_.high + (wide_ ? wide_words(bases) : 0);
+    rows_.wide = wide_ ? 0xff : 0;
     uint32_t row = 0, chunks = 0;
     uint64_t offset = 0;
     for (int e = g_.begin; e < g_.end; ++e) {
@@ -675,9 +696,10 @@ class Tree {
     }
     for (uint32_t i = 0; i < row; ++i) {
       uint32_t* d = rows_.d + i * l_.words;
-      d[0] = (uint32_t)((at[i][0] - base[0]) / (to_output ? sizeof(D) : sizeof(W)));
+      std::fill(d + l_.high, d + l_.words, 0u);
+      set_distance(d, 0, l_.high, 0, (at[i][0] - base[0]) / (to_output ? sizeof(D) : sizeof(W)), wide_);
       for (uint32_t k = 1; k < bases; ++k)
-        d[kRowHead - 1 + k] = (uint32_t)((at[i][k] - base[k]) / (work_too ? sizeof(W) : sizeof(S)));
+        set_distance(d, kRowHead - 1 + k, l_.high, k, (at[i][k] - base[k]) / (work_too ? sizeof(W) : sizeof(S)), wide_);
     }
     for (; row < kMaxShortRows; ++row) rows_.first[row] = ~0u;
   }
@@ -691,6 +713,7 @@ class Tree {
   unsigned char* ws_;
   Group g_;
   Level l_;
+  bool wide_;  // the group's distances take more than 32 bits
   ShortRows rows_;
 };
 

@@ -26,19 +26,33 @@ __device__ __forceinline__ uint32_t row_of(const Rows& rows, uint32_t nrows, uin
   return (uint32_t)__popcll(__ballot(rows.first[threadIdx.x & 63] <= chunk)) - 1;
 }
 
-// The same for up to eight ranks with addresses as 32-bit distances, in elements, from the lowest one of each rank (and of
-// the outputs): half the size, so that a launch carries up to 128 tensors, 85 of eight ranks where 64-bit addresses leave
-// room for 44.  Each launch more costs the stream 4 to 5 us between one's drain and the next one's start: sums of eight
-// ranks, ResNet-50's 161 gradients 153 -> 146 us, 320 tensors of 8 million elements in all 77 -> 63, 200 of 2 million
-// 47 -> 38.
+// The same for up to eight ranks with addresses as distances, in elements, from the lowest one of each rank (and of the
+// outputs): 32 bits each, and where some are further apart 8 more, four to a word behind the row's others.  A launch
+// carries up to 128 tensors so, 84 of eight ranks (65 with the wide distances) where 64-bit addresses leave room for 44.
+// Each launch more costs the stream 4 to 5 us between one's drain and the next one's start: sums of eight ranks,
+// ResNet-50's 161 gradients 153 -> 146 us, 320 tensors of 8 million elements in all 77 -> 63, 200 of 2 million 47 -> 38.
+// (Two allocations of the framework's are easily 32 GiB apart: its small segments and its large ones.)
 constexpr uint32_t kMaxShortRows = 128;  // two per lane of a wavefront
-constexpr uint32_t kShortWords = 850;
+constexpr uint32_t kShortWords = 848;
 struct ShortRows {
   uint32_t first[kMaxShortRows];  // as in Rows
   uint64_t base[9];               // outputs, rank 0, 1 ...
-  uint32_t d[kShortWords];        // a few words per row, distances from the bases among them
+  uint32_t wide;                  // 0xff if the rows have the words with bits 32 to 39, else 0
+  uint32_t d[kShortWords + 3];    // a few words per row; the last three are there to be loaded, not used
 };
-constexpr uint64_t kMaxDistance = 0xffffffffull;
+constexpr uint64_t kShortReach = 0xffffffffull, kWideReach = 0xffffffffffull;  // largest distances
+constexpr uint32_t wide_words(uint32_t distances) { return (distances + 3) / 4; }
+
+// Distance k of a row: its low word is d[low], the words of high bits start at d[high].
+__device__ __forceinline__ uint64_t distance(const ShortRows& rows, const uint32_t* d, uint32_t low, uint32_t high,
+                                             uint32_t k) {
+  return d[low] | (uint64_t)(d[high + k / 4] >> k % 4 * 8 & rows.wide) << 32;
+}
+// The host's side of it: the row's words of high bits are zero before the first call.
+inline void set_distance(uint32_t* d, uint32_t low, uint32_t high, uint32_t k, uint64_t value, bool wide) {
+  d[low] = (uint32_t)value;
+  if (wide) d[high + k / 4] |= (uint32_t)(value >> 32) << k % 4 * 8;
+}
 
 __device__ __forceinline__ uint32_t row_of(const ShortRows& rows, uint32_t nrows, uint32_t chunk) {
   if (nrows <= 1) return 0;

@@ -11,7 +11,7 @@
 // same order (to the wire type after the prescale and after every rank).
 //
 // There is no table in device memory.  A launch carries the addresses of up to 128 tensors
-// (what fits in 4 KiB of kernel arguments: 85 tensors of 8 ranks), a response of more is several
+// (what fits in 4 KiB of kernel arguments: 84 tensors of 8 ranks), a response of more is several
 // launches.  A table would have to be built and copied for every new set of addresses, and new
 // outputs are what an out-of-place call brings each time: with a cache of tables, BERT-large's
 // step spent 16 ms on rebuilding them whenever more sets rotated than it held.
@@ -93,7 +93,8 @@ __device__ __forceinline__ void add_ranks(Arr<W, N>& acc, uint32_t rank, uint32_
   if constexpr (B > 1) add_ranks<B / 2, W, N>(acc, rank, world, load, wire);
 }
 
-// What a workgroup needs of its row: of K ranks {output, elements, rank 0, 1 ...}, or of `world` ranks, more than eight.
+// What a workgroup needs of its row: of K ranks {output, elements, rank 0, 1 ...; wide_words(K + 1) if they are wide}, or
+// of `world` ranks, more than eight.
 static_assert(sizeof(ShortRows) + 40 <= 4096, "kernel arguments");
 template <typename S, typename D, int K>
 struct ShortRow {
@@ -102,11 +103,13 @@ struct ShortRow {
   uint32_t row;
   __device__ __forceinline__ ShortRow(const ShortRows& r, uint32_t nrows, uint32_t chunk, uint32_t)
       : rows(r), row(row_of(r, nrows, chunk)) {
-    d = r.d + row * (K + 2);
+    d = r.d + row * (K + 2 + (r.wide ? wide_words(K + 1) : 0));
   }
   __device__ __forceinline__ uint64_t elements() const { return d[1]; }
-  __device__ __forceinline__ gptr<D> output() const { return as_global<D>(rows.base[0]) + d[0]; }
-  __device__ __forceinline__ gptr<const S> input(uint32_t r) const { return as_global<const S>(rows.base[1 + r]) + d[2 + r]; }
+  __device__ __forceinline__ gptr<D> output() const { return as_global<D>(rows.base[0]) + distance(rows, d, 0, K + 2, 0); }
+  __device__ __forceinline__ gptr<const S> input(uint32_t r) const {
+    return as_global<const S>(rows.base[1 + r]) + distance(rows, d, 2 + r, K + 2, 1 + r);
+  }
 };
 template <typename S, typename D>
 struct LongRow {
@@ -306,40 +309,53 @@ class ShortTable {
  public:
   explicit ShortTable(uint32_t) {}
   uint32_t rows() const { return n_; }
-  static uint64_t most(uint64_t tile) { return kMaxDistance / tile * tile; }
+  static uint64_t most(uint64_t tile) { return kShortReach / tile * tile; }
   template <typename Input>
   bool add(uint32_t first, uint64_t output, uint64_t elements, Input&& input) {
-    constexpr uint32_t max = std::min(kMaxShortRows, kShortWords / (K + 2));
-    if (n_ == max) return false;
+    constexpr uint32_t short_max = std::min(kMaxShortRows, kShortWords / (K + 2));
+    constexpr uint32_t wide_max = std::min(kMaxShortRows, kShortWords / (K + 2 + wide_words(K + 1)));
+    if (n_ == short_max || (wide_ && n_ == wide_max)) return false;
     uint64_t* at = at_[n_];
     at[0] = output;
     for (uint32_t r = 0; r < K; ++r) at[1 + r] = input(r);
     uint64_t lo[K + 1], hi[K + 1];
+    bool wide = wide_;
     for (uint32_t r = 0; r <= K; ++r) {
       lo[r] = n_ ? std::min(lo_[r], at[r]) : at[r];
       hi[r] = n_ ? std::max(hi_[r], at[r]) : at[r];
-      if ((hi[r] - lo[r]) / (r ? IS : OS) > kMaxDistance) return false;  // never the first row of a launch
+      const uint64_t span = (hi[r] - lo[r]) / (r ? IS : OS);  // 0 for the first row of a launch
+      if (span > kShortReach) wide = true;
+      if (span > kWideReach || (wide && n_ >= wide_max)) return false;
     }
+    wide_ = wide;
     std::copy(lo, lo + K + 1, lo_);
     std::copy(hi, hi + K + 1, hi_);
-    table_.d[n_ * (K + 2) + 1] = (uint32_t)elements;
+    elements_[n_] = (uint32_t)elements;
     table_.first[n_++] = first;
     return true;
   }
   const ShortRows& finished() {
+    constexpr uint32_t high = K + 2;
+    const uint32_t words = high + (wide_ ? wide_words(K + 1) : 0);
     for (uint32_t i = 0; i < n_; ++i) {
-      uint32_t* d = table_.d + i * (K + 2);
-      d[0] = (uint32_t)((at_[i][0] - lo_[0]) / OS);
-      for (uint32_t r = 0; r < K; ++r) d[2 + r] = (uint32_t)((at_[i][1 + r] - lo_[1 + r]) / IS);
+      uint32_t* d = table_.d + i * words;
+      std::fill(d + high, d + words, 0u);
+      d[1] = elements_[i];
+      set_distance(d, 0, high, 0, (at_[i][0] - lo_[0]) / OS, wide_);
+      for (uint32_t r = 0; r < K; ++r) set_distance(d, 2 + r, high, 1 + r, (at_[i][1 + r] - lo_[1 + r]) / IS, wide_);
     }
     std::copy(lo_, lo_ + K + 1, table_.base);
+    table_.wide = wide_ ? 0xff : 0;
     for (uint32_t i = n_; i < kMaxShortRows; ++i) table_.first[i] = ~0u;
     n_ = 0;
+    wide_ = false;
     return table_;
   }
 
  private:
   uint32_t n_ = 0;
+  bool wide_ = false;
+  uint32_t elements_[kMaxShortRows];
   uint64_t lo_[K + 1], hi_[K + 1], at_[kMaxShortRows][K + 1];
   ShortRows table_;
 };

@@ -147,20 +147,21 @@ def test_short_rows_give_the_same_bits_in_one_launch(gpu, dtype, world, chunks, 
 
 
 @pytest.mark.parametrize("world", [2, 8])
-def test_rows_that_32_bits_do_not_span(gpu, world):
-    """Halves more than 2^32 elements apart, in a rank and then in the outputs: in groups of their own, with the bits
-    that the rows give close together; beside a row of three chunks, so that levels and workspace are used."""
-    code, far, n = DTYPE["float16"], (1 << 32) + 4096, 3 * 8192 + 5
+@pytest.mark.parametrize("count,n", [(3, 3 * 8192 + 5), (100, 3 * 8192 + 5), (100, 1000)])
+def test_rows_that_32_bits_do_not_span(gpu, world, count, n):
+    """Halves more than 2^32 elements apart in turn, in a rank and then in the outputs: the bits that the rows give close
+    together.  More rows than a launch carries with such distances, through the levels and in one launch."""
+    code, far = DTYPE["float16"], 1 << 32
     gen = torch.Generator(device="cuda").manual_seed(world)
-    wide = torch.empty(far + n, dtype=torch.float16, device="cuda")
-    ends = [wide[:n], wide[far:], wide[n:2 * n]]
+    wide = torch.empty(far + count * n, dtype=torch.float16, device="cuda")
+    ends = [wide[i * n:(i + 1) * n] if i % 2 else wide[far + i * n:far + (i + 1) * n] for i in range(count)]
     ranks = [[torch.empty(n, dtype=torch.float16, device="cuda").normal_(generator=gen) for _ in ends] for _ in range(world)]
-    need = H.adasum_ranks_workspace([n] * 3, world, code)
+    need = H.adasum_ranks_workspace([n] * count, world, code)
     work = torch.empty(need, dtype=torch.uint8, device="cuda")
 
     def run(outs, ins):
         torch.cuda.synchronize()
-        assert H.adasum_ranks([o.data_ptr() for o in outs], [t.data_ptr() for r in ins for t in r], [n] * 3, world, code,
+        assert H.adasum_ranks([o.data_ptr() for o in outs], [t.data_ptr() for r in ins for t in r], [n] * count, world, code,
                               code, code, 1.0, 1.0, work.data_ptr(), need, gpu.stream)
         gpu.stream.synchronize()
         return [o.clone() for o in outs]
