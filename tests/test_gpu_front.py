@@ -102,6 +102,23 @@ def test_work_of_a_busy_stream_is_waited_for(hvd, stream, peers):
         other.synchronize()
 
 
+@pytest.mark.parametrize("n", [1, 1000, 1 << 20, 5 << 20])
+def test_what_an_idle_stream_has_written_is_read(hvd, n):
+    """Without an event between the two streams: tensors that the sum has read before, so that its caches may hold them,
+    rewritten on the framework's stream, which is then only polled until it has nothing left."""
+    x, y = (torch.zeros(n, device="cuda") for _ in range(2))
+    hvd.init(size=3, peer_source=lambda rank, name, t: y)
+    out = torch.empty_like(x)
+    stream = torch.cuda.current_stream()
+    for i in range(200):
+        x.fill_(i)
+        y.fill_(3 * i)
+        while not stream.query():
+            pass
+        out = hvd.synchronize(hvd.allreduce_async(x, name="t", op=hvd.Sum))
+        assert float(out.min()) == float(out.max()) == 7 * i, i
+
+
 def test_idle_is_said_of_idle_streams_only():
     L = horovod_amd.lib()
 
