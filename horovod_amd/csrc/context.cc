@@ -321,17 +321,15 @@ int hvdhip_stream_idle(void* stream, int* idle) {
   if (!idle) return fail(HVDHIP_ERR_INVALID_ARGUMENT, "idle is NULL");
   *idle = 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  HVDHIP_CHECK(hipStreamIsCapturing(s, &capture));
-  if (capture != hipStreamCaptureStatusNone) return ok();  // a query would end the capture
   const hipError_t before = hipPeekAtLastError();
-  const hipError_t e = hipStreamQuery(s);
-  if (e == hipErrorNotReady) {
-    if (before == hipSuccess) (void)hipGetLastError();  // not an error: leave none behind
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const bool may_ask = hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+  if (may_ask && hipStreamQuery(s) == hipSuccess) {  // a query would end the stream's capture
+    *idle = 1;
     return ok();
   }
-  HVDHIP_CHECK(e);
-  *idle = 1;
+  // Busy, or nothing that can be said (another thread's capture forbids the question): an event will tell.
+  if (before == hipSuccess) (void)hipGetLastError();  // leave no error of this call's behind
   return ok();
 }
 
