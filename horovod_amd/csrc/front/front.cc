@@ -534,6 +534,19 @@ PyTypeObject state_type = type_of<State>("horovod_amd.torch._front.State", nullp
 
 // ---- a cycle -------------------------------------------------------------------------------------
 
+// take(queue): a list of what the queue holds, which is empty then.  One step for the threads that append to it: nothing
+// between the two copies allocates an object or runs Python code, so the interpreter changes no threads there.
+PyObject* take(PyObject*, PyObject* queue) {
+  if (!PyList_CheckExact(queue)) {
+    PyErr_SetString(PyExc_TypeError, "the queue is a list");
+    return nullptr;
+  }
+  Ref taken(PyList_New(0));
+  if (!taken || PyList_SetSlice(taken.get(), 0, 0, queue) || PyList_SetSlice(queue, 0, PyList_GET_SIZE(queue), nullptr))
+    return nullptr;
+  return taken.release();
+}
+
 typedef int (*Fuse)(const int64_t* sizes, const int* keys, int n, int64_t threshold, int unpadded, int* group_of);
 
 // plan(requests, padded, threshold, address of hvd_adapter_fuse_keyed): the fused responses, each a list of (request,
@@ -837,7 +850,8 @@ PyObject* places(PyObject*, PyObject* args) {
   });
 }
 
-PyMethodDef methods[] = {{"plan", plan, METH_VARARGS, nullptr},
+PyMethodDef methods[] = {{"take", take, METH_O, nullptr},
+                         {"plan", plan, METH_VARARGS, nullptr},
                          {"addresses", addresses, METH_VARARGS, nullptr},
                          {"requests", requests, METH_O, nullptr},
                          {"attach", attach, METH_VARARGS, nullptr},

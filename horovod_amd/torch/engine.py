@@ -160,8 +160,7 @@ class Engine:
     def run_cycle(self):
         """Fuses and queues everything enqueued so far (one pass of RunLoopOnce,
         common/operations.cc:593-717, with every request already agreed upon)."""
-        pending = list(self.queue)
-        self.queue.clear()
+        pending = _front.take(self.queue)  # other threads may be enqueuing
         if not pending:
             return
         self.cycles += 1

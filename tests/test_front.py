@@ -45,6 +45,14 @@ def test_a_cycle_fuses_by_bytes_on_the_wire(front, wire, es, padded):
     assert all(requests[int(e.name)] is r for g in groups for r, e in g)
 
 
+def test_a_queue_is_emptied_into_the_list_that_is_taken(front):
+    queue = [_request(front, [_entry(front, str(i), 1)]) for i in range(3)]
+    want = list(queue)
+    assert front.take(queue) == want and queue == [] and front.take(queue) == []
+    with pytest.raises(TypeError):
+        front.take(tuple(want))
+
+
 def test_requests_of_different_kinds_do_not_share_a_response(front):
     variants = [{}, {"op": 2}, {"prescale": 0.25}, {"postscale": 1.0}, {"wire_dtype": F16}, {"tensor_dtype": 4, "wire_dtype": 4},
                 {"device": 1}, {"kind": "allgather"}]
