@@ -119,6 +119,7 @@ struct Request {
   PyObject* objects[kObjects];
   int op, tensor_dtype, wire_dtype;
   double prescale, postscale;
+  Py_ssize_t left;  // entries whose response has not been executed
   char submitted, grouped;
 };
 PyMemberDef request_members[] = {
@@ -147,6 +148,7 @@ Request* new_request(PyTypeObject* type, PyObject* entries, PyObject* device, Py
   r->objects[Request::entries] = borrowed(entries);
   r->objects[Request::device] = borrowed(device);
   r->objects[Request::markers] = markers.release();
+  r->left = PyList_GET_SIZE(entries);
   return r;
 }
 PyObject* request_new(PyTypeObject* type, PyObject* args, PyObject* kwargs) {
@@ -740,6 +742,19 @@ PyObject* requests(PyObject*, PyObject* group) {
   });
 }
 
+// executed(group): the response has been queued, or has failed; a request is submitted with the last of its responses.
+PyObject* executed(PyObject*, PyObject* group) {
+  if (!is_group(group)) {
+    PyErr_SetString(PyExc_TypeError, "a group is a list of (request, entry)");
+    return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(group); ++i) {
+    Request* r = as_request(PyTuple_GET_ITEM(PyList_GET_ITEM(group, i), 0));
+    if (--r->left == 0) r->submitted = 1;
+  }
+  Py_RETURN_NONE;
+}
+
 // attach(requests, marker): the marker of the response that carries an entry of each.
 PyObject* attach(PyObject*, PyObject* args) {
   PyObject *list, *marker;
@@ -854,6 +869,7 @@ PyMethodDef methods[] = {{"take", take, METH_O, nullptr},
                          {"plan", plan, METH_VARARGS, nullptr},
                          {"addresses", addresses, METH_VARARGS, nullptr},
                          {"requests", requests, METH_O, nullptr},
+                         {"executed", executed, METH_O, nullptr},
                          {"attach", attach, METH_VARARGS, nullptr},
                          {"parts", parts, METH_VARARGS, nullptr},
                          {"places", places, METH_VARARGS, nullptr},

@@ -22,6 +22,7 @@ so too, a pass per level of the pairwise tree; only where a node has several ran
 a buffer per node first.
 """
 import ctypes
+import threading
 from ctypes import c_int, c_void_p
 
 import torch
@@ -107,6 +108,10 @@ class Engine:
         self.batch_d2d_memcopies = bool(batch_d2d_memcopies)
         self.streams = [H.Stream() for _ in range(max(1, num_streams))]
         self.slot = 0
+        # Held for a whole cycle: the slots, their buffers and events are one thread's at a time, and whoever waits for a
+        # request that another thread's cycle has taken waits for that cycle first.  Again by the same thread where
+        # peer_source calls back.
+        self.cycling = threading.RLock()
         self.queue = []
         self.inflight = {}       # tensor name -> request, until synchronised
         self.buffers = {}        # (slot, what for) -> torch uint8 tensor
@@ -160,24 +165,29 @@ class Engine:
     def run_cycle(self):
         """Fuses and queues everything enqueued so far (one pass of RunLoopOnce,
         common/operations.cc:593-717, with every request already agreed upon)."""
-        pending = _front.take(self.queue)  # other threads may be enqueuing
-        if not pending:
-            return
-        self.cycles += 1
-        self.ready = {}
-        fuse = ctypes.cast(adapter_lib().hvd_adapter_fuse_keyed, c_void_p).value
-        groups = _front.plan(pending, self.batch_d2d_memcopies, self.fusion_threshold, fuse)
-        for g in groups:
+        with self.cycling:
+            pending = _front.take(self.queue)  # other threads may be enqueuing
+            if not pending:
+                return
+            self.cycles += 1
+            self.ready = {}
             try:
-                if g[0][0].kind == "allgather":
-                    self._execute_allgather(g)
-                else:
-                    self._execute(g)
-            except Exception as exc:  # surfaces in synchronize(), like a Status passed to the callback
-                for r, _ in g:
-                    r.error = exc
-        for r in pending:
-            r.submitted = True
+                fuse = ctypes.cast(adapter_lib().hvd_adapter_fuse_keyed, c_void_p).value
+                for g in _front.plan(pending, self.batch_d2d_memcopies, self.fusion_threshold, fuse):
+                    try:
+                        if g[0][0].kind == "allgather":
+                            self._execute_allgather(g)
+                        else:
+                            self._execute(g)
+                    except Exception as exc:  # surfaces in synchronize(), like a Status passed to the callback
+                        for r, _ in g:
+                            r.error = exc
+                    _front.executed(g)
+            except BaseException as exc:  # an interrupt: the rest is not executed
+                for r in pending:
+                    if not r.submitted:
+                        r.error, r.submitted = exc, True
+                raise
 
     # ---- resources ------------------------------------------------------
 
@@ -396,7 +406,14 @@ class Engine:
 
     def poll(self, request):
         if not request.submitted:
-            self.run_cycle()
+            if not self.cycling.acquire(blocking=False):
+                return False  # in another thread's cycle, or in the next
+            try:
+                self.run_cycle()
+            finally:
+                self.cycling.release()
+            if not request.submitted:
+                return False  # asked from within its own cycle
         if request.error is not None:
             return True
         for m in request.markers:
@@ -409,6 +426,8 @@ class Engine:
     def wait(self, request):
         if not request.submitted:
             self.run_cycle()
+            if not request.submitted:  # still in flight, and the tensor as it was
+                raise HorovodInternalError("An operation cannot be waited for from within its own cycle before its response.")
         try:
             for m in request.markers:
                 if not m.done:

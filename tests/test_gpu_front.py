@@ -2,6 +2,7 @@
 and give the same, work of busy streams is waited for whether or not the engine looks, and nothing is left behind."""
 import ctypes
 import gc
+import threading
 
 import pytest
 import torch
@@ -198,3 +199,37 @@ def test_behind_a_large_response_a_cycle_keeps_its_stream(hvd, monkeypatch):
         for h, t in zip(handles, tensors):
             assert torch.equal(hvd.synchronize(h), 2 * t)
     assert slots == [0, 1, 0] + [1, 0, 0, 0, 0] + [0] + [1]
+
+
+def test_threads_share_the_engine(hvd):
+    """Two threads on streams of their own hand over and wait: Adasum of several ranks, whose levels go through a workspace
+    of the stream slot, sums and allgathers.  Each gets what it gets alone, whichever thread's cycle executes it."""
+    hvd.init(size=8, peer_source=lambda rank, name, t: t * (1 + rank % 3))
+    torch.manual_seed(1)
+    sets = [[torch.randn(n, device="cuda") for n in (300000, 5, 70001, 40000)] for _ in range(2)]
+
+    def step(tensors, tag):
+        handles = [hvd.grouped_allreduce_async(tensors, name=tag + "a", op=hvd.Adasum), hvd.allreduce_async(tensors[0], name=tag + "s"),
+                   hvd.allgather_async(tensors[2], name=tag + "g")]
+        adasum, total, rows = [hvd.synchronize(h) for h in reversed(handles)][::-1]
+        return adasum + [total, rows]
+
+    want = [step(tensors, "alone") for tensors in sets]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(which):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for i in range(60):
+                    got = step(sets[which], "%d.%d" % (which, i))
+                    wrong.extend((which, i, k) for k, (g, w) in enumerate(zip(got, want[which])) if not torch.equal(g, w))
+        except Exception as e:
+            wrong.append((which, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(w,)) for w in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
