@@ -297,11 +297,13 @@ PyObject* current_producer(State* s) {
   return borrowed(known);
 }
 
-// The counter in a list of one; false with an error set.
-bool count_up(PyObject* counter, long long* value) {
+// What the counter in a list of one comes to next; counted() moves it there.  False with an error set.
+bool next_of(PyObject* counter, long long* value) {
   *value = PyLong_AsLongLong(PyList_GET_ITEM(counter, 0)) + 1;
-  if (PyErr_Occurred()) return false;
-  PyObject* next = PyLong_FromLongLong(*value);
+  return !PyErr_Occurred();
+}
+bool counted(PyObject* counter, long long value) {
+  PyObject* next = PyLong_FromLongLong(value);
   return next && PyList_SetItem(counter, 0, next) == 0;
 }
 
@@ -383,7 +385,7 @@ PyObject* enqueue(State* s, PyObject* entries, const at::Tensor& first, const Ca
   r->objects[Request::producer] = current_producer(s);
   if (!r->objects[Request::producer]) return nullptr;
   long long handle;
-  if (!count_up(s->objects[State::next_handle], &handle)) return nullptr;
+  if (!next_of(s->objects[State::next_handle], &handle) || !counted(s->objects[State::next_handle], handle)) return nullptr;
   Ref h(PyLong_FromLongLong(handle));
   if (!h) return nullptr;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(entries); ++i) {
@@ -410,19 +412,19 @@ PyObject* state_submit(PyObject* self, PyObject* const* args, Py_ssize_t nargs) 
     Call c;
     if (!t || !fits(*t, t, o) || !call_of(s, *t, args[3], args[4], args[5], args[6], &c)) Py_RETURN_NONE;
     Ref full;
+    long long unnamed = 0;
     if (name != Py_None) {
       if (!PyUnicode_CheckExact(name)) Py_RETURN_NONE;
       full = Ref(PyUnicode_FromFormat("allreduce.%U", name));
-      if (!full) return nullptr;
-      const int there = PyDict_Contains(s->objects[State::inflight], full.get());
-      if (there < 0) return nullptr;
-      if (there) Py_RETURN_NONE;
     } else {
-      long long n;
-      if (!count_up(s->objects[State::noname], &n)) return nullptr;
-      full = Ref(PyUnicode_FromFormat("allreduce.noname.%lld", n));
-      if (!full) return nullptr;
+      if (!next_of(s->objects[State::noname], &unnamed)) return nullptr;
+      full = Ref(PyUnicode_FromFormat("allreduce.noname.%lld", unnamed));
     }
+    if (!full) return nullptr;
+    const int there = PyDict_Contains(s->objects[State::inflight], full.get());
+    if (there < 0) return nullptr;
+    if (there) Py_RETURN_NONE;  // before the name is counted, which Python does
+    if (unnamed && !counted(s->objects[State::noname], unnamed)) return nullptr;
     Ref entries(PyList_New(1));
     if (!entries) return nullptr;
     PyObject* entry = new_entry(full.get(), args[0], args[1], *t);

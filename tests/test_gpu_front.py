@@ -65,6 +65,22 @@ def test_a_group_is_summed_whatever_its_tensors_are(hvd, odd):
         hvd.grouped_allreduce_async([tensors[0], tensors[1].double()])
 
 
+def test_an_unnamed_tensor_does_not_take_a_name_in_flight(hvd):
+    """Unnamed tensors are numbered; one that a script has named like the next of them is in its way until it is finished."""
+    from horovod_amd.torch import mpi_ops
+    hvd.init(size=2)
+    for kind in (KINDS["plain"], KINDS["subclass"]):  # both ways in
+        t = kind(torch.arange(100, dtype=torch.float32, device="cuda"))
+        taken = hvd.allreduce_async(t, name="noname.%d" % (mpi_ops._noname[0] + 1), op=hvd.Sum)
+        with pytest.raises(hvd.HorovodInternalError, match="same name"):
+            hvd.allreduce_async(t, op=hvd.Sum)
+        assert len(mpi_ops._engine.inflight) == 1
+        later = hvd.allreduce_async(t, op=hvd.Sum)  # the next number
+        for h in (later, taken):
+            assert torch.equal(hvd.synchronize(h).as_subclass(torch.Tensor), 2 * t.as_subclass(torch.Tensor))
+        assert not mpi_ops._engine.inflight
+
+
 @pytest.mark.parametrize("wrong", [lambda t: t.double(), lambda t: t[:-1], lambda t: t.cpu(), lambda t: None,
                                    lambda t: torch.stack([t, t], 1)[:, 0], lambda t: t.double().as_subclass(Sub)])
 def test_a_peer_that_does_not_fit_is_an_error_of_its_response(hvd, wrong):
