@@ -249,3 +249,31 @@ def test_threads_share_the_engine(hvd):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("peers", [True, False])
+def test_the_null_stream_is_busy_with_a_blocking_one(hvd, peers):
+    """An event on the null stream lies behind all that blocking streams, as other libraries make them, hold by then.  The
+    look at the null stream has to say the same, or a tensor written there is read too early."""
+    L = horovod_amd.lib()
+    handle, idle = ctypes.c_void_p(), ctypes.c_int(-1)
+    assert L.hipStreamCreateWithFlags(ctypes.byref(handle), 0) == 0  # of the HIP runtime below the library
+    other = torch.cuda.ExternalStream(handle.value)
+    x, y = (torch.zeros(1 << 16, device="cuda") for _ in range(2))
+    hvd.init(size=2, peer_source=(lambda rank, name, t: y) if peers else None)
+    torch.cuda.synchronize()
+    assert torch.cuda.current_stream().cuda_stream == 0
+    for i in range(1, 21):
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(2000000)
+            x.fill_(i)
+            y.fill_(2 * i)
+        if i % 6 == 1:  # the engine looks, too: it takes a stream that it found busy to be so for four cycles
+            check(L.hvdhip_stream_idle(None, ctypes.byref(idle)), "hvdhip_stream_idle")
+            assert idle.value == 0
+        out = hvd.synchronize(hvd.allreduce_async(x, op=hvd.Sum))
+        assert float(out[0]) == float(out[-1]) == (3 * i if peers else 2 * i), i
+        torch.cuda.synchronize()
+    check(L.hvdhip_stream_idle(None, ctypes.byref(idle)), "hvdhip_stream_idle")
+    assert idle.value == 1
+    assert L.hipStreamDestroy(handle) == 0
