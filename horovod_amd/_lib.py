@@ -1,6 +1,7 @@
 """ctypes binding of libhvdhip.so: one prototype per function of include/hvdhip.h."""
 import ctypes
 import os
+import sys
 from ctypes import (POINTER, c_char_p, c_double, c_float, c_int, c_int64, c_size_t,
                     c_uint, c_uint64, c_void_p)
 
@@ -145,6 +146,17 @@ def adapter_lib():
 _front = None
 
 
+def front_for():
+    """The torch and the interpreter that lib/_front.so is built for: it reads torch's objects inline.  Known without
+    importing torch, for the build."""
+    import importlib.util
+    import runpy
+    import sysconfig
+    torch = importlib.util.find_spec("torch")
+    version = runpy.run_path(os.path.join(os.path.dirname(torch.origin), "version.py"))
+    return ",".join((version["__version__"], str(version.get("git_version")), str(sysconfig.get_config_var("SOABI"))))
+
+
 def front():
     """lib/_front.so: the per-tensor part of horovod_amd.torch, an extension module over torch's own headers."""
     global _front
@@ -156,6 +168,13 @@ def front():
     if not os.path.exists(path):
         raise RuntimeError("%s is missing: build it with `make -C horovod_amd/csrc`; "
                            "there is no fallback path" % path)
+    try:
+        built_for = ctypes.string_at(ctypes.addressof(ctypes.c_char.in_dll(ctypes.CDLL(path), "hvd_front_built_for"))).decode()
+    except (OSError, ValueError) as e:
+        built_for = str(e)
+    if built_for != front_for():
+        raise RuntimeError("%s is not built for this torch and interpreter (%s, here %s): build it again with "
+                           "`make -C horovod_amd/csrc PYTHON=%s`" % (path, built_for, front_for(), sys.executable))
     spec = importlib.util.spec_from_file_location("horovod_amd.torch._front", path)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)

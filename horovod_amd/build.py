@@ -2,6 +2,7 @@
 end's extension module, gcc for the C99 example client)."""
 import os
 import subprocess
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
@@ -9,7 +10,7 @@ CSRC = os.path.join(_HERE, "csrc")
 
 def build(force=False, jobs=8):
     """Runs make in csrc/; force=True rebuilds everything."""
-    cmd = ["make", "-j%d" % jobs, "-C", CSRC]
+    cmd = ["make", "-j%d" % jobs, "-C", CSRC, "PYTHON=%s" % (sys.executable or "python3")]  # the front end is this one's
     if force:
         cmd.insert(1, "-B")
     subprocess.check_call(cmd)

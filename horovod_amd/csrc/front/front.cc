@@ -16,6 +16,12 @@
 #include <unordered_set>
 #include <vector>
 
+// What this was built for, as _lib.front_for() says it; read before the module is imported.
+extern "C" {
+extern const char hvd_front_built_for[];
+const char hvd_front_built_for[] = HVD_FRONT_FOR;
+}
+
 namespace {
 
 // Owned reference.

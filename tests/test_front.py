@@ -1,12 +1,14 @@
 """The native half of the torch front end without a GPU: the records of a request, the fusion of a cycle, completion,
 and what it hands back to Python."""
 import ctypes
+import os
 import random
+import sys
 
 import pytest
 import torch
 
-from horovod_amd import _lib
+from horovod_amd import _lib, build
 from horovod_amd import workloads as W
 
 F32, F16 = 7, 6
@@ -133,3 +135,26 @@ def test_what_is_not_plain_goes_back_to_python(front):
     for bad in ([], [1], [(1, 2)]):
         with pytest.raises(TypeError):
             front.addresses(bad, 1, None, print)
+
+
+def test_a_module_built_for_another_torch_or_interpreter_is_not_imported(front, monkeypatch, tmp_path):
+    here = _lib.front_for()
+    assert here.startswith(torch.__version__ + ",") and "cpython-%d%d" % sys.version_info[:2] in here
+    monkeypatch.setattr(_lib, "_front", None)
+    monkeypatch.setattr(_lib, "front_for", lambda: "2.0.0,other,cpython-30")
+    with pytest.raises(RuntimeError, match="not built for this torch and interpreter"):
+        _lib.front()
+    monkeypatch.undo()
+    monkeypatch.setattr(_lib, "_front", None)
+    monkeypatch.setattr(_lib, "_HERE", str(tmp_path))
+    os.mkdir(tmp_path / "lib")
+    (tmp_path / "lib" / "_front.so").write_bytes(b"from before it said so")
+    with pytest.raises(RuntimeError, match="not built for this torch and interpreter"):
+        _lib.front()
+
+
+def test_the_build_is_for_the_interpreter_that_asks(monkeypatch):
+    commands = []
+    monkeypatch.setattr(build.subprocess, "check_call", commands.append)
+    build.build()
+    assert "PYTHON=" + sys.executable in commands[0]
