@@ -679,7 +679,6 @@ PyObject* addresses(PyObject*, PyObject* args) {
     const Py_ssize_t n = PyList_GET_SIZE(group);
     std::vector<uint64_t> inputs((size_t)n), outputs((size_t)n);
     std::vector<int64_t> counts((size_t)n);
-    std::vector<PyObject*> held;  // entries, for the calls below
     const at::Tensor* first = plain(entry_at(group, 0)->objects[Entry::tensor]);
     for (Py_ssize_t i = 0; i < n; ++i) {
       Entry* e = entry_at(group, i);

@@ -108,6 +108,7 @@ def test_completion_waits_for_every_marker_and_releases_an_event_once(front):
 
 
 def test_what_is_not_plain_goes_back_to_python(front):
+    """No tensor of the host is; those of the device are told apart in test_gpu_front.py."""
     handles, queue = {}, []
     state = front.State(2, 1, {}, queue, handles, [0], [0], print)
     t = torch.zeros(4)

@@ -41,6 +41,50 @@ def test_every_kind_of_tensor_is_summed(hvd, own, peer):
         [torch.full((10, 100), float(r), device="cuda") for r in (1, 2)]))
 
 
+def test_what_is_not_the_plain_case_is_not_submitted_natively():
+    """Whatever the native half hands back reaches the checks in Python; it leaves nothing behind then."""
+    handles, queue, inflight, next_handle, noname = {}, [], {}, [0], [0]
+    state = front().State(6, 2, inflight, queue, handles, next_handle, noname, print)
+    t = torch.zeros(4, 6, device="cuda")
+    plain = dict(tensor=t, output=torch.zeros_like(t), name=None, op=1, pre=1.0, post=1.0, wire=None)
+
+    def submitted(**changed):
+        a = {**plain, **changed}
+        rest = (a["op"], a["pre"], a["post"], a["wire"])
+        one = state.submit(a["tensor"], a["output"], a["name"], *rest)
+        group = state.submit_group([t, a["tensor"]], [t, a["output"]], str(a["name"]), *rest)
+        return one, group
+
+    wrapped = []
+
+    def inside(x):
+        wrapped.append(submitted(tensor=x, output=x))
+        return x.sum()
+
+    torch.func.vmap(inside)(t)
+    torch.func.grad(inside)(t)
+    functional = torch._to_functional_tensor(t)
+    nested = torch.nested.nested_tensor([t[0], t[1]])
+    refused = [submitted(tensor=x, output=x) for x in (
+        t.as_subclass(Sub), t.to_sparse(), t.t(), t[:, ::2], functional, nested, t.cpu(), t.to(torch.bfloat16), None)]
+    refused += [submitted(output=x) for x in (
+        torch.zeros(6, 4, device="cuda"), t.double(), t.cpu(), torch.zeros(6, 4, device="cuda").t(), t.as_subclass(Sub), None)]
+    refused += [submitted(op=x) for x in (3, -1, 1 << 70, True, 1.0, None, 2)]  # Adasum of three nodes, too
+    refused += [submitted(**{k: x}) for k in ("pre", "post") for x in (True, 1 << 60, "1", None, torch.tensor(1.0))]
+    refused += [submitted(wire=x) for x in (torch.bfloat16, "fp16", 6)]
+    assert len(wrapped) == 2 and all(r == (None, None) for r in wrapped + refused), refused
+    assert state.submit(t, t, 7, 1, 1.0, 1.0, None) is None
+    assert state.submit_group([t, t.double()], [t, t], "x", 1, 1.0, 1.0, None) is None
+    assert state.submit_group([t], [t, t], "x", 1, 1.0, 1.0, None) is None
+    assert not handles and not queue and not inflight and next_handle == noname == [0]
+    for i, changed in enumerate((dict(name="x"), dict(output=t), dict(op=0, pre=2, wire=torch.float16),
+                                 dict(tensor=torch.nn.Parameter(t), name="y"))):
+        assert submitted(**changed) == (2 * i + 1, 2 * i + 2)
+        assert submitted(**{**plain, "name": "x"}) == (None, None)  # in flight
+        inflight.pop("None_1of2", None), inflight.pop("None_2of2", None)
+    assert sorted(handles) == list(range(1, 9)) and queue == list(handles.values()) and noname == [2]
+
+
 @pytest.mark.parametrize("odd", [None, 0, 1, 2])
 def test_a_group_is_summed_whatever_its_tensors_are(hvd, odd):
     """One that is no plain tensor takes the whole group through Python; the names and results are the same."""
