@@ -377,8 +377,9 @@ struct Held {
 // The whole combine of layers that fit the registers of a workgroup, one workgroup each: both vectors are read once,
 // kept while the sums go through LDS, and written from there: three vectors of traffic in one launch instead of five in
 // two.  G groups of 256 lanes have C chunks each.  Bound by the chain of one workgroup (load, sums, two trips through
-// LDS and lanes, divide, store: about 3 us with the launch) where the device holds all of them, by memory beyond: 61 fp16
-// layers of a few hundred to 19,000 elements 6.4 -> 4.4 us, 1,000 fp32 layers of 16 KB 13.7 -> 9.5.
+// LDS and lanes, divide, store: about 3 us with the launch) where the device holds all of them, by memory beyond: call
+// after call, 61 fp16 layers of a few hundred to 19,000 elements 7.8 -> 4.6 us (the kernel traced alone 5.0), 1,000 fp32
+// layers of 16 KB 13.7 -> 9.5.
 template <typename T, int G, int C>
 __global__ __launch_bounds__(G * kWG) void combine_held_k(const Span* __restrict__ spans, T* a,
                                                           const T* __restrict__ b, double* __restrict__ normdots,
@@ -538,8 +539,8 @@ hipError_t launch_scaled_add(hvdhip_adasum_plan* p, void* a, const void* b, cons
   const uint32_t workgroups = (t.nchunks + kXcds - 1) / kXcds * kXcds;
   return with_store_policy(Stores::kAdasum, [&](auto st) {
     return launch(scaled_add_k<T, FUSED, decltype(st)::value>, workgroups, s, t.chunks, static_cast<T*>(a),
-                  static_cast<const T*>(b), add_turn(t.nchunks), workgroups, t.nchunks, coeffs, ca, cb, p->layers, p->partials, p->normdots, p->coeffs,
-                  std::sqrt(DBL_MIN), (uint32_t)p->nlayers);
+                  static_cast<const T*>(b), add_turn(t.nchunks), workgroups, t.nchunks, coeffs, ca, cb, p->layers,
+                  p->partials, p->normdots, p->coeffs, std::sqrt(DBL_MIN), (uint32_t)p->nlayers);
   });
 }
 

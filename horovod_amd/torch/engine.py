@@ -261,8 +261,8 @@ class Engine:
     def _sum(self, slot, s, req, inputs, outputs, counts, event):
         """outputs = postscale * (sum over ranks of prescale * inputs), in one pass if the outputs lie over no
         other tensor of the response.  The event is bound to the last launch, for callers that wait for handles: a
-        small tensor of eight ranks takes 45 us (48 with the event recorded by itself, as an allgather's is); with a
-        device-wide synchronization behind each call 60 (53)."""
+        small tensor of eight ranks takes 23 us (25 with the event recorded by itself, as an allgather's is); with a
+        device-wide synchronization behind each call 35 (29)."""
         tdt, wire = req.tensor_dtype, req.wire_dtype
         if self.size <= H.RANKS_SUM_MAX_WORLD:
             if H.ranks_sum(outputs, inputs, counts, self.size, tdt, wire, tdt, req.prescale, req.postscale, s,
@@ -361,7 +361,7 @@ class Engine:
         try:
             if not H.ranks_sum(places, sources, counts, 1, dtype, dtype, dtype, 1.0, 1.0, s):
                 raise RuntimeError("an allgather's output lies over one of its inputs")
-            # recorded by itself: bound to the copy's launch it saves 3 us here, and costs 17 in a device-wide
+            # recorded by itself: bound to the copy's launch it saves 2 us here, and costs 6 in a device-wide
             # synchronization that follows, as scripts that read the rows on the host do
             check(lib().hvdhip_event_record(event, s.handle), "hvdhip_event_record")
         except Exception:
@@ -385,9 +385,9 @@ class Engine:
             inputs, source, prescale = [b + o for b in sums for o in offsets], wire, 1.0
         space = H.adasum_ranks_workspace(counts, nodes, wire)
         work = self._buffer(slot, "adasum", space)
-        # Two nodes are two launches, and the event is recorded by itself as in an allgather: 4 million fp32 66 us either
-        # way, and with a device-wide synchronization behind the call 70 (79 with the event bound to the last launch).
-        # Eight nodes take 101 and 115 with the event bound, 106 and 128 without.
+        # Two nodes are two launches, and the event is recorded by itself as in an allgather: 4 million fp32 37 us either
+        # way, and with a device-wide synchronization behind the call 41 (48 with the event bound to the last launch).
+        # Eight nodes take 109 and 121 with the event bound, 112 and 138 without.
         bound = event if nodes > 2 else None
         if H.adasum_ranks(outputs, inputs, counts, nodes, source, wire, tdt, prescale, req.postscale, work, space, s,
                           event=bound):
