@@ -321,3 +321,52 @@ def test_the_null_stream_is_busy_with_a_blocking_one(hvd, peers):
     check(L.hvdhip_stream_idle(None, ctypes.byref(idle)), "hvdhip_stream_idle")
     assert idle.value == 1
     assert L.hipStreamDestroy(handle) == 0
+
+
+@pytest.mark.parametrize("peers", [True, False])
+@pytest.mark.parametrize("stream", ["default", "side"])
+@pytest.mark.parametrize("behind", ["a wait for another stream", "a graph", "a graph of two branches", "a copy from the host"])
+def test_a_stream_is_busy_with_whatever_it_holds(hvd, behind, stream, peers):
+    """What a framework's stream has to do may be no kernel of its own: the look has to find it all the same."""
+    x, y = (torch.zeros(1 << 16, device="cuda") for _ in range(2))
+    hvd.init(size=2, peer_source=(lambda rank, name, t: y) if peers else None)
+    cur = torch.cuda.default_stream() if stream == "default" else torch.cuda.Stream()
+    other, host = torch.cuda.Stream(), torch.zeros(1 << 16).pin_memory()
+    i_dev = torch.zeros(1, device="cuda")
+
+    def write():
+        torch.cuda._sleep(2000000)
+        x.copy_(i_dev.expand_as(x))
+        y.copy_((2 * i_dev).expand_as(y))
+
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    if behind.startswith("a graph"):
+        capturing = torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=capturing):
+            if behind == "a graph":
+                write()
+            else:
+                other.wait_stream(capturing)
+                with torch.cuda.stream(other):
+                    write()
+                capturing.wait_stream(other)
+    for i in range(1, 21):
+        i_dev.fill_(i)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(cur):
+            if behind.startswith("a graph"):
+                graph.replay()
+            elif behind == "a wait for another stream":
+                with torch.cuda.stream(other):
+                    write()
+                cur.wait_stream(other)
+            else:
+                torch.cuda._sleep(2000000)
+                host.fill_(i)
+                x.copy_(host, non_blocking=True)
+                y.copy_(host, non_blocking=True)
+            out = hvd.synchronize(hvd.allreduce_async(x, op=hvd.Sum))
+        want = i + (i if not peers or behind == "a copy from the host" else 2 * i)
+        assert float(out.min()) == float(out.max()) == want, i
+        torch.cuda.synchronize()
