@@ -160,12 +160,13 @@ Request* new_request(PyTypeObject* type, PyObject* entries, PyObject* device, Py
 PyObject* request_new(PyTypeObject* type, PyObject* args, PyObject* kwargs) {
   static const char* names[] = {"entries", "op", "prescale", "postscale", "tensor_dtype", "wire_dtype",
                                 "device", "kind", "grouped", nullptr};
-  PyObject *entries, *device, *kind = g_allreduce;
+  PyObject *entries, *pre, *post, *device, *kind = g_allreduce;
   int op, tensor_dtype, wire_dtype, grouped = 0;
-  double prescale, postscale;
-  if (!PyArg_ParseTupleAndKeywords(args, kwargs, "O!iddiiO|Up", const_cast<char**>(names), &PyList_Type, &entries, &op,
-                                   &prescale, &postscale, &tensor_dtype, &wire_dtype, &device, &kind, &grouped))
+  if (!PyArg_ParseTupleAndKeywords(args, kwargs, "O!iOOiiO|Up", const_cast<char**>(names), &PyList_Type, &entries, &op, &pre,
+                                   &post, &tensor_dtype, &wire_dtype, &device, &kind, &grouped))
     return nullptr;
+  Ref prescale(PyNumber_Float(pre)), postscale(prescale ? PyNumber_Float(post) : nullptr);  // what float() takes, text too
+  if (!postscale) return nullptr;
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(entries); ++i)
     if (Py_TYPE(PyList_GET_ITEM(entries, i)) != &entry_type) {
       PyErr_SetString(PyExc_TypeError, "a request holds entries");
@@ -176,8 +177,8 @@ PyObject* request_new(PyTypeObject* type, PyObject* args, PyObject* kwargs) {
   r->op = op;
   r->tensor_dtype = tensor_dtype;
   r->wire_dtype = wire_dtype;
-  r->prescale = prescale;
-  r->postscale = postscale;
+  r->prescale = PyFloat_AS_DOUBLE(prescale.get());
+  r->postscale = PyFloat_AS_DOUBLE(postscale.get());
   r->grouped = (char)grouped;
   return reinterpret_cast<PyObject*>(r);
 }

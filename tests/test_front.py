@@ -4,6 +4,8 @@ import ctypes
 import os
 import random
 import sys
+from decimal import Decimal
+from fractions import Fraction
 
 import pytest
 import torch
@@ -159,3 +161,16 @@ def test_the_build_is_for_the_interpreter_that_asks(monkeypatch):
     monkeypatch.setattr(build.subprocess, "check_call", commands.append)
     build.build()
     assert "PYTHON=" + sys.executable in commands[0]
+
+
+@pytest.mark.parametrize("factor", [0.5, 2, True, "0.25", Fraction(1, 8), Decimal("0.75"), torch.tensor(1.5), b"3"])
+def test_a_factor_is_whatever_float_takes(front, factor):
+    r = _request(front, [_entry(front, "a", 1)], prescale=factor, postscale=factor)
+    assert r.prescale == r.postscale == float(factor)
+
+
+@pytest.mark.parametrize("factor, error", [(None, TypeError), ("half", ValueError), (10 ** 400, OverflowError)])
+def test_what_float_refuses_is_no_factor(front, factor, error):
+    for which in ("prescale", "postscale"):
+        with pytest.raises(error):
+            _request(front, [_entry(front, "a", 1)], **{which: factor})
