@@ -323,12 +323,19 @@ int hvdhip_stream_idle(void* stream, int* idle) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   const hipError_t before = hipPeekAtLastError();
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  const bool may_ask = hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
-  if (may_ask && hipStreamQuery(s) == hipSuccess) {  // a query would end the stream's capture
-    *idle = 1;
-    return ok();
+  // A query would end the stream's own capture, and in the thread's usual mode any that is going on, of every stream and
+  // thread.
+  if (hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HVDHIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    const bool done = hipStreamQuery(s) == hipSuccess;
+    HVDHIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    if (done) {
+      *idle = 1;
+      return ok();
+    }
   }
-  // Busy, or nothing that can be said (another thread's capture forbids the question): an event will tell.
+  // Busy, or nothing that can be said (a blocking stream's capture forbids to ask the null stream): an event will tell.
   if (before == hipSuccess) (void)hipGetLastError();  // leave no error of this call's behind
   return ok();
 }

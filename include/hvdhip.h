@@ -138,7 +138,8 @@ int hvdhip_stream_synchronize(void* stream);
  * host synchronisation: ops/nccl_operations.cc:140-154. */
 int hvdhip_stream_wait_event(void* stream, void* event);
 /* *idle = 1 if everything that was queued on the stream (any stream of the caller's, NULL for the null
- * stream) has completed, so that nothing need wait for it; 0 if not, or while the stream is being captured.
+ * stream) has completed, so that nothing need wait for it; 0 if not, or while the stream is being captured.  Allowed
+ * while others are captured.
  * No counterpart in the reference, which records a ready event on a stream that is idle as well. */
 int hvdhip_stream_idle(void* stream, int* idle);
 

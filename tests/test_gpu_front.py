@@ -210,6 +210,50 @@ def test_idle_is_said_of_idle_streams_only():
         assert float(x[0]) == 2 * (i + 1)
 
 
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+@pytest.mark.parametrize("stream", ["default", "side"])
+@pytest.mark.parametrize("where", ["here", "in another thread"])
+def test_the_capture_of_another_stream_goes_on(hvd, where, stream, mode):
+    """Whoever asks for a stream that is not being captured, or hands over and waits for a tensor there in another thread, is
+    no concern of a capture that is going on."""
+    L = horovod_amd.lib()
+    hvd.init(size=2)
+    cur = torch.cuda.default_stream() if stream == "default" else torch.cuda.Stream()
+    x, t = torch.zeros(64, device="cuda"), torch.ones(64, device="cuda")
+    g, said = torch.cuda.CUDAGraph(), []
+
+    def work():
+        try:
+            with torch.cuda.stream(cur):
+                for _ in range(3):
+                    idle = ctypes.c_int(-1)
+                    check(L.hvdhip_stream_idle(cur.cuda_stream, ctypes.byref(idle)), "hvdhip_stream_idle")
+                    said.append(idle.value)
+                    if where != "here":
+                        hvd.synchronize(hvd.allreduce_async_(t, op=hvd.Sum))
+        except Exception as e:
+            said.append(repr(e))
+
+    with torch.cuda.stream(cur):
+        hvd.synchronize(hvd.allreduce_async_(t, op=hvd.Average))
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(), capture_error_mode=mode):
+        x.add_(1)
+        if where == "here":
+            work()
+        else:
+            thread = threading.Thread(target=work)
+            thread.start()
+            thread.join()
+        x.add_(1)
+    assert said == [1] * 3
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert float(x.sum()) == 64 * 2 * (i + 1)
+    assert float(t.sum()) == (64 if where == "here" else 64 * 2 ** 3)
+
+
 def test_the_stream_of_a_request_is_the_current_one(hvd, gpu):
     from horovod_amd.torch import engine, mpi_ops
     hvd.init(size=2)
