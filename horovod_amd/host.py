@@ -12,8 +12,9 @@ from ._lib import DTYPE, check, lib
 
 def _ptr_array(values):
     """A C array of addresses; through array.array, which converts a list several times faster
-    than filling a ctypes array element by element and is taken as it is where the caller has one."""
-    raw = values if isinstance(values, array.array) else array.array("Q", values)
+    than filling a ctypes array element by element and is taken as it is where the caller has one of
+    that type."""
+    raw = values if isinstance(values, array.array) and values.typecode == "Q" else array.array("Q", values)
     return (c_void_p * len(raw)).from_buffer(raw) if len(raw) else (c_void_p * 0)()
 
 
@@ -23,7 +24,7 @@ def _size_array(values):
 
 
 def _count_array(values):
-    raw = values if isinstance(values, array.array) else array.array("q", values)
+    raw = values if isinstance(values, array.array) and values.typecode == "q" else array.array("q", values)
     return (c_int64 * len(raw)).from_buffer(raw) if len(raw) else (c_int64 * 0)()
 
 

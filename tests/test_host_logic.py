@@ -1,6 +1,10 @@
 """Host-side arithmetic of the bench/test driver that needs no GPU."""
+import array
 import os
 
+import pytest
+
+from horovod_amd import host as H
 from horovod_amd import workloads as W
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -52,6 +56,26 @@ def test_bert_large_cycles_reduce_an_eighth():
         n = sum((2 * counts[i] + 15) // 16 * 16 for i in g) // 2  # padded fp16 elements of the cycle
         per = W.reduce_scatter_share(n, 8)
         assert 0 <= per - n / 8 < 64
+
+
+@pytest.mark.parametrize("of", [H._ptr_array, H._size_array, H._count_array])
+def test_a_c_array_has_the_values_of_any_sequence_of_integers(of):
+    values = [1, 2, 255]
+    for typecode in "BhHiIlLqQ":
+        assert list(of(array.array(typecode, values))) == values, typecode
+    assert list(of(values)) == list(of(tuple(values))) == values
+    assert list(of(array.array("Q"))) == list(of(array.array("i"))) == []
+    for wrong in (array.array("d", [4.0]), array.array("f", [4.0, 8.0])):  # their bits are no addresses or lengths
+        with pytest.raises(TypeError):
+            of(wrong)
+
+
+def test_a_value_outside_the_range_is_refused():
+    for of in (H._ptr_array, H._size_array):
+        with pytest.raises(OverflowError):
+            of(array.array("q", [-1]))
+    with pytest.raises(OverflowError):
+        H._count_array(array.array("Q", [1 << 63]))
 
 
 def _profile_rows(path):
